@@ -174,12 +174,32 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ counts, in
 
 // A batch of gradient additions dst_j[r][c] += src[off_j + r * lds_j + c]
 // (launch_add_jobs; passed by value as a kernel argument).
+// 96 tensors a launch keep the argument block under 3 KB (a layer of 8
+// experts has 50 tensors: one launch instead of three).
 struct AddJobs {
-  static constexpr int kMax = 24;
+  static constexpr int kMax = 96;
   float* dst[kMax];
   size_t off[kMax];
   int rows[kMax], cols[kMax], lds[kMax];
   int n;
+};
+
+// The six fp32 parameters (W_gate, b_gate, W_up, b_up, W_down, b_down) of up
+// to kMaxExperts experts (launch_pack_experts; passed by value as a kernel
+// argument, 3 KB).
+struct ExpertParams {
+  const float* p[kMaxExperts][6];
+};
+
+// Where launch_pack_experts puts a group of experts, each pointer at the
+// group's first one: the forward's operands wgu [2Hp][C] and wd [Cp][Hp] and
+// the padded biases, and, where the backward's buffers exist, its layouts
+// wgub [Cp][2Hp] and wdb [Hq][C] (both or neither; null: not written).
+template <typename DT>
+struct ExpertPacks {
+  DT *wgu, *wd;
+  float *bg, *bu, *bd;
+  DT *wgub, *wdb;
 };
 
 // Per-expert gradient slices (expert e's slice of piece p: base[p] +

@@ -55,8 +55,10 @@ template <int BM, int BN, int WM, int WN, typename AT, typename WT, int EPI, typ
 hipError_t launch_grouped_gemm(const AT*, const WT*, const float*, const float*, const float*,
                                const int32_t*, int, int, int, int, int, OutT*, int, int, OutT*,
                                int, hipStream_t, float* partials = nullptr, int split_slots = 0);
+hipError_t launch_pack_transpose(const float*, int, int, float*, int, int, int, hipStream_t);
 template <typename DT>
-hipError_t launch_pack_transpose(const float*, int, int, DT*, int, int, int, hipStream_t);
+hipError_t launch_pack_experts(const ExpertParams&, int, const ExpertPacks<DT>&, int, int, int, int,
+                               int, int, hipStream_t);
 hipError_t launch_quantize_rows(const float*, int, int, uint8_t*, float*, hipStream_t);
 hipError_t launch_pad_row(const float*, int, float*, int, hipStream_t);
 template <typename XT>
@@ -64,8 +66,8 @@ hipError_t launch_gemm_decode_gather(const XT*, const fp8_t*, const float*, cons
                                      const float*, const int32_t*, int, int, int, int, int, int,
                                      int, bf16_t*, int, int, int32_t*, int32_t*, int32_t*,
                                      hipStream_t);
-hipError_t launch_pack_router(const float*, int, int, int, int, float*, hipStream_t);
-hipError_t launch_pack_router_quads(const float*, int, int, int, float*, hipStream_t);
+hipError_t launch_pack_router(const float*, const float*, int, int, int, int, float*, float*, float*,
+                              float*, float*, hipStream_t);
 template <int EPI>
 hipError_t launch_gemm_dma(const bf16_t*, const bf16_t*, const float*, const float*,
                            const int32_t*, int, int, int, int, int, bf16_t*, int, int, float*, int,
@@ -226,20 +228,21 @@ struct mgpt_moe {
   float* bg = nullptr;     // [E][Hp]
   float* bu = nullptr;     // [E][Hp]
   float* bd = nullptr;     // [E][Cp]
-  // staging of host parameters (one of the largest size) and, for fp8, the
+  // staging of host parameters (the router's or one expert's) and, for fp8, the
   // packed fp32 rows before quantisation; kept for later loads
   float* stage = nullptr;
   float* stage_tmp = nullptr;
   bool loaded = false;
   // Backward: the weights in the layouts the data-gradient products read,
-  // derived from the forward packs on the first backward after a load
+  // derived from the forward packs on the first backward, then written by
+  // every load (bwd_init: an eager backward has filled them, padding included)
   // (wdb [E][Hq][C]: W_down rows h; wgub [E][Cp][2Hp]: W_gate/W_up rows c,
   // columns in the packed gate/up order), and the fp32 gradients.
   int Hq = 0;
   void* wdb = nullptr;
   void* wgub = nullptr;
   float* wrt = nullptr;    // W_r as [E][C] (fp32)
-  bool bwd_ready = false;
+  bool bwd_ready = false, bwd_init = false;
   float* grad = nullptr;   // gWr [C][E], gbr [E], gWg [E][C][H], gbg [E][H],
                            // gWu [E][C][H], gbu [E][H], gWd [E][H][C], gbd [E][C]
   size_t g_off[8] = {};
@@ -388,7 +391,7 @@ void free_weights(mgpt_moe* h) {
   h->stage = h->stage_tmp = nullptr;
   h->wgu = h->wd = h->wdb = h->wgub = h->wgu_t = h->wd_t = nullptr;
   h->loaded = false;
-  h->bwd_ready = false;
+  h->bwd_ready = h->bwd_init = false;
 }
 
 // Training is built for bf16 x bf16 and fp32 x fp32 handles (fp8 weights
@@ -430,7 +433,8 @@ int materialize_grad(mgpt_moe* h, hipStream_t st) {
   return MGPT_OK;
 }
 
-// The backward weight layouts, transposed from the forward packs.
+// The backward weight layouts, transposed from the forward packs on the
+// first backward of a handle (later loads write them with the packs).
 int ensure_bwd_weights(mgpt_moe* h, hipStream_t st) {
   if (h->bwd_ready) return MGPT_OK;
   const int C = h->C, E = h->E, Hp = h->Hp, Cp = h->Cp;
@@ -457,6 +461,11 @@ int ensure_bwd_weights(mgpt_moe* h, hipStream_t st) {
                                         (float*)h->wgub, Cp, 2 * Hp, (size_t)Cp * 2 * Hp, E, st));
   }
   h->bwd_ready = true;
+  // A captured backward fills them only when its graph runs: loads then go on
+  // leaving them to the backward.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  if (cap == hipStreamCaptureStatusNone) h->bwd_init = true;
   return MGPT_OK;
 }
 
@@ -569,7 +578,8 @@ int mgpt_moe_load_parameters(mgpt_moe* h, const float* const* params, int num_pa
   // The packed buffers depend only on the handle's shape: the first load
   // allocates them (and zeroes the padding the packs never write), later
   // loads re-pack into them, stream-ordered, with no allocation.  The
-  // backward's transposed copies are rebuilt from the new packs.
+  // backward's copies are rebuilt too: by this load once they exist, else by
+  // the first backward.
   h->loaded = false;
   h->bwd_ready = false;
   const bool first = h->wgu == nullptr;
@@ -592,82 +602,106 @@ int mgpt_moe_load_parameters(mgpt_moe* h, const float* const* params, int num_pa
     HIP_TRY(hipMemsetAsync(h->wgu, 0, wb * E * 2 * Hp * C, st));
   }
 
-  // Host parameters are staged through one device buffer of the largest size.
-  const size_t max_elems = std::max<size_t>((size_t)Cx * std::max(H, E), (size_t)H * Cx);
-  if (!params_on_device && !h->stage) HIP_TRY(hipMalloc(&h->stage, sizeof(float) * max_elems));
+  // Host parameters are staged through one device buffer, the router's two
+  // or one expert's six at a time (each at a multiple of 4 floats).
+  auto up4 = [](size_t n) { return (n + 3) / 4 * 4; };
+  const size_t CH = (size_t)Cx * H;
+  const size_t sizes[6] = {CH, (size_t)H, CH, (size_t)H, CH, (size_t)Cx};
+  const size_t stage_elems = std::max(up4((size_t)Cx * E) + up4(E), 3 * up4(CH) + 2 * up4(H) + up4(Cx));
+  if (!params_on_device && !h->stage) HIP_TRY(hipMalloc(&h->stage, sizeof(float) * stage_elems));
   if (fp8 && !h->stage_tmp)
     HIP_TRY(hipMalloc(&h->stage_tmp,
                       sizeof(float) * std::max<size_t>((size_t)2 * Hp * C, (size_t)Cp * Hp)));
-  float* stage = h->stage;
   float* fp32tmp = h->stage_tmp;   // fp8: packed fp32 before quantisation
   int rc = MGPT_OK;
-  auto src = [&](int i, size_t n) -> const float* {
-    if (params_on_device) return params[i];
-    hipError_t e = hipMemcpyAsync(stage, params[i], sizeof(float) * n, hipMemcpyHostToDevice, st);
-    if (e != hipSuccess) {
-      rc = fail(MGPT_ERR_HIP, "parameter %d upload failed: %s", i, hipGetErrorString(e));
-      return nullptr;
+  // Device addresses of parameters i0 .. i0+n-1 (sizes sz) in p.
+  auto fetch = [&](int i0, int n, const size_t* sz, const float** p) -> bool {
+    float* d = h->stage;
+    for (int i = 0; i < n; ++i) {
+      p[i] = params[i0 + i];
+      if (params_on_device) continue;
+      const hipError_t e =
+          hipMemcpyAsync(d, params[i0 + i], sizeof(float) * sz[i], hipMemcpyHostToDevice, st);
+      if (e != hipSuccess) {
+        rc = fail(MGPT_ERR_HIP, "parameter %d upload failed: %s", i0 + i, hipGetErrorString(e));
+        return false;
+      }
+      p[i] = d;
+      d += up4(sz[i]);
     }
-    return stage;
+    return true;
   };
-  auto pack = [&](const float* s, int Kin, int Nout, void* dst, int ldd, int mode, int off) {
-    hipError_t e;
-    if (bf)
-      e = launch_pack_transpose<bf16_t>(s, Kin, Nout, (bf16_t*)dst, ldd, mode, off, st);
-    else
-      e = launch_pack_transpose<float>(s, Kin, Nout, (float*)dst, ldd, mode, off, st);
-    if (e != hipSuccess) rc = fail(MGPT_ERR_HIP, "pack failed: %s", hipGetErrorString(e));
+  // Host sources share the stage: finish before it is filled again.
+  auto staged = [&]() -> bool {
+    if (params_on_device) return true;
+    const hipError_t e = hipStreamSynchronize(st);
+    if (e != hipSuccess) rc = fail(MGPT_ERR_HIP, "parameter packing failed: %s", hipGetErrorString(e));
+    return e == hipSuccess;
   };
+  // The backward's layouts are written here as well once a backward has
+  // filled them (and zeroed their padding).
+  const bool bwd = h->bwd_init;
   do {
-    const float* s = src(0, (size_t)Cx * E);
-    if (!s) break;
-    if (launch_pack_router(s, Cx, C, E, RE, h->wr_g, st) != hipSuccess ||
-        (h->wr1 && launch_pack_router(s, Cx, C, E, 1, h->wr1, st) != hipSuccess) ||
-        (h->wr4 && launch_pack_router_quads(s, Cx, C, E, h->wr4, st) != hipSuccess)) {
-      rc = fail(MGPT_ERR_HIP, "router pack failed");
+    const float* rp[2];
+    const size_t rsz[2] = {(size_t)Cx * E, (size_t)E};
+    if (!fetch(0, 2, rsz, rp)) break;
+    const hipError_t re = launch_pack_router(rp[0], rp[1], Cx, C, E, RE, h->wr_g, h->wr1, h->wr4,
+                                             bwd ? h->wrt : nullptr, h->br, st);
+    if (re != hipSuccess) {
+      rc = fail(MGPT_ERR_HIP, "router pack failed: %s", hipGetErrorString(re));
       break;
     }
-    s = src(1, E);
-    if (!s) break;
-    HIP_TRY(hipMemcpyAsync(h->br, s, sizeof(float) * E, hipMemcpyDeviceToDevice, st));
+    if (!staged()) break;
+    if (!fp8) {
+      // one launch per group of experts; host sources go expert by expert
+      const int step = params_on_device ? kMaxExperts : 1;
+      for (int e0 = 0; e0 < E && rc == MGPT_OK; e0 += step) {
+        const int n = std::min(step, E - e0);
+        ExpertParams ep;
+        for (int e = 0; e < n && rc == MGPT_OK; ++e) fetch(2 + 6 * (e0 + e), 6, sizes, ep.p[e]);
+        if (rc) break;
+        auto launch = [&](auto tag) {
+          typedef decltype(tag) DT;
+          ExpertPacks<DT> out{};
+          out.wgu = (DT*)h->wgu + (size_t)e0 * 2 * Hp * C;
+          out.wd = (DT*)h->wd + (size_t)e0 * Cp * Hp;
+          out.bg = h->bg + (size_t)e0 * Hp;
+          out.bu = h->bu + (size_t)e0 * Hp;
+          out.bd = h->bd + (size_t)e0 * Cp;
+          if (bwd) {
+            out.wgub = (DT*)h->wgub + (size_t)e0 * Cp * 2 * Hp;
+            out.wdb = (DT*)h->wdb + (size_t)e0 * h->Hq * C;
+          }
+          return launch_pack_experts<DT>(ep, n, out, Cx, C, H, Hp, Cp, h->Hq, st);
+        };
+        const hipError_t pe = bf ? launch(bf16_t()) : launch(float());
+        if (pe != hipSuccess) rc = fail(MGPT_ERR_HIP, "pack failed: %s", hipGetErrorString(pe));
+        else staged();
+      }
+      break;
+    }
     for (int e = 0; e < E && rc == MGPT_OK; ++e) {
-      const int p = 2 + 6 * e;
+      const float* s[6];
+      if (!fetch(2 + 6 * e, 6, sizes, s)) break;
       const size_t gu_off = (size_t)e * 2 * Hp * C;
       const size_t d_off = (size_t)e * Cp * Hp;
-      if (fp8) HIP_TRY(hipMemsetAsync(fp32tmp, 0, sizeof(float) * 2 * Hp * C, st));
-      for (int which = 0; which < 2 && rc == MGPT_OK; ++which) {   // gate, up
+      HIP_TRY(hipMemsetAsync(fp32tmp, 0, sizeof(float) * 2 * Hp * C, st));
+      for (int which = 0; which < 2; ++which) {   // gate, up
         // [Cx][H] -> rows of the packed [2Hp][C]: columns past Cx stay zero
-        if (!(s = src(p + 2 * which, (size_t)Cx * H))) break;
-        if (fp8) {
-          if (launch_pack_transpose<float>(s, Cx, H, fp32tmp, C, 1, 32 * which, st) != hipSuccess)
-            rc = fail(MGPT_ERR_HIP, "pack failed");
-        } else {
-          pack(s, Cx, H, (char*)h->wgu + gu_off * h->w_bytes(), C, 1, 32 * which);
-        }
-        if (!(s = src(p + 2 * which + 1, H))) break;
-        HIP_TRY(launch_pad_row(s, H, (which ? h->bu : h->bg) + (size_t)e * Hp, Hp, st));
+        HIP_TRY(launch_pack_transpose(s[2 * which], Cx, H, fp32tmp, C, 1, 32 * which, st));
+        HIP_TRY(launch_pad_row(s[2 * which + 1], H, (which ? h->bu : h->bg) + (size_t)e * Hp, Hp, st));
       }
-      if (rc) break;
-      if (fp8)
-        HIP_TRY(launch_quantize_rows(fp32tmp, 2 * Hp, C, (uint8_t*)h->wgu + gu_off,
-                                     h->sgu + (size_t)e * 2 * Hp, st));
+      HIP_TRY(launch_quantize_rows(fp32tmp, 2 * Hp, C, (uint8_t*)h->wgu + gu_off,
+                                   h->sgu + (size_t)e * 2 * Hp, st));
       // [H][Cx] -> rows 0..Cx of the packed [Cp][Hp]; the rest stay zero
-      if (!(s = src(p + 4, (size_t)H * Cx))) break;
-      if (fp8) {
-        HIP_TRY(hipMemsetAsync(fp32tmp, 0, sizeof(float) * Cp * Hp, st));
-        if (launch_pack_transpose<float>(s, H, Cx, fp32tmp, Hp, 0, 0, st) != hipSuccess)
-          rc = fail(MGPT_ERR_HIP, "pack failed");
-        HIP_TRY(launch_quantize_rows(fp32tmp, Cp, Hp, (uint8_t*)h->wd + d_off,
-                                     h->sd + (size_t)e * Cp, st));
-      } else {
-        pack(s, H, Cx, (char*)h->wd + d_off * h->w_bytes(), Hp, 0, 0);
-      }
-      if (!(s = src(p + 5, Cx))) break;
-      HIP_TRY(launch_pad_row(s, Cx, h->bd + (size_t)e * Cp, Cp, st));
-      // Host sources are staged through one buffer: finish before reuse.
-      if (!params_on_device) HIP_TRY(hipStreamSynchronize(st));
+      HIP_TRY(hipMemsetAsync(fp32tmp, 0, sizeof(float) * Cp * Hp, st));
+      HIP_TRY(launch_pack_transpose(s[4], H, Cx, fp32tmp, Hp, 0, 0, st));
+      HIP_TRY(launch_quantize_rows(fp32tmp, Cp, Hp, (uint8_t*)h->wd + d_off,
+                                   h->sd + (size_t)e * Cp, st));
+      HIP_TRY(launch_pad_row(s[5], Cx, h->bd + (size_t)e * Cp, Cp, st));
+      if (!staged()) break;
     }
-    if (rc == MGPT_OK && fp8 && C % 128 == 0 && Hp % 128 == 0 && Cp % 256 == 0) {
+    if (rc == MGPT_OK && C % 128 == 0 && Hp % 128 == 0 && Cp % 256 == 0) {
       // the decode stream's contiguous 32 KB stage tiles (a second copy)
       if (!h->wgu_t) HIP_TRY(hipMalloc(&h->wgu_t, (size_t)E * 2 * Hp * C));
       if (!h->wd_t) HIP_TRY(hipMalloc(&h->wd_t, (size_t)E * Cp * Hp));
@@ -690,6 +724,7 @@ int mgpt_moe_load_parameters(mgpt_moe* h, const float* const* params, int num_pa
     }
   }
   h->loaded = true;
+  h->bwd_ready = bwd;
   return MGPT_OK;
 }
 
