@@ -54,8 +54,16 @@ hipError_t launch_add_jobs(const float*, const AddJobs&, size_t, hipStream_t);
 template <int BM, int BN, int WM, int WN, typename AT, typename WT, int EPI, typename OutT>
 hipError_t launch_grouped_gemm(const AT*, const WT*, const float*, const float*, const float*,
                                const int32_t*, int, int, int, int, int, OutT*, int, int, OutT*,
-                               int, hipStream_t, float* partials = nullptr, int split_slots = 0);
+                               int, hipStream_t);
 hipError_t launch_pack_transpose(const float*, int, int, float*, int, int, int, hipStream_t);
+template <int EPI>
+hipError_t launch_gemm_f32(const float*, const float*, const float*, const float*, const int32_t*,
+                           int, int, int, int, int, float*, int, size_t, float*, int, int,
+                           hipStream_t);
+template <int MODE>
+hipError_t launch_wgrad_f32(const float*, int, int, const float*, int, int, const int32_t*, int,
+                            float*, float*, int, size_t, int, int, float*, float*, size_t, int,
+                            bool, hipStream_t);
 template <typename DT>
 hipError_t launch_pack_experts(const ExpertParams&, int, const ExpertPacks<DT>&, int, int, int, int,
                                int, int, hipStream_t);
@@ -91,9 +99,9 @@ hipError_t launch_rmsnorm_bwd(const ActT*, ActT*, const ActT*, const float*, con
 template <typename T>
 hipError_t launch_transpose_pad(const T*, int, int, size_t, T*, int, int, size_t, int,
                                 hipStream_t);
-template <typename T, int MODE>
-hipError_t launch_wgrad(const T*, int, int, const T*, int, int, const int32_t*, int, float*,
-                        float*, int, size_t, int, int, float*, float*, size_t, int, float*,
+template <int MODE>
+hipError_t launch_wgrad(const bf16_t*, int, int, const bf16_t*, int, int, const int32_t*, int,
+                        float*, float*, int, size_t, int, int, float*, float*, size_t, int, float*,
                         size_t, float*, size_t, int, bool, hipStream_t);
 hipError_t launch_zero_idle_experts(const int32_t*, int, const IdleSlices&, hipStream_t);
 hipError_t launch_fill_zero(float* p, size_t n, hipStream_t stream);
@@ -134,10 +142,6 @@ namespace {
 
 constexpr size_t kAlign = 256;
 constexpr size_t kGemmPartialBytes = 512 * 128 * 4;   // one 256x256 fp32 tile
-// fp32 handles: one 64x128 fp32 partial tile per CU for the split-K down
-// product of small token counts (a fixed size, so the workspace stays
-// monotonic in N)
-constexpr size_t kF32PartialBytes = 64 * 128 * 4;
 constexpr int kRowPad = 256;   // rows of slack after activation buffers (GEMM tile overrun)
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -329,9 +333,7 @@ struct mgpt_moe {
     L.hbuf = take((A + kRowPad) * Hp * act_bytes());
     L.obuf = take((A + kRowPad) * C * act_bytes());
     // fp32 partial tiles of the large-M GEMMs' split last round (one per CU)
-    L.partials = take(uses_gemm_dma(N)             ? (size_t)num_cus * kGemmPartialBytes
-                      : act == MGPT_DTYPE_F32 ? (size_t)num_cus * kF32PartialBytes
-                                              : 0);
+    L.partials = take(uses_gemm_dma(N) ? (size_t)num_cus * kGemmPartialBytes : 0);
     L.rstd = take((size_t)N * 4);
     const size_t pad_rows = padded() ? (size_t)N * C * io_bytes() : 0;
     L.xpad = take(pad_rows);
@@ -854,15 +856,11 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
                                        counts, perm, slot_of, xg, rstd, gamma, st)));
   HIP_TRY(mark(2));
   if constexpr (sizeof(ActT) == 4) {
-    const int mt = (int)((A + 63) / 64) + E;
-    HIP_TRY((launch_grouped_gemm<64, 128, 2, 2, float, float, kEpiGateUp, float>(
-        xg, (const float*)h->wgu, nullptr, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp,
-        mt, gu, 2 * Hp, st)));
+    HIP_TRY(launch_gemm_f32<kEpiGateUp>(xg, (const float*)h->wgu, h->bg, h->bu, counts, E, C, 2 * Hp,
+                                        2 * Hp, Hp, hb, Hp, A, gu, 2 * Hp, h->num_cus, st));
     HIP_TRY(mark(3));
-    // few tiles (small N): split along K over the CUs (fp32 partials, in-order reduce)
-    HIP_TRY((launch_grouped_gemm<64, 128, 2, 2, float, float, kEpiDown, float>(
-        hb, (const float*)h->wd, nullptr, h->bd, nullptr, counts, E, Hp, Cp, C, Cp, ob, C, mt,
-        nullptr, 0, st, (float*)(ws + L.partials), h->num_cus)));
+    HIP_TRY(launch_gemm_f32<kEpiDown>(hb, (const float*)h->wd, h->bd, nullptr, counts, E, Hp, Cp, C,
+                                      Cp, ob, C, A, nullptr, 0, h->num_cus, st));
   } else {
     const bool fp8 = h->wdt == MGPT_DTYPE_FP8_E4M3;
     if (small_m(h, N)) {
@@ -1018,10 +1016,27 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
       z.n = 6;
       HIP_TRY(launch_zero_idle_experts(counts, E, z, s));
     }
-    HIP_TRY((launch_wgrad<ActT, 0>(hb, Hp, Hp, dgo, C, C, counts, E, g + h->g_off[6], nullptr, C,
-                                   (size_t)H * C, H, C, g + h->g_off[7], nullptr, (size_t)C, A,
-                                   wpart, wpart_bytes, wbpart, wbpart_bytes, h->num_cus, store,
-                                   s)));
+    if constexpr (sizeof(ActT) == 4)
+      HIP_TRY(launch_wgrad_f32<0>(hb, Hp, Hp, dgo, C, C, counts, E, g + h->g_off[6], nullptr, C,
+                                  (size_t)H * C, H, C, g + h->g_off[7], nullptr, (size_t)C,
+                                  h->num_cus, store, s));
+    else
+      HIP_TRY(launch_wgrad<0>(hb, Hp, Hp, dgo, C, C, counts, E, g + h->g_off[6], nullptr, C,
+                              (size_t)H * C, H, C, g + h->g_off[7], nullptr, (size_t)C, A, wpart,
+                              wpart_bytes, wbpart, wbpart_bytes, h->num_cus, store, s));
+    return MGPT_OK;
+  };
+  // dW_gate/up; `part` takes the row chunks' partial tiles
+  auto gateup_wgrad = [&](float* part, hipStream_t s) -> int {
+    if constexpr (sizeof(ActT) == 4)
+      HIP_TRY(launch_wgrad_f32<1>(xg, C, C, gu, 2 * Hp, 2 * Hp, counts, E, g + h->g_off[2],
+                                  g + h->g_off[4], H, (size_t)C * H, C, H, g + h->g_off[3],
+                                  g + h->g_off[5], (size_t)H, h->num_cus, store, s));
+    else
+      HIP_TRY(launch_wgrad<1>(xg, C, C, gu, 2 * Hp, 2 * Hp, counts, E, g + h->g_off[2],
+                              g + h->g_off[4], H, (size_t)C * H, C, H, g + h->g_off[3],
+                              g + h->g_off[5], (size_t)H, A, part, wpart_bytes, wbpart,
+                              wbpart_bytes, h->num_cus, store, s));
     return MGPT_OK;
   };
 
@@ -1029,14 +1044,11 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
   HIP_TRY(launch_scatter_bwd<ActT>(dy, ob, perm, topp, A, C, k, dgo, dtp, st));
   HIP_TRY(mark(1));
   if constexpr (sizeof(ActT) == 4) {
-    const int mt = (A + 63) / 64 + E;
-    HIP_TRY((launch_grouped_gemm<64, 128, 2, 2, float, float, kEpiSwigluBwd, float>(
-        dgo, wdb, nullptr, nullptr, nullptr, counts, E, C, h->Hq, Hp, 0, gu, 2 * Hp, mt, gu,
-        2 * Hp, st)));
+    HIP_TRY(launch_gemm_f32<kEpiSwigluBwd>(dgo, wdb, nullptr, nullptr, counts, E, C, h->Hq, Hp, 0, gu,
+                                           2 * Hp, A, gu, 2 * Hp, h->num_cus, st));
     HIP_TRY(mark(2));
-    HIP_TRY((launch_grouped_gemm<64, 128, 2, 2, float, float, kEpiDown, float>(
-        gu, wgub, nullptr, nullptr, nullptr, counts, E, 2 * Hp, Cp, C, 0, ob, C, mt, nullptr, 0,
-        st)));
+    HIP_TRY(launch_gemm_f32<kEpiDown>(gu, wgub, nullptr, nullptr, counts, E, 2 * Hp, Cp, C, 0, ob, C, A,
+                                      nullptr, 0, h->num_cus, st));
   } else if (h->uses_gemm_dma(N)) {
     // prefill-shaped segments: the 256x256 direct-to-LDS kernel; the dX
     // product splits its last round like the forward's down GEMM
@@ -1070,11 +1082,7 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
       // -> 2.22-2.23 ms with dX on 128 of 256 CUs; 96: 2.26, 160: 2.23).
       HIP_TRY(hipEventRecord(h->fork_ev, st));
       HIP_TRY(hipStreamWaitEvent(h->side, h->fork_ev, 0));
-      HIP_TRY((launch_wgrad<ActT, 1>(xg, C, C, gu, 2 * Hp, 2 * Hp, counts, E, g + h->g_off[2],
-                                     g + h->g_off[4], H, (size_t)C * H, C, H, g + h->g_off[3],
-                                     g + h->g_off[5], (size_t)H, A, (float*)(ws + L.wg_part2),
-                                     wpart_bytes, wbpart, wbpart_bytes, h->num_cus, store,
-                                     h->side)));
+      if (int rc = gateup_wgrad((float*)(ws + L.wg_part2), h->side)) return rc;
       HIP_TRY(hipEventRecord(h->join_ev, h->side));
       gateup_done = true;
     }
@@ -1106,10 +1114,7 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
     if (int rc = down_wgrad(st)) return rc;
   HIP_TRY(mark(4));
   if (!gateup_done)
-    HIP_TRY((launch_wgrad<ActT, 1>(xg, C, C, gu, 2 * Hp, 2 * Hp, counts, E, g + h->g_off[2],
-                                   g + h->g_off[4], H, (size_t)C * H, C, H, g + h->g_off[3],
-                                   g + h->g_off[5], (size_t)H, A, wpart, wpart_bytes, wbpart,
-                                   wbpart_bytes, h->num_cus, store, st)));
+    if (int rc = gateup_wgrad(wpart, st)) return rc;
   HIP_TRY(mark(5));
   HIP_TRY(launch_token_bwd<ActT>(ob, slot_of, idx, dtp, probs, counts, h->wrt, N, C, E, k, dx,
                                  dlog, st));
