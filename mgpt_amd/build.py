@@ -19,7 +19,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "lib")
 OBJ = os.path.join(HERE, "_build")
 
-HIP_SOURCES = ["router.hip", "dispatch.hip", "gemm.hip", "gemm_f32.hip", "gemm_dma.hip", "gemm_decode.hip", "combine.hip",
+HIP_SOURCES = ["router.hip", "dispatch.hip", "gemm.hip", "gemm_f32.hip", "gemm_dma.hip", "gemm_stream.hip",
+               "gemm_decode.hip", "combine.hip",
                "pack.hip", "backward.hip", "wgrad.hip", "moe_capi.hip", "checkpoint.cpp"]
 ARCH = os.environ.get("MGPT_OFFLOAD_ARCH", "gfx950")
 

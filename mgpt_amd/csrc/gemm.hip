@@ -1,5 +1,6 @@
-// gemm.hip -- grouped expert GEMMs on CDNA4 matrix cores, bf16 activations
-// (gemm_f32.hip has the fp32 ones).
+// gemm.hip -- grouped bf16 expert GEMMs with register-staged 128 x 128 tiles,
+// the alternative to gemm_dma.hip's 256 x 256 ones for large segments that
+// MGPT_MOE_GEMM_TILE=128 selects.
 //
 // Reference: per expert e with count_e > 0, SwiGLU::forward_into
 // (layers/SwiGLU.cpp:23-50): g = X_e W_g + b_g, u = X_e W_u + b_u,
@@ -13,18 +14,17 @@
 // B = packed weights [E][Npad][K] (K contiguous, so both MFMA operands are
 // read as 16-byte K-runs); C = A . B^T.  Tiles: block BM x BN x BK with 4
 // waves in a WM x WN grid; each wave owns (BM/WM) x (BN/WN) made of 32x32
-// MFMA tiles: v_mfma_f32_32x32x16_bf16 (fp8 weights are widened to bf16
-// exactly while being staged into LDS).  Global -> register -> LDS double buffering: the next K-slab is
+// MFMA tiles: v_mfma_f32_32x32x16_bf16.  Global -> register -> LDS double buffering: the next K-slab is
 // fetched while the current one feeds the MFMAs; one barrier per slab.
 //
 // Epilogues: GATEUP (B rows interleaved in 64-row groups [32 gate | 32 up]
 // for the same 32 hidden units, so a wave's two adjacent 32x32 tiles hold
 // g and u of the same (row, h) in the same lane) computes
-// h = silu(g*s_g + b_g) * (u*s_u + b_u) and stores bf16 h, and, when
+// h = silu(g + b_g) * (u + b_u) and stores bf16 h, and, when
 // `aux` is given, also the pre-activations g, u in the interleaved layout
 // (aux[row][packed column], the caches of layers/SwiGLU.cpp:30-31 that the
 // backward pass reads);
-// DOWN stores o = acc*s + b_d in the activation dtype (no bias if bias0 is
+// DOWN stores o = acc + b_d in the activation dtype (no bias if bias0 is
 // null);
 // SWIGLU_BWD treats the product as d(act)[row][h] and applies the CPU
 // swiglu_backward of utils/Tensor.cpp:2006-2030 with the saved g, u read
@@ -48,40 +48,28 @@ struct alignas(16) U4 {
 };
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// e4m3 byte pair -> two bf16 in one dword (exact: every e4m3 value is a bf16 value).
-template <bool HI>
-__device__ __forceinline__ uint32_t e4m3x2_to_bf16x2(uint32_t packed_bytes) {
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-  bf16x2_t v = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)packed_bytes, 1.0f, HI);
-  uint32_t r;
-  __builtin_memcpy(&r, &v, 4);
-  return r;
-}
-
-template <int BM, int BN, int WM, int WN, typename AT, typename WT, int EPI, typename OutT>
+template <int BM, int BN, int WM, int WN, int EPI>
 __global__ __launch_bounds__(256) void grouped_gemm_kernel(
-    const AT* __restrict__ A, const WT* __restrict__ B, const float* __restrict__ wscale,
-    const float* __restrict__ bias0, const float* __restrict__ bias1,
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, const float* __restrict__ bias0, const float* __restrict__ bias1,
     const int32_t* __restrict__ counts, int E, int K, int Npad, int n_store, int bias_ld,
-    OutT* out, int ldo, OutT* aux, int aux_ld) {
+    bf16_t* out, int ldo, bf16_t* aux, int aux_ld) {
   constexpr int BK = kSlab;
-  constexpr int PAD = 16 / (int)sizeof(AT);
+  constexpr int PAD = 16 / 2;
   constexpr int LDK = BK + PAD;
   constexpr int WTM = BM / WM, WTN = BN / WN;
   constexpr int TM = WTM / 32, TN = WTN / 32;
   static_assert(WM * WN == 4, "4 waves");
   static_assert(TM >= 1 && TN >= 1, "wave tile >= 32x32");
   static_assert(EPI != kEpiGateUp || (TN % 2 == 0), "gate/up pairs");
-  constexpr bool kFp8 = sizeof(WT) == 1;
   // 16-byte chunks per K-slab row, and per-thread chunk counts.
-  constexpr int A_CPR = BK * (int)sizeof(AT) / 16;             // 8
-  constexpr int B_CPR = BK * (int)sizeof(WT) / 16;             // 8 (bf16/f32) or 4 (fp8)
+  constexpr int A_CPR = BK * 2 / 16;             // 8
+  constexpr int B_CPR = BK * 2 / 16;             // 8
   constexpr int A_CH = BM * A_CPR / 256;
   constexpr int B_CH = BN * B_CPR / 256;
   static_assert(A_CH >= 1 && B_CH >= 1, "tile too small for 256 threads");
 
-  __shared__ __attribute__((aligned(16))) AT sA[2][BM][LDK];
-  __shared__ __attribute__((aligned(16))) AT sB[2][BN][LDK];
+  __shared__ __attribute__((aligned(16))) bf16_t sA[2][BM][LDK];
+  __shared__ __attribute__((aligned(16))) bf16_t sB[2][BN][LDK];
 
   // XCD-aware order: the hardware deals consecutive workgroups round-robin
   // to the 8 XCDs (each with its own L2); remap so each XCD receives a
@@ -101,8 +89,8 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(
   const int w = tid / kWave, lane = lane_id();
   const int wm = w / WN, wn = w % WN;
 
-  const AT* Ablk = A + (size_t)ti.row0 * K;
-  const WT* Bblk = B + ((size_t)e * Npad + n0) * K;
+  const bf16_t* Ablk = A + (size_t)ti.row0 * K;
+  const bf16_t* Bblk = B + ((size_t)e * Npad + n0) * K;
 
   U4 ra[A_CH], rb[B_CH];
   auto gload = [&](int kt) __attribute__((always_inline)) {
@@ -112,14 +100,14 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(
     for (int i = 0; i < A_CH; ++i) {
       const int q = tid + 256 * i;
       const int r = q / A_CPR, c = q % A_CPR;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(abase + (size_t)r * K * sizeof(AT) + c * 16);
+      const u32x4 v = *reinterpret_cast<const u32x4*>(abase + (size_t)r * K * 2 + c * 16);
       ra[i].x = v.x; ra[i].y = v.y; ra[i].z = v.z; ra[i].w = v.w;
     }
 #pragma unroll
     for (int i = 0; i < B_CH; ++i) {
       const int q = tid + 256 * i;
       const int r = q / B_CPR, c = q % B_CPR;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(bbase + (size_t)r * K * sizeof(WT) + c * 16);
+      const u32x4 v = *reinterpret_cast<const u32x4*>(bbase + (size_t)r * K * 2 + c * 16);
       rb[i].x = v.x; rb[i].y = v.y; rb[i].z = v.z; rb[i].w = v.w;
     }
   };
@@ -134,19 +122,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(
     for (int i = 0; i < B_CH; ++i) {
       const int q = tid + 256 * i;
       const int r = q / B_CPR, c = q % B_CPR;
-      if constexpr (kFp8) {
-        // 16 e4m3 bytes -> 16 bf16 (32 bytes) at element offset c*16.
-        U4 lo, hi;
-        lo.x = e4m3x2_to_bf16x2<false>(rb[i].x); lo.y = e4m3x2_to_bf16x2<true>(rb[i].x);
-        lo.z = e4m3x2_to_bf16x2<false>(rb[i].y); lo.w = e4m3x2_to_bf16x2<true>(rb[i].y);
-        hi.x = e4m3x2_to_bf16x2<false>(rb[i].z); hi.y = e4m3x2_to_bf16x2<true>(rb[i].z);
-        hi.z = e4m3x2_to_bf16x2<false>(rb[i].w); hi.w = e4m3x2_to_bf16x2<true>(rb[i].w);
-        U4* dst = reinterpret_cast<U4*>(&sB[buf][r][c * 16]);
-        dst[0] = lo;
-        dst[1] = hi;
-      } else {
-        *reinterpret_cast<U4*>(reinterpret_cast<char*>(&sB[buf][r][0]) + c * 16) = rb[i];
-      }
+      *reinterpret_cast<U4*>(reinterpret_cast<char*>(&sB[buf][r][0]) + c * 16) = rb[i];
     }
   };
 
@@ -205,8 +181,6 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(
     for (int q = 0; q < TN / 2; ++q) {
       const int prow = n0 + wn * WTN + q * 64 + lrow;   // packed row of the gate column
       const int hcol = (n0 + wn * WTN) / 2 + q * 32 + lrow;
-      const float sg = kFp8 ? wscale[(size_t)e * Npad + prow] : 1.0f;
-      const float su = kFp8 ? wscale[(size_t)e * Npad + prow + 32] : 1.0f;
       const float bg = bias0[(size_t)e * bias_ld + hcol];
       const float bu = bias1[(size_t)e * bias_ld + hcol];
 #pragma unroll
@@ -217,7 +191,6 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(
           if (row < ti.row_end) {
             float g = acc[i][2 * q][v];
             float u = acc[i][2 * q + 1][v];
-            if (kFp8) { g = g * sg; u = u * su; }
             g = g + bg;
             u = u + bu;
             const float ex = __expf(-g);
@@ -261,7 +234,6 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(
     for (int j = 0; j < TN; ++j) {
       const int col = n0 + wn * WTN + j * 32 + lrow;
       if (col >= n_store) continue;
-      const float s = kFp8 ? wscale[(size_t)e * Npad + col] : 1.0f;
       const float b = bias0 ? bias0[(size_t)e * bias_ld + col] : 0.0f;
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
@@ -269,9 +241,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(
         for (int v = 0; v < 16; ++v) {
           const int row = row_base + i * 32 + 8 * (v / 4) + 4 * lhalf + (v % 4);
           if (row < ti.row_end) {
-            float o = acc[i][j][v];
-            if (kFp8) o = o * s;
-            store_act(out + (size_t)row * ldo + col, o + b);
+            store_act(out + (size_t)row * ldo + col, acc[i][j][v] + b);
           }
         }
       }
@@ -287,37 +257,26 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(
 // pre-activations SWIGLU_BWD reads (required).
 // DOWN and SWIGLU_BWD cover only the n-tiles that hold stored columns
 // (n_store; Npad is the weights' row stride).
-template <int BM, int BN, int WM, int WN, typename AT, typename WT, int EPI, typename OutT>
-hipError_t launch_grouped_gemm(const AT* A, const WT* B, const float* wscale, const float* bias0,
+template <int BM, int BN, int WM, int WN, int EPI>
+hipError_t launch_grouped_gemm(const bf16_t* A, const bf16_t* B, const float* bias0,
                                const float* bias1, const int32_t* counts, int E, int K, int Npad,
-                               int n_store, int bias_ld, OutT* out, int ldo, int max_mtiles,
-                               OutT* aux, int aux_ld, hipStream_t stream) {
+                               int n_store, int bias_ld, bf16_t* out, int ldo, int max_mtiles,
+                               bf16_t* aux, int aux_ld, hipStream_t stream) {
   if (max_mtiles <= 0) return hipSuccess;
   if (EPI == kEpiSwigluBwd && aux == nullptr) return hipErrorInvalidValue;
   const int ntiles = EPI == kEpiGateUp ? Npad / BN : std::min(Npad / BN, (n_store + BN - 1) / BN);
-  hipLaunchKernelGGL((grouped_gemm_kernel<BM, BN, WM, WN, AT, WT, EPI, OutT>),
-                     dim3(ntiles, max_mtiles), dim3(256), 0, stream, A, B, wscale, bias0, bias1,
+  hipLaunchKernelGGL((grouped_gemm_kernel<BM, BN, WM, WN, EPI>),
+                     dim3(ntiles, max_mtiles), dim3(256), 0, stream, A, B, bias0, bias1,
                      counts, E, K, Npad, n_store, bias_ld, out, ldo, aux, aux_ld);
   return hipGetLastError();
 }
 
-#define MGPT_INST_GEMM(BM, BN, WM, WN, AT, WT, EPI, OT)                                     \
-  template hipError_t launch_grouped_gemm<BM, BN, WM, WN, AT, WT, EPI, OT>(                 \
-      const AT*, const WT*, const float*, const float*, const float*, const int32_t*, int, int, \
-      int, int, int, OT*, int, int, OT*, int, hipStream_t);
-
-// Large-M tiles (prefill-shaped segments).
-MGPT_INST_GEMM(128, 128, 2, 2, bf16_t, bf16_t, kEpiGateUp, bf16_t)
-MGPT_INST_GEMM(128, 128, 2, 2, bf16_t, bf16_t, kEpiDown, bf16_t)
-MGPT_INST_GEMM(128, 128, 2, 2, bf16_t, fp8_t, kEpiGateUp, bf16_t)
-MGPT_INST_GEMM(128, 128, 2, 2, bf16_t, fp8_t, kEpiDown, bf16_t)
-// Small-M tiles (decode-shaped segments of a few rows per expert).
-MGPT_INST_GEMM(32, 256, 1, 4, bf16_t, bf16_t, kEpiGateUp, bf16_t)
-MGPT_INST_GEMM(32, 256, 1, 4, bf16_t, bf16_t, kEpiDown, bf16_t)
-MGPT_INST_GEMM(32, 256, 1, 4, bf16_t, fp8_t, kEpiGateUp, bf16_t)
-MGPT_INST_GEMM(32, 256, 1, 4, bf16_t, fp8_t, kEpiDown, bf16_t)
-// Backward data-gradient products (d(act) with the SwiGLU backward; dX).
-MGPT_INST_GEMM(128, 128, 2, 2, bf16_t, bf16_t, kEpiSwigluBwd, bf16_t)
-MGPT_INST_GEMM(32, 256, 1, 4, bf16_t, bf16_t, kEpiSwigluBwd, bf16_t)
+#define MGPT_INST_GEMM(EPI)                                                                  \
+  template hipError_t launch_grouped_gemm<128, 128, 2, 2, EPI>(                              \
+      const bf16_t*, const bf16_t*, const float*, const float*, const int32_t*, int, int, int, \
+      int, int, bf16_t*, int, int, bf16_t*, int, hipStream_t);
+MGPT_INST_GEMM(kEpiGateUp)
+MGPT_INST_GEMM(kEpiDown)
+MGPT_INST_GEMM(kEpiSwigluBwd)
 
 }  // namespace mgpt

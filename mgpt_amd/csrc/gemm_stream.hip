@@ -1,0 +1,439 @@
+// gemm_stream.hip -- grouped expert GEMMs whose weights are the larger
+// operand: bf16 weights under few rows per expert (decode steps, short
+// prompts), and fp8 weights at every row count the decode kernel does not
+// take.
+//
+// Same contract as gemm_dma.hip (A = expert-contiguous bf16 rows [rows][K],
+// B = packed weights [E][Npad][K], bf16 or e4m3 with per-output-channel
+// scales; gate/up, down and SwiGLU-backward epilogues) and the same frame:
+// a persistent block per CU walks BM x BN tiles in an order that shares
+// operand panels within an XCD, operands go HBM -> LDS by untracked
+// 1 KB loads, waves of 64 features x BM/2 tokens run
+// v_mfma_f32_32x32x16_bf16 on D = W . X^T.  What differs:
+//  * The ring holds ST stages, each a whole 64-column slab (BM rows of A, BN
+//    rows of B), ST - 1 slabs ahead.  With fp8 weights a slab is 48 KB (BM =
+//    256) instead of 64 KB, so both operands lead by two slabs in 144 KB; the
+//    64 x 128 tiles take 24 KB (bf16) or 16 KB (fp8) a slab, with 112 to 120 KB
+//    of loads in flight a CU, which a weight stream from HBM needs.
+//  * Within a slab, lane half h and k-step ks stand for columns 32h + 8ks ..
+//    +7 in both operands, so a lane's fp8 weights of two k-steps are one
+//    16-byte LDS read; they become bf16 in registers (exact).  fp8 rows are 64
+//    bytes: 16-byte chunk c of row r sits at slot c ^ ((r >> 2) & 3), which
+//    spreads the 16 lanes served together over all banks.
+//  * Scales and biases are applied after the contraction from scalar loads (a
+//    vector load would wait for the ring's loads as well).
+//  * Few rows take 64 x 128 tiles (4 waves): the narrower they are, the more
+//    evenly a step's few tiles spread over the CUs (16 experts of H = 2816:
+//    704 gate/up tiles are 2.75 rounds, 352 of 256 columns 1.4, paid as 2).
+//  * Where the tiles do not reach half the CUs and the contraction is long,
+//    they are split along K like gemm_dma's last round (us for the down product
+//    with and without, its reduction included, E = 16, C = 1024, H = 2816: 1
+//    token 14.8 / 22.7, 4 tokens 18.5 / 24.7, 24 tokens 27.2 / 29.7; H = 1408:
+//    24 tokens 19.3 / 17.5, so a contraction of 22 slabs stays whole).
+//
+// Measured on MI355X, stage times with cold weights, against the register-staged
+// 32 x 256 (bf16) and 128 x 128 (fp8) tiles used before, gate/up + down us:
+// bf16, C = 1024, H = 2816, E = 16, k = 2: 1 token 33 + 38 -> 14 + 15, 24
+// tokens 51 + 62 -> 43 + 27, 300 tokens 80 + 65 -> 46 + 34; C = 2048, H = 1408,
+// E = 64, k = 8 (1.1 GB of weights): 64 tokens 201 + 110 -> 164 + 75 (4.6 TB/s),
+// 400 tokens 310 + 193 -> 175 + 86.  fp8, the latter layer: 600 tokens 209 + 142
+// -> 128 + 73, 1999 tokens 356 + 236 -> 220 + 136 (840 TFLOP/s in gate/up),
+// 4096 tokens 585 + 389 -> 382 + 229.
+#include <type_traits>
+
+#include "gemm_ring.hpp"
+
+namespace mgpt {
+namespace {
+
+// e4m3 byte pair (low or high half of a dword) -> two bf16 in one dword.
+template <bool HI>
+__device__ __forceinline__ uint32_t e4m3x2_to_bf16x2(uint32_t packed) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const bf16x2_t v = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)packed, 1.0f, HI);
+  uint32_t r;
+  __builtin_memcpy(&r, &v, 4);
+  return r;
+}
+
+__device__ __forceinline__ bf16x8 fp8x8_to_bf16x8(uint32_t lo, uint32_t hi) {
+  const uint32_t w[4] = {e4m3x2_to_bf16x2<false>(lo), e4m3x2_to_bf16x2<true>(lo),
+                         e4m3x2_to_bf16x2<false>(hi), e4m3x2_to_bf16x2<true>(hi)};
+  bf16x8 r;
+  __builtin_memcpy(&r, w, 16);
+  return r;
+}
+
+constexpr int kStreamMinSlabs = 32;   // shorter contractions stay whole
+
+// acc = acc * scale + bias, per output feature (register v of a 32x32 tile
+// holds feature 8*(v/4) + 4*lhalf + v%4 of the tile, a token per lane);
+// scale null: 1, bias null: none.
+template <typename W>
+__device__ __forceinline__ void affine(f32x16 (&acc)[W::TN][W::TM], int j, const float* scale,
+                                       const float* bias, int lhalf) {
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int f = 8 * g + q;
+      float s = 1.0f, b = 0.0f;
+      if (scale) {
+        const float s0 = uniform_load(scale + f), s1 = uniform_load(scale + f + 4);
+        s = lhalf ? s1 : s0;
+      }
+      if (bias) {
+        const float b0 = uniform_load(bias + f), b1 = uniform_load(bias + f + 4);
+        b = lhalf ? b1 : b0;
+      }
+#pragma unroll
+      for (int i = 0; i < W::TM; ++i) {
+        float a = acc[j][i][4 * g + q];
+        if (scale) a = a * s;
+        acc[j][i][4 * g + q] = a + b;
+      }
+      // one feature at a time (keeps the scalar loads from piling up)
+      if (q & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+template <int EPI, typename WT, int NW, int BM, int BN, int ST, bool kSave>
+__global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
+    const bf16_t* __restrict__ A, const WT* __restrict__ B, const float* __restrict__ wscale,
+    const float* __restrict__ bias0, const float* __restrict__ bias1,
+    const int32_t* __restrict__ counts, int E, int e_base, int K, int Npad, int nbx,
+    int n_store, int bias_ld, bf16_t* out, int ldo, float* __restrict__ partials, bf16_t* save, int save_ld) {
+  using W = Waves<NW, BM, BN>;
+  constexpr int kTN = W::TN, kTM = W::TM;
+  constexpr bool kFp8 = sizeof(WT) == 1;
+  constexpr int kARow = 128, kBRow = 64 * (int)sizeof(WT);   // LDS bytes per row of a slab
+  constexpr int kABytes = BM * kARow, kBBytes = BN * kBRow;
+  constexpr int kStage = kABytes + kBBytes;
+  constexpr int kDA = kABytes / 1024 / NW, kDB = kBBytes / 1024 / NW, kD = kDA + kDB;   // loads per wave
+  constexpr int kBPer = 1024 / kBRow;                         // B rows per load
+  __shared__ __attribute__((aligned(1024))) char smem[ST * kStage];
+
+  const int G = gridDim.x;
+  int t = (G % kNumXcd == 0) ? (blockIdx.x % kNumXcd) * (G / kNumXcd) + blockIdx.x / kNumXcd
+                             : blockIdx.x;
+  const int KT = K / 64;
+  SegScan<BM> sc;
+  sc.init(counts, E, e_base);
+  SplitPlan plan;
+  plan.init(sc.tm * nbx, G, KT, partials != nullptr, kStreamMinSlabs);
+  Work cur;
+  if (!locate_work<BN>(sc, plan, E, nbx, KT, t, &cur)) return;
+
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = lane_id();
+  const int wn = w % W::WN, wm = w / W::WN;
+  const int lrow = lane & 31, lhalf = lane >> 5;
+
+  // Loads of a slab: wave w fills A rows w*BM/NW .. and B rows w*BN/NW ..  Lane
+  // offsets from the tile's first row; A chunk c of row r at slot c ^ ((r >>
+  // 1) & 7), B likewise (bf16) or c ^ ((r >> 2) & 3) of 64-byte rows (fp8).
+  uint32_t a_off[kDA], b_off[kDB];
+  int a_row[kDA];
+#pragma unroll
+  for (int i = 0; i < kDA; ++i) {
+    a_row[i] = (w * kDA + i) * 8 + lane / 8;
+    a_off[i] = (uint32_t)(((lane % 8) ^ ((a_row[i] >> 1) & 7)) * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < kDB; ++i) {
+    const int r = (w * kDB + i) * kBPer + lane / (kBRow / 16), s = lane % (kBRow / 16);
+    b_off[i] = (uint32_t)r * (uint32_t)(K * (int)sizeof(WT)) +
+               (uint32_t)((kFp8 ? s ^ ((r >> 2) & 3) : s ^ ((r >> 1) & 7)) * 16);
+  }
+  const uint32_t lds_a = (uint32_t)(uintptr_t)(lds_char*)smem + (uint32_t)(w * kDA * 1024);
+  const uint32_t lds_b = (uint32_t)(uintptr_t)(lds_char*)smem + (uint32_t)(kABytes + w * kDB * 1024);
+
+  // Cursor over slabs (work item dwk, slab dkt, ring stage dstage).  Past the
+  // end of the block's work it repeats the last slab (in bounds, into a freed
+  // stage), so every slab issues the same loads and waits the same way.
+  Work dwk = cur;
+  int dt = t, dkt = cur.k0, dstage = 0;
+  bool dvalid = true;
+  const char *dga, *dgb;
+  uint32_t ga_off[kDA];
+  auto enter_item = [&]() __attribute__((always_inline)) {
+    dga = reinterpret_cast<const char*>(A + (size_t)dwk.tile.row0 * K);
+    dgb = reinterpret_cast<const char*>(B + ((size_t)dwk.tile.expert * Npad + dwk.tile.n0) * K);
+    // (few rows: those past the segment re-read its last one, in L1)
+    const int rows = dwk.tile.row_end - dwk.tile.row0;
+#pragma unroll
+    for (int i = 0; i < kDA; ++i)
+      ga_off[i] = a_off[i] + (uint32_t)(BM <= 64 ? min(a_row[i], rows - 1) : a_row[i]) * (uint32_t)(K * 2);
+  };
+  enter_item();
+  const char *ua, *ub;   // the slab being issued
+  uint32_t uda, udb;
+  auto next_slab = [&]() __attribute__((always_inline)) {
+    ua = dga + (size_t)dkt * kARow;
+    ub = dgb + (size_t)dkt * kBRow;
+    uda = lds_a + (uint32_t)(dstage * kStage);
+    udb = lds_b + (uint32_t)(dstage * kStage);
+    dstage = dstage + 1 == ST ? 0 : dstage + 1;
+    if (dvalid && ++dkt == dwk.k1) {
+      dt += G;
+      Work nx;
+      dvalid = locate_work<BN>(sc, plan, E, nbx, KT, dt, &nx);
+      if (dvalid) {
+        dwk = nx;
+        dkt = dwk.k0;
+      } else {
+        --dkt;
+      }
+    }
+  };
+  int item_of_offs = t;   // the item that ga_off belongs to
+  auto issue = [&](int d0, int d1) __attribute__((always_inline)) {
+#pragma unroll
+    for (int d = d0; d < d1; ++d) {
+      if (d < kDA)
+        dma16(ua + ga_off[d], uda + d * 1024);
+      else
+        dma16(ub + b_off[d - kDA], udb + (d - kDA) * 1024);
+    }
+  };
+  // after the last loads of a slab: the offsets of the next one's item
+  auto settle = [&]() __attribute__((always_inline)) {
+    if (dvalid && dt != item_of_offs) {
+      item_of_offs = dt;
+      enter_item();
+    }
+  };
+  auto quarter = [&](int q) __attribute__((always_inline)) { issue(q * kD / 4, (q + 1) * kD / 4); };
+  auto slab_wait = [&]() __attribute__((always_inline)) {
+    slab_barrier<(ST - 2) * kD>();
+    settle();
+    next_slab();
+  };
+
+  const int swz = (lrow >> 1) & 7, swz4 = (lrow >> 2) & 3;
+  const char* x_base = smem + (wm * W::WTM + lrow) * kARow;
+  const char* w_base = smem + kABytes + (wn * W::WTN + lrow) * kBRow;
+  bf16x8 xf[2][kTM];
+  bf16x8 wf[2][kFp8 ? 1 : kTN];   // bf16 weights by k-step
+  uint4 wr[2][kFp8 ? kTN : 1];    // fp8 weights by pair of k-steps
+  auto frags = [&](int stage, int ks) __attribute__((always_inline)) {
+    const int cofs = ((4 * lhalf + ks) ^ swz) << 4;
+#pragma unroll
+    for (int i = 0; i < kTM; ++i)
+      xf[ks & 1][i] = *reinterpret_cast<const bf16x8*>(x_base + stage * kStage + i * 32 * kARow + cofs);
+    if constexpr (kFp8) {
+      if ((ks & 1) == 0) {
+        const int c4 = ((2 * lhalf + ks / 2) ^ swz4) << 4;
+#pragma unroll
+        for (int j = 0; j < kTN; ++j)
+          wr[(ks >> 1) & 1][j] =
+              *reinterpret_cast<const uint4*>(w_base + stage * kStage + j * 32 * kBRow + c4);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < kTN; ++j)
+        wf[ks & 1][j] =
+            *reinterpret_cast<const bf16x8*>(w_base + stage * kStage + j * 32 * kBRow + cofs);
+    }
+  };
+
+#pragma unroll
+  for (int s = 0; s < ST - 1; ++s) {
+    settle();
+    next_slab();
+    issue(0, kD);
+  }
+  slab_wait();
+  quarter(0);
+  int stage = 0;
+  frags(0, 0);
+
+  for (;;) {
+    Work nxt;
+    const bool have_next = locate_work<BN>(sc, plan, E, nbx, KT, t + G, &nxt);
+    f32x16 acc[kTN][kTM];
+#pragma unroll
+    for (int j = 0; j < kTN; ++j)
+#pragma unroll
+      for (int i = 0; i < kTM; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[j][i][v] = 0.0f;
+
+    // the k loop for MT live 32-token sub-tiles of this wave (as gemm_dma's)
+    auto kloop = [&](auto mt_c) __attribute__((always_inline)) {
+      constexpr int MT = decltype(mt_c)::value;
+      constexpr int kMfma = kTN * MT;
+      for (int kt = cur.k0; kt < cur.k1; ++kt) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          if (ks < 3) {
+            quarter(ks + 1);
+            frags(stage, ks + 1);
+          } else {
+            stage = stage + 1 == ST ? 0 : stage + 1;
+            slab_wait();
+            quarter(0);
+            frags(stage, 0);
+          }
+#pragma unroll
+          for (int j = 0; j < kTN; ++j) {
+            if constexpr (MT > 0) {
+              bf16x8 wv;
+              if constexpr (kFp8) {
+                const uint4 r = wr[(ks >> 1) & 1][j];
+                wv = (ks & 1) ? fp8x8_to_bf16x8(r.z, r.w) : fp8x8_to_bf16x8(r.x, r.y);
+              } else {
+                wv = wf[ks & 1][j];
+              }
+#pragma unroll
+              for (int i = 0; i < MT; ++i)
+                acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, xf[ks & 1][i], acc[j][i], 0, 0, 0);
+            }
+          }
+          constexpr int kReads = kTM + (kFp8 ? (1) : kTN);
+          constexpr int kPairs = kReads < kMfma ? kReads : kMfma;
+#pragma unroll
+          for (int q = 0; q < kPairs; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // one LDS read
+          }
+        }
+      }
+    };
+    const int wrows = cur.tile.row_end - (cur.tile.row0 + wm * W::WTM);
+    const int mt_live = wrows <= 0 ? 0 : min(kTM, (wrows + 31) / 32);
+    if constexpr (kTM == 4) {
+      switch (mt_live) {
+        case 0: kloop(IntC<0>{}); break;
+        case 1: kloop(IntC<1>{}); break;
+        case 2: kloop(IntC<2>{}); break;
+        case 3: kloop(IntC<3>{}); break;
+        default: kloop(IntC<4>{}); break;
+      }
+    } else if constexpr (kTM == 2) {
+      if (mt_live == 0) kloop(IntC<0>{});
+      else if (mt_live == 1) kloop(IntC<1>{});
+      else kloop(IntC<2>{});
+    } else {
+      if (mt_live == 0) kloop(IntC<0>{});
+      else kloop(IntC<1>{});
+    }
+    if (mt_live > 0) {
+      if (cur.sidx < 0) {
+        // the lane recomputed rather than kept live across the k loop (the 256-
+        // row tiles run at the register limit)
+        int lane_now;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_now));
+        const int lrow = lane_now & 31, lhalf = lane_now >> 5;
+        const size_t e = cur.tile.expert;
+        const int nw = cur.tile.n0 + wn * W::WTN;
+        if constexpr (EPI == kEpiGateUp) {
+          const int hb = nw / 2;   // [32 gate | 32 up] of units hb .. hb+31
+          affine<W>(acc, 0, kFp8 ? wscale + e * Npad + nw : nullptr, bias0 + e * bias_ld + hb, lhalf);
+          affine<W>(acc, 1, kFp8 ? wscale + e * Npad + nw + 32 : nullptr, bias1 + e * bias_ld + hb, lhalf);
+        } else if constexpr (EPI == kEpiDown) {
+#pragma unroll
+          for (int j = 0; j < kTN; ++j)
+            if (kFp8 || bias0)
+              affine<W>(acc, j, kFp8 ? wscale + e * Npad + nw + 32 * j : nullptr,
+                        bias0 ? bias0 + e * bias_ld + nw + 32 * j : nullptr, lhalf);
+        }
+        store_tile<EPI, W, kSave, true>(acc, cur.tile, wn, wm, lrow, lhalf, n_store, out, ldo, save, save_ld);
+      } else {
+        float4* P = reinterpret_cast<float4*>(partials + (size_t)cur.sidx * (BM * BN)) + tid;
+#pragma unroll
+        for (int j = 0; j < kTN; ++j)
+#pragma unroll
+          for (int i = 0; i < kTM; ++i)
+#pragma unroll
+            for (int v4 = 0; v4 < 4; ++v4)
+              P[((j * kTM + i) * 4 + v4) * W::kThreads] =
+                  make_float4(acc[j][i][4 * v4], acc[j][i][4 * v4 + 1], acc[j][i][4 * v4 + 2],
+                              acc[j][i][4 * v4 + 3]);
+      }
+    }
+    if (!have_next) break;
+    t += G;
+    cur = nxt;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the repeated tail loads
+}
+
+}  // namespace
+
+// Persistent launch, one block per CU.  Tiles of 64 rows x 128 features
+// (small) or 256 x 256.  partials (num_cus x 64 x 128 floats, small tiles
+// only, or null): the split last round's.  save: the training pre-activations
+// (gate/up: written; SwiGLU backward: read, bf16 weights only).  K % 64 == 0,
+// Npad % 256 == 0, n_store % 64 == 0; A has 256 rows of slack.
+template <int EPI, typename WT>
+hipError_t launch_gemm_stream(const bf16_t* A, const WT* B, const float* wscale, const float* bias0,
+                              const float* bias1, const int32_t* counts, int E, int K, int Npad,
+                              int n_store, int bias_ld, bf16_t* out, int ldo, size_t rows, bool small,
+                              float* partials, int num_cus, bf16_t* save, int save_ld,
+                              hipStream_t stream) {
+  constexpr bool kFp8 = sizeof(WT) == 1;
+  if (rows == 0) return hipSuccess;
+  if (E <= 0 || E > kMaxExpertsWide || K % 64 || Npad % 256 || n_store % 64 || num_cus <= 0 ||
+      ldo % 8 || (reinterpret_cast<uintptr_t>(out) & 15) ||
+      (save && (save_ld % 8 || (reinterpret_cast<uintptr_t>(save) & 15))) ||
+      (EPI == kEpiSwigluBwd && !save) || (kFp8 && (save || !wscale)))
+    return hipErrorInvalidValue;
+  const int BM = small ? 64 : 256, BN = small ? 128 : 256;
+  const int nt = EPI == kEpiGateUp ? Npad / BN : (n_store + BN - 1) / BN;
+  // more than 64 experts: one launch per group of 64 (as in gemm_dma.hip)
+  for (int e0 = 0; e0 < E; e0 += kMaxExperts) {
+    const int Eg = std::min(kMaxExperts, E - e0);
+    // at most this many tiles (an expert with rows has one more than its
+    // whole ones at most)
+    const long tiles = ((long)(rows / BM) + (long)std::min<size_t>(Eg, rows)) * nt;
+    const int KT = K / 64;
+    float* part = partials;
+    if (!small || save || KT < kStreamMinSlabs || 2 * tiles > num_cus) part = nullptr;
+    // (with split tiles every CU has work, also where there are fewer tiles)
+    const int grid = part ? num_cus : (int)std::min<long>(tiles, num_cus);
+    const WT* Bg = B + (size_t)e0 * Npad * K;
+    const float* sg = wscale ? wscale + (size_t)e0 * Npad : nullptr;
+    const float* b0 = bias0 ? bias0 + (size_t)e0 * bias_ld : nullptr;
+    const float* b1 = bias1 ? bias1 + (size_t)e0 * bias_ld : nullptr;
+    auto launch = [&](auto kernel, int threads) {
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, A, Bg, sg, b0, b1, counts, Eg, e0,
+                         K, Npad, nt, n_store, bias_ld, out, ldo, part, save, save_ld);
+    };
+    if constexpr (kFp8) {
+      if (small)
+        launch(gemm_stream_kernel<EPI, fp8_t, 4, 64, 128, 8, false>, 256);
+      else
+        launch(gemm_stream_kernel<EPI, fp8_t, 8, 256, 256, 3, false>, 512);
+    } else {
+      if (!small) return hipErrorInvalidValue;   // gemm_dma.hip's
+      if constexpr (EPI == kEpiGateUp) {
+        if (save)
+          launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, true>, 256);
+        else
+          launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, false>, 256);
+      } else {
+        launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, false>, 256);
+      }
+    }
+    if constexpr (EPI != kEpiSwigluBwd) {
+      if (part)
+        hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI, Waves<4, 64, 128>>), dim3(2 * grid), dim3(256),
+                           0, stream, part, sg, b0, b1, counts, Eg, e0, K, Npad, nt, n_store, bias_ld,
+                           out, ldo, grid, kStreamMinSlabs);
+    }
+  }
+  return hipGetLastError();
+}
+
+#define MGPT_INST_STREAM(EPI, WT)                                                                   \
+  template hipError_t launch_gemm_stream<EPI, WT>(                                                  \
+      const bf16_t*, const WT*, const float*, const float*, const float*, const int32_t*, int, int, \
+      int, int, int, bf16_t*, int, size_t, bool, float*, int, bf16_t*, int, hipStream_t);
+MGPT_INST_STREAM(kEpiGateUp, bf16_t)
+MGPT_INST_STREAM(kEpiDown, bf16_t)
+MGPT_INST_STREAM(kEpiSwigluBwd, bf16_t)
+MGPT_INST_STREAM(kEpiGateUp, fp8_t)
+MGPT_INST_STREAM(kEpiDown, fp8_t)
+
+}  // namespace mgpt

@@ -51,11 +51,15 @@ hipError_t launch_combine(const ActT*, const int32_t*, const float*, const int32
 template <typename T>
 hipError_t launch_copy_cols(const T*, int, T*, int, int, int, int, hipStream_t);
 hipError_t launch_add_jobs(const float*, const AddJobs&, size_t, hipStream_t);
-template <int BM, int BN, int WM, int WN, typename AT, typename WT, int EPI, typename OutT>
-hipError_t launch_grouped_gemm(const AT*, const WT*, const float*, const float*, const float*,
-                               const int32_t*, int, int, int, int, int, OutT*, int, int, OutT*,
+template <int BM, int BN, int WM, int WN, int EPI>
+hipError_t launch_grouped_gemm(const bf16_t*, const bf16_t*, const float*, const float*,
+                               const int32_t*, int, int, int, int, int, bf16_t*, int, int, bf16_t*,
                                int, hipStream_t);
 hipError_t launch_pack_transpose(const float*, int, int, float*, int, int, int, hipStream_t);
+template <int EPI, typename WT>
+hipError_t launch_gemm_stream(const bf16_t*, const WT*, const float*, const float*, const float*,
+                              const int32_t*, int, int, int, int, int, bf16_t*, int, size_t, bool,
+                              float*, int, bf16_t*, int, hipStream_t);
 template <int EPI>
 hipError_t launch_gemm_f32(const float*, const float*, const float*, const float*, const int32_t*,
                            int, int, int, int, int, float*, int, size_t, float*, int, int,
@@ -142,6 +146,7 @@ namespace {
 
 constexpr size_t kAlign = 256;
 constexpr size_t kGemmPartialBytes = 512 * 128 * 4;   // one 256x256 fp32 tile
+constexpr size_t kStreamPartialBytes = 64 * 128 * 4;   // one 64x128 fp32 tile
 constexpr int kRowPad = 256;   // rows of slack after activation buffers (GEMM tile overrun)
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -304,9 +309,19 @@ struct mgpt_moe {
     return act == MGPT_DTYPE_BF16 && wdt == MGPT_DTYPE_BF16 && gemm_tile == 256 &&
            (size_t)N * k >= (size_t)64 * E;
   }
+  // fp8 weights on the decode kernel's tiled copies: its 32-row tiles read the
+  // weights once per 32 rows of an expert, so past 40 rows on average the
+  // 256-row tiles of gemm_stream.hip are faster (us for both expert products
+  // on MI355X, E = 64, C = 2048, H = 1408: 33 rows per expert 175 against 185,
+  // 45 rows 201 against 191, 60 rows 234 against 195).
+  bool fp8_decode(int N) const {
+    return wgu_t && !wide() && (size_t)N * k < (size_t)40 * E;
+  }
   size_t w_bytes() const { return wdt == MGPT_DTYPE_FP8_E4M3 ? 1 : (wdt == MGPT_DTYPE_BF16 ? 2 : 4); }
   // h (SwiGLU output) is kept in the activation dtype.
-  Layout layout(int N, bool train = false) const {
+  // stream_part: with the weight-streaming GEMMs' partial tiles (bf16 weights,
+  // few rows per expert; those GEMMs also run without)
+  Layout layout(int N, bool train = false, bool stream_part = true) const {
     Layout L{};
     const size_t A = (size_t)N * k;
     const size_t TB = router_tokens_per_block(E);
@@ -333,7 +348,10 @@ struct mgpt_moe {
     L.hbuf = take((A + kRowPad) * Hp * act_bytes());
     L.obuf = take((A + kRowPad) * C * act_bytes());
     // fp32 partial tiles of the large-M GEMMs' split last round (one per CU)
-    L.partials = take(uses_gemm_dma(N) ? (size_t)num_cus * kGemmPartialBytes : 0);
+    // (one 64-row tile per CU for the weight-streaming ones)
+    L.partials = take(uses_gemm_dma(N) ? (size_t)num_cus * kGemmPartialBytes
+                      : wdt == MGPT_DTYPE_BF16 && stream_part ? (size_t)num_cus * kStreamPartialBytes
+                                                              : 0);
     L.rstd = take((size_t)N * 4);
     const size_t pad_rows = padded() ? (size_t)N * C * io_bytes() : 0;
     L.xpad = take(pad_rows);
@@ -788,9 +806,9 @@ struct BlockArgs {
 
 // IoT: the caller's x and y; ActT: the gathered rows, h and expert outputs.
 template <typename IoT, typename ActT>
-int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
+int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train, bool stream_part,
                  hipStream_t st, BlockArgs blk = BlockArgs()) {
-  const Layout L = h->layout(N, train);
+  const Layout L = h->layout(N, train, stream_part);
   const int C = h->C, Cx = h->Cx, E = h->E, k = h->k, Hp = h->Hp, Cp = h->Cp;
   const size_t A = (size_t)N * k;
   int32_t* idx = (int32_t*)(ws + L.topk_idx);
@@ -848,9 +866,8 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
   // training caches): the gate/up weight-streaming GEMM routes the ids
   // itself and reads the caller's rows of x (bf16, or fp32 rounded as the
   // permute would), so no permute runs.
-  const bool gather_decode = !train && !gamma && !h->wide() && h->wdt == MGPT_DTYPE_FP8_E4M3 &&
-                             h->wgu_t &&
-                             small_m(h, N) && A <= (size_t)kRouterTokens * kMaxTopK;
+  const bool gather_decode = !train && !gamma && h->fp8_decode(N) &&
+                             A <= (size_t)kRouterTokens * kMaxTopK;
   if (!gather_decode)
     HIP_TRY((launch_permute<IoT, ActT>(xi, idx, one_launch ? nullptr : hist, base, N, C, E, k,
                                        counts, perm, slot_of, xg, rstd, gamma, st)));
@@ -863,43 +880,53 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
                                       Cp, ob, C, A, nullptr, 0, h->num_cus, st));
   } else {
     const bool fp8 = h->wdt == MGPT_DTYPE_FP8_E4M3;
-    if (small_m(h, N)) {
+    const bool few = small_m(h, N);
+    // A down product too narrow for 256 x 256 tiles to reach the CUs goes by
+    // 64 x 128 ones: up to 1.5 of them per CU they are faster (us on MI355X,
+    // bf16, E = 16, C = 1024, H = 2816: 800 tokens 51 -> 34, 1120 (1.6 per CU)
+    // 52 -> 52; E = 8, C = 512, H = 1376: 1040 tokens 33 -> 17; fp8, the
+    // former's 640 tokens: 55 -> 30).
+    const bool narrow_down =
+        2 * (A / 64 + std::min<size_t>(E, A)) * ((C + 127) / 128) <= 3 * (size_t)h->num_cus;
+    float* part = (float*)(ws + L.partials);
+    if (h->fp8_decode(N)) {
+      // weight streaming: the persistent direct-to-LDS decode kernel on the
+      // tiled copies
       const int mt = (int)((A + 31) / 32) + E;
-      if (fp8 && h->wgu_t && !h->wide()) {
-        // weight streaming: the persistent direct-to-LDS decode kernel on the
-        // tiled copies
-        if (gather_decode)
-          HIP_TRY(launch_gemm_decode_gather<IoT>(xi, (const fp8_t*)h->wgu_t, h->sgu, h->bg, h->bu, idx,
-                                            (int)A, k, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, mt, counts,
-                                            perm, slot_of, st));
-        else
-          HIP_TRY(launch_gemm_decode<kEpiGateUp>(xg, (const fp8_t*)h->wgu_t, h->sgu, h->bg, h->bu,
-                                                 counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, mt,
-                                                 st));
-        HIP_TRY(mark(3));
-        HIP_TRY(launch_gemm_decode<kEpiDown>(hb, (const fp8_t*)h->wd_t, h->sd, h->bd, nullptr,
-                                             counts, E, Hp, Cp, C, Cp, ob, C, mt, st));
-      } else if (fp8) {
-        HIP_TRY((launch_grouped_gemm<32, 256, 1, 4, bf16_t, fp8_t, kEpiGateUp, bf16_t>(
-            xg, (const fp8_t*)h->wgu, h->sgu, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp, hb,
-            Hp, mt, nullptr, 0, st)));
-        HIP_TRY(mark(3));
-        HIP_TRY((launch_grouped_gemm<32, 256, 1, 4, bf16_t, fp8_t, kEpiDown, bf16_t>(
-            hb, (const fp8_t*)h->wd, h->sd, h->bd, nullptr, counts, E, Hp, Cp, C, Cp, ob, C, mt,
-            nullptr, 0, st)));
-      } else {
-        HIP_TRY((launch_grouped_gemm<32, 256, 1, 4, bf16_t, bf16_t, kEpiGateUp, bf16_t>(
-            xg, (const bf16_t*)h->wgu, nullptr, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp,
-            hb, Hp, mt, gu, 2 * Hp, st)));
-        HIP_TRY(mark(3));
-        HIP_TRY((launch_grouped_gemm<32, 256, 1, 4, bf16_t, bf16_t, kEpiDown, bf16_t>(
-            hb, (const bf16_t*)h->wd, nullptr, h->bd, nullptr, counts, E, Hp, Cp, C, Cp, ob, C,
-            mt, nullptr, 0, st)));
-      }
-    } else if (h->gemm_tile == 256 && !fp8) {
+      if (gather_decode)
+        HIP_TRY(launch_gemm_decode_gather<IoT>(xi, (const fp8_t*)h->wgu_t, h->sgu, h->bg, h->bu, idx,
+                                               (int)A, k, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, mt, counts,
+                                               perm, slot_of, st));
+      else
+        HIP_TRY(launch_gemm_decode<kEpiGateUp>(xg, (const fp8_t*)h->wgu_t, h->sgu, h->bg, h->bu,
+                                               counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, mt, st));
+      HIP_TRY(mark(3));
+      HIP_TRY(launch_gemm_decode<kEpiDown>(hb, (const fp8_t*)h->wd_t, h->sd, h->bd, nullptr, counts,
+                                           E, Hp, Cp, C, Cp, ob, C, mt, st));
+    } else if (fp8) {
+      // 256 x 256 tiles, except where the decode kernel's shape rules do not
+      // hold (width, more than 64 experts) and rows are few
+      HIP_TRY((launch_gemm_stream<kEpiGateUp, fp8_t>(
+          xg, (const fp8_t*)h->wgu, h->sgu, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, A,
+          A < (size_t)32 * E, nullptr, h->num_cus, nullptr, 0, st)));
+      HIP_TRY(mark(3));
+      HIP_TRY((launch_gemm_stream<kEpiDown, fp8_t>(hb, (const fp8_t*)h->wd, h->sd, h->bd, nullptr,
+                                                   counts, E, Hp, Cp, C, Cp, ob, C, A,
+                                                   A < (size_t)32 * E || narrow_down, nullptr, h->num_cus,
+                                                   nullptr, 0, st)));
+    } else if (few) {
+      // few rows per expert: the weights are the larger operand
+      float* sp = stream_part ? part : nullptr;
+      HIP_TRY((launch_gemm_stream<kEpiGateUp, bf16_t>(
+          xg, (const bf16_t*)h->wgu, nullptr, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, A,
+          true, sp, h->num_cus, (bf16_t*)gu, 2 * Hp, st)));
+      HIP_TRY(mark(3));
+      HIP_TRY((launch_gemm_stream<kEpiDown, bf16_t>(hb, (const bf16_t*)h->wd, nullptr, h->bd, nullptr,
+                                                    counts, E, Hp, Cp, C, Cp, ob, C, A, true, sp,
+                                                    h->num_cus, nullptr, 0, st)));
+    } else if (h->gemm_tile == 256) {
       // bf16 weights, prefill-shaped segments: 256x256 direct-to-LDS kernel.
       const int mt = (int)((A + 255) / 256) + E;
-      float* part = (float*)(ws + L.partials);
       // The gate/up GEMM has ~12x more tiles than CUs at prefill shapes, so a
       // partial last round costs little; only the down GEMM splits it
       // (splitting gate/up's last round too measured within noise at cfg2-cfg4).
@@ -907,27 +934,22 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
                                           2 * Hp, 2 * Hp, Hp, hb, Hp, mt, nullptr, h->num_cus,
                                           (bf16_t*)gu, 2 * Hp, st));
       HIP_TRY(mark(3));
-      HIP_TRY(launch_gemm_dma<kEpiDown>(hb, (const bf16_t*)h->wd, h->bd, nullptr, counts, E, Hp,
-                                        Cp, C, Cp, ob, C, mt, part, h->num_cus, nullptr, 0, st));
+      if (narrow_down)
+        HIP_TRY((launch_gemm_stream<kEpiDown, bf16_t>(hb, (const bf16_t*)h->wd, nullptr, h->bd, nullptr,
+                                                      counts, E, Hp, Cp, C, Cp, ob, C, A, true, part,
+                                                      h->num_cus, nullptr, 0, st)));
+      else
+        HIP_TRY(launch_gemm_dma<kEpiDown>(hb, (const bf16_t*)h->wd, h->bd, nullptr, counts, E, Hp,
+                                          Cp, C, Cp, ob, C, mt, part, h->num_cus, nullptr, 0, st));
     } else {
       const int mt = (int)((A + 127) / 128) + E;
-      if (fp8) {
-        HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, bf16_t, fp8_t, kEpiGateUp, bf16_t>(
-            xg, (const fp8_t*)h->wgu, h->sgu, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp, hb,
-            Hp, mt, nullptr, 0, st)));
-        HIP_TRY(mark(3));
-        HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, bf16_t, fp8_t, kEpiDown, bf16_t>(
-            hb, (const fp8_t*)h->wd, h->sd, h->bd, nullptr, counts, E, Hp, Cp, C, Cp, ob, C, mt,
-            nullptr, 0, st)));
-      } else {
-        HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, bf16_t, bf16_t, kEpiGateUp, bf16_t>(
-            xg, (const bf16_t*)h->wgu, nullptr, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp,
-            hb, Hp, mt, gu, 2 * Hp, st)));
-        HIP_TRY(mark(3));
-        HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, bf16_t, bf16_t, kEpiDown, bf16_t>(
-            hb, (const bf16_t*)h->wd, nullptr, h->bd, nullptr, counts, E, Hp, Cp, C, Cp, ob, C,
-            mt, nullptr, 0, st)));
-      }
+      HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, kEpiGateUp>(
+          xg, (const bf16_t*)h->wgu, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, mt, gu,
+          2 * Hp, st)));
+      HIP_TRY(mark(3));
+      HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, kEpiDown>(
+          hb, (const bf16_t*)h->wd, h->bd, nullptr, counts, E, Hp, Cp, C, Cp, ob, C, mt, nullptr, 0,
+          st)));
     }
   }
   HIP_TRY(mark(4));
@@ -1091,23 +1113,20 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
                                       (float*)(ws + L.partials), fork2 ? h->dx_cus : h->num_cus,
                                       nullptr, 0, st));
   } else if (small_m(h, N)) {
-    const int mt = (A + 31) / 32 + E;
-    HIP_TRY((launch_grouped_gemm<32, 256, 1, 4, bf16_t, bf16_t, kEpiSwigluBwd, bf16_t>(
-        dgo, wdb, nullptr, nullptr, nullptr, counts, E, C, h->Hq, Hp, 0, gu, 2 * Hp, mt, gu,
-        2 * Hp, st)));
+    HIP_TRY((launch_gemm_stream<kEpiSwigluBwd, bf16_t>(
+        (const bf16_t*)dgo, (const bf16_t*)wdb, nullptr, nullptr, nullptr, counts, E, C, h->Hq, Hp, 0,
+        (bf16_t*)gu, 2 * Hp, A, true, nullptr, h->num_cus, (bf16_t*)gu, 2 * Hp, st)));
     HIP_TRY(mark(2));
-    HIP_TRY((launch_grouped_gemm<32, 256, 1, 4, bf16_t, bf16_t, kEpiDown, bf16_t>(
-        gu, wgub, nullptr, nullptr, nullptr, counts, E, 2 * Hp, Cp, C, 0, ob, C, mt, nullptr, 0,
-        st)));
+    HIP_TRY((launch_gemm_stream<kEpiDown, bf16_t>(
+        (const bf16_t*)gu, (const bf16_t*)wgub, nullptr, nullptr, nullptr, counts, E, 2 * Hp, Cp, C, 0,
+        (bf16_t*)ob, C, A, true, (float*)(ws + L.partials), h->num_cus, nullptr, 0, st)));
   } else {
     const int mt = (A + 127) / 128 + E;
-    HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, bf16_t, bf16_t, kEpiSwigluBwd, bf16_t>(
-        dgo, wdb, nullptr, nullptr, nullptr, counts, E, C, h->Hq, Hp, 0, gu, 2 * Hp, mt, gu,
-        2 * Hp, st)));
+    HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, kEpiSwigluBwd>(
+        dgo, wdb, nullptr, nullptr, counts, E, C, h->Hq, Hp, 0, gu, 2 * Hp, mt, gu, 2 * Hp, st)));
     HIP_TRY(mark(2));
-    HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, bf16_t, bf16_t, kEpiDown, bf16_t>(
-        gu, wgub, nullptr, nullptr, nullptr, counts, E, 2 * Hp, Cp, C, 0, ob, C, mt, nullptr, 0,
-        st)));
+    HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, kEpiDown>(
+        gu, wgub, nullptr, nullptr, counts, E, 2 * Hp, Cp, C, 0, ob, C, mt, nullptr, 0, st)));
   }
   HIP_TRY(mark(3));
   if (!down_done)
@@ -1132,17 +1151,18 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
 
 // The forward for the handle's (boundary, compute) dtype pair.
 int dispatch_forward(mgpt_moe* h, const void* x, void* y, int N, char* ws, bool train,
-                     hipStream_t st, BlockArgs blk) {
+                     hipStream_t st, BlockArgs blk, bool stream_part = true) {
   if (h->act == MGPT_DTYPE_F32)
-    return forward_impl<float, float>(h, (const float*)x, (float*)y, N, ws, train, st, blk);
+    return forward_impl<float, float>(h, (const float*)x, (float*)y, N, ws, train, stream_part, st, blk);
   if (h->io == MGPT_DTYPE_F32)
-    return forward_impl<float, bf16_t>(h, (const float*)x, (float*)y, N, ws, train, st, blk);
-  return forward_impl<bf16_t, bf16_t>(h, (const bf16_t*)x, (bf16_t*)y, N, ws, train, st, blk);
+    return forward_impl<float, bf16_t>(h, (const float*)x, (float*)y, N, ws, train, stream_part, st, blk);
+  return forward_impl<bf16_t, bf16_t>(h, (const bf16_t*)x, (bf16_t*)y, N, ws, train, stream_part, st, blk);
 }
 
 // Shared argument checks of the forward entry points.
 int check_forward_args(const mgpt_moe* h, const void* x, const void* y, int num_tokens,
-                       const void* workspace, size_t workspace_bytes, bool train) {
+                       const void* workspace, size_t workspace_bytes, bool train,
+                       bool stream_part = true) {
   if (!h) return fail(MGPT_ERR_INVALID_ARGUMENT, "null handle");
   if (!h->loaded) return fail(MGPT_ERR_NOT_READY, "parameters not loaded");
   if (num_tokens < 0) return fail(MGPT_ERR_INVALID_ARGUMENT, "negative num_tokens");
@@ -1152,7 +1172,7 @@ int check_forward_args(const mgpt_moe* h, const void* x, const void* y, int num_
     return fail(MGPT_ERR_INVALID_ARGUMENT, "x and y must be 16-byte aligned");
   if ((uintptr_t)workspace % kAlign != 0)
     return fail(MGPT_ERR_INVALID_ARGUMENT, "workspace must be %zu-byte aligned", kAlign);
-  const size_t need = h->layout(num_tokens, train).total;
+  const size_t need = h->layout(num_tokens, train, stream_part).total;
   if (workspace_bytes < need)
     return fail(MGPT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu bytes < required %zu",
                 workspace_bytes, need);
@@ -1216,7 +1236,10 @@ int mgpt_moe_forward(mgpt_moe* h, const void* x, void* y, int num_tokens, void* 
 int mgpt_moe_forward_noalloc(mgpt_moe* h, const void* x, void* y, int num_tokens, void* stream) {
   if (!h) return fail(MGPT_ERR_INVALID_ARGUMENT, "null handle");
   if (num_tokens < 0) return fail(MGPT_ERR_INVALID_ARGUMENT, "negative num_tokens");
-  const size_t need = h->layout(num_tokens).total;
+  // the weight-streaming GEMMs' partial tiles only where the scratch has room
+  // for them too
+  const bool stream_part = h->layout(num_tokens).total <= (size_t)MGPT_MOE_NOALLOC_SCRATCH_BYTES;
+  const size_t need = h->layout(num_tokens, false, stream_part).total;
   if (need > (size_t)MGPT_MOE_NOALLOC_SCRATCH_BYTES)
     return fail(MGPT_ERR_WORKSPACE_TOO_SMALL,
                 "%d tokens need %zu workspace bytes; the built-in scratch holds %zu "
@@ -1224,12 +1247,13 @@ int mgpt_moe_forward_noalloc(mgpt_moe* h, const void* x, void* y, int num_tokens
                 num_tokens, need, (size_t)MGPT_MOE_NOALLOC_SCRATCH_BYTES);
   void* ws = nullptr;
   if (int rc = scratch_address(h->device, &ws)) return rc;
-  if (int rc = check_forward_args(h, x, y, num_tokens, ws, MGPT_MOE_NOALLOC_SCRATCH_BYTES, false))
+  if (int rc = check_forward_args(h, x, y, num_tokens, ws, MGPT_MOE_NOALLOC_SCRATCH_BYTES, false,
+                                  stream_part))
     return rc;
   if (num_tokens == 0) return MGPT_OK;
   HIP_TRY(hipSetDevice(h->device));
   return dispatch_forward(h, x, y, num_tokens, (char*)ws, false, (hipStream_t)stream,
-                          BlockArgs());
+                          BlockArgs(), stream_part);
 }
 
 int mgpt_moe_forward_block(mgpt_moe* h, const void* x, const float* gamma, float eps, void* out,

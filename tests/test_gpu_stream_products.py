@@ -1,0 +1,71 @@
+"""The weight-streaming expert products (gemm_stream.hip) at the edges of what
+they take: bf16 weights under 64 rows per expert (and narrow down products
+above), fp8 weights outside the decode kernel's range.  Segments that end
+inside, at and one past a 64- or 256-row tile, one token, contractions of one
+slab and of enough slabs to be split along K, widths that are not a multiple of
+128, more experts than a launch takes, and training through the 64-row tiles.
+Against the oracle at the layer's bars (bf16 2e-2, fp8 6e-2 of the fp32 path,
+which rounds the rows and products in between), and against the same rows one
+token at a time, which other tiles and splits compute, at a few bf16 roundings.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as O
+from mgpt_amd import workload as wl
+from mgpt_amd.moe import MoELayer
+
+pytestmark = pytest.mark.gpu
+
+# (N, C, E, k, H, weights)
+SHAPES = [
+    (1, 64, 4, 2, 64, "bf16"), (1, 1024, 16, 2, 2816, "bf16"), (24, 1024, 4, 2, 2112, "bf16"),
+    (63, 192, 3, 1, 96, "bf16"), (130, 320, 2, 1, 4096, "bf16"), (257, 256, 4, 2, 2560, "bf16"),
+    (900, 128, 4, 2, 3000, "bf16"), (70, 64, 70, 2, 40, "bf16"),
+    (255, 128, 1, 1, 128, "fp8"), (257, 128, 1, 1, 192, "fp8"), (300, 192, 3, 2, 160, "fp8"),
+    (40, 192, 3, 2, 160, "fp8"), (600, 256, 8, 3, 1408, "fp8"), (260, 128, 80, 3, 96, "fp8"),
+    (9, 128, 70, 2, 96, "fp8"),
+]
+
+
+@pytest.mark.parametrize("N,C,E,k,H,weights", SHAPES)
+def test_forward_against_the_oracle(N, C, E, k, H, weights):
+    cfg = wl.MoEConfig("stream", N, C, E, k, H, "bf16", weights, "normal")
+    inp = wl.make_inputs(cfg, seed=N + C, bias_std=0.05)
+    layer = MoELayer(C, H, E, k, act="bf16", weights=weights)
+    layer.load_parameters(inp.params(raw=True))
+    x = torch.from_numpy(inp.x).to("cuda").bfloat16()
+    y = layer.forward(x)
+    idx = layer.routing()["topk_idx"].cpu().numpy()
+    ref = O.forward(inp)
+    assert np.array_equal(idx, ref["idx"])
+    bar = 2e-2 if weights == "bf16" else 6e-2
+    err = np.linalg.norm(y.float().cpu().numpy() - ref["y"]) / np.linalg.norm(ref["y"])
+    assert err < bar, err
+    again = layer.forward(x)
+    assert torch.equal(y, again)
+    # a few of the rows by themselves: h and the output are rounded to bf16 (2^-9
+    # each), sums differ by fp32 roundings, so within two bf16 steps of the row
+    for t in sorted({0, N // 2, N - 1}):
+        one = layer.forward(x[t:t + 1].contiguous()).float()
+        scale = y[t].float().abs().max()
+        assert (one[0] - y[t].float()).abs().max() <= 2.0 ** -6 * scale, t
+
+
+@pytest.mark.parametrize("N,C,E,k,H", [(24, 128, 8, 2, 256), (70, 192, 6, 3, 100), (1, 64, 2, 1, 2100)])
+def test_training_through_few_rows(N, C, E, k, H):
+    cfg = wl.MoEConfig("stream", N, C, E, k, H, "bf16", "bf16", "normal")
+    inp = wl.make_inputs(cfg, seed=N, bias_std=0.05)
+    dy = wl.bf16_round(wl.normal_f32(5, 1, N * C).reshape(N, C))
+    layer = MoELayer(C, H, E, k, act="bf16")
+    layer.load_parameters(inp.params())
+    layer.forward(torch.from_numpy(inp.x).to("cuda").bfloat16(), train=True)
+    dx = layer.backward(torch.from_numpy(dy).to("cuda").bfloat16())
+    ref = O.backward(inp, dy)
+    g = [t.cpu().numpy() for t in layer.get_gradients()]
+    got = [dx.float().cpu().numpy(), g[0], g[1]]
+    got += [np.stack([g[2 + 6 * e + i] for e in range(E)]) for i in range(6)]
+    for name, a in zip(("dx",) + tuple(O.GRAD_NAMES), got):
+        b = np.asarray(ref[name], np.float64).reshape(a.shape)
+        assert np.linalg.norm(a - b) <= 2e-2 * np.linalg.norm(b) + 1e-12, name
