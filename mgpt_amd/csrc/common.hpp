@@ -38,6 +38,14 @@ __host__ __device__ inline int router_tokens_per_block(int /*E*/) { return kRout
 // fp32, 32 KB at this width).
 constexpr int kDecodeRouterMaxC = 8192;
 
+// The calls that the one-launch decode router takes: one router block of
+// tokens, a wave of experts, plain rows (us of the router stage on MI355X with
+// the fused kernel and with this one, 24 tokens: E = 8, C = 512 11.2 -> 8.5; E =
+// 16, C = 1024 25.6 -> 11.0; E = 16, C = 2048 46 -> 16).
+__host__ __device__ inline bool router_decode_range(int N, int C, int E, bool norm) {
+  return N <= kRouterTokens && E <= kMaxExperts && !norm && C % 64 == 0 && C <= kDecodeRouterMaxC;
+}
+
 // Router experts per wave (the router block has ceil(E / RE) <= 16 waves);
 // router weights are packed [ceil(E/RE)][C][RE], zero-padded.  Two experts
 // per wave share the activation loads and conversions of their chains:

@@ -223,8 +223,8 @@ struct mgpt_moe {
   int num_cus = 0;         // compute units of the device (persistent grids)
   int gemm_tile = 256;     // block tile of the large-M bf16 GEMMs (256 or 128)
   float* wr_g = nullptr;   // router weights [G][C][RE] (router_experts_per_wave)
-  float* wr1 = nullptr;    // router weights [E][C] (split decode router, E > 16)
-  float* wr4 = nullptr;    // router weights [C/4][E][4] (one-launch decode router, E > 16)
+  float* wr1 = nullptr;    // router weights [E][C] (a block or wave per expert)
+  float* wr4 = nullptr;    // router weights [C/4][E][4] (an expert per lane; null: too wide)
   float* br = nullptr;     // [E]
   void* wgu = nullptr;     // [E][2Hp][C] of bf16 / fp8 / f32
   void* wd = nullptr;      // [E][Cp][Hp]
@@ -287,17 +287,17 @@ struct mgpt_moe {
   size_t act_bytes() const { return act == MGPT_DTYPE_BF16 ? 2 : 4; }
   size_t io_bytes() const { return io == MGPT_DTYPE_BF16 ? 2 : 4; }
   bool padded() const { return Cx != C; }
-  // Few tokens and many experts: the router's logits are spread over more
-  // blocks (one expert per wave) instead of one block per 64 tokens.
-  bool router_split(int N) const { return E > 16 && (N < 4096 || wide()); }
   // more experts than a wave has lanes: the forward's generic paths only
   bool wide() const { return E > kMaxExperts; }
   // one router block of tokens: logits and softmax in one launch, and the
   // permute counts the ids itself (no histogram)
   bool router_one_launch(int N, bool norm) const {
-    return wr4 && !wide() && N <= kRouterTokens && !norm && C % 64 == 0 &&
-           C <= kDecodeRouterMaxC;
+    return wr4 && router_decode_range(N, C, E, norm);
   }
+  // Where the router may keep its logits [N][E]: a region of their own for few
+  // tokens and many experts (E > 16), else the expert outputs' region, which
+  // is written only after them, if they fit there.
+  bool logits_region(int N) const { return E > 16 && (N < 4096 || wide()); }
   // The bf16 large-M path (gemm_dma.hip), which may split its last round.
   // bias partials of the weight gradients' row chunks: at most 64 chunks of
   // the wider tile row (2Hp gate/up columns or C down columns) of
@@ -309,13 +309,17 @@ struct mgpt_moe {
     return act == MGPT_DTYPE_BF16 && wdt == MGPT_DTYPE_BF16 && gemm_tile == 256 &&
            (size_t)N * k >= (size_t)64 * E;
   }
-  // fp8 weights on the decode kernel's tiled copies: its 32-row tiles read the
-  // weights once per 32 rows of an expert, so past 40 rows on average the
-  // 256-row tiles of gemm_stream.hip are faster (us for both expert products
+  // fp8 weights on the decode kernel's tiled copies, up to 64 rows per expert on
+  // average.  Its 32-row tiles read the weights once per 32 rows of an expert,
+  // so past 40 rows the 256-row tiles of gemm_stream.hip are faster where the
+  // gate/up product has enough of them, two a CU (us for both expert products
   // on MI355X, E = 64, C = 2048, H = 1408: 33 rows per expert 175 against 185,
-  // 45 rows 201 against 191, 60 rows 234 against 195).
+  // 45 rows 201 against 191, 60 rows 234 against 195; E = 16, C = 1024, H =
+  // 2816, 1.4 tiles a CU: 60 rows 80 against 82; a layer of E = 16, C = 512, H =
+  // 1376, 0.7 a CU: 56 rows 61 against 68).
   bool fp8_decode(int N) const {
-    return wgu_t && !wide() && (size_t)N * k < (size_t)40 * E;
+    const size_t rows = (size_t)E * ((2 * Hp + 255) / 256) >= (size_t)2 * num_cus ? 40 : 64;
+    return wgu_t && !wide() && (size_t)N * k < rows * E;
   }
   size_t w_bytes() const { return wdt == MGPT_DTYPE_FP8_E4M3 ? 1 : (wdt == MGPT_DTYPE_BF16 ? 2 : 4); }
   // h (SwiGLU output) is kept in the activation dtype.
@@ -340,9 +344,8 @@ struct mgpt_moe {
     L.base = take(nb * E * 4);
     L.counts = take((size_t)E * 4);
     // Sized for min(N, 4095) tokens whenever E > 16, so that the workspace
-    // never shrinks as N grows past the split router's range.
-    // (every N when E > 64: the wide forward always routes through the
-    // split logits)
+    // never shrinks as N grows past 4095 (every N when E > 64: the wide
+    // forward always routes through the logits)
     L.logits = take(E > 16 ? (size_t)(wide() ? N : std::min(N, 4095)) * E * 4 : 0);
     L.xg = take((A + kRowPad) * C * act_bytes());
     L.hbuf = take((A + kRowPad) * Hp * act_bytes());
@@ -605,8 +608,8 @@ int mgpt_moe_load_parameters(mgpt_moe* h, const float* const* params, int num_pa
   const bool first = h->wgu == nullptr;
   if (first) {
     HIP_TRY(hipMalloc(&h->wr_g, sizeof(float) * ((E + RE - 1) / RE) * RE * C));
-    if (E > 16) HIP_TRY(hipMalloc(&h->wr1, sizeof(float) * E * C));
-    if (E > 16 && C % 64 == 0 && C <= kDecodeRouterMaxC)
+    HIP_TRY(hipMalloc(&h->wr1, sizeof(float) * E * C));
+    if (C % 64 == 0 && C <= kDecodeRouterMaxC)
       HIP_TRY(hipMalloc(&h->wr4, sizeof(float) * E * C));
     HIP_TRY(hipMalloc(&h->br, sizeof(float) * E));
     HIP_TRY(hipMalloc(&h->bg, sizeof(float) * E * Hp));
@@ -852,13 +855,15 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
       gamma = gp;
     }
   }
-  float* logits = h->router_split(N) ? (float*)(ws + L.logits) : nullptr;
+  float* logits = h->logits_region(N) ? (float*)(ws + L.logits)
+                  : (size_t)N * E * 4 <= (A + kRowPad) * C * sizeof(ActT) ? (float*)ob
+                                                                           : nullptr;
   // training: keep the router probabilities and the gate/up pre-activations
   float* probs = train ? (float*)(ws + L.probs) : nullptr;
   ActT* gu = train ? (ActT*)(ws + L.gu) : nullptr;
   float* rstd = gamma ? (float*)(ws + L.rstd) : nullptr;
   const bool one_launch = h->router_one_launch(N, gamma != nullptr);
-  HIP_TRY(launch_router<IoT>(xi, h->wr_g, h->wr1, one_launch ? h->wr4 : nullptr, h->br, N, C, E,
+  HIP_TRY(launch_router<IoT>(xi, h->wr_g, h->wr1, h->wr4, h->br, N, C, E,
                              k, idx, topp, hist, logits,
                              probs, gamma, blk.eps, Cx, rstd, st));
   HIP_TRY(mark(1));

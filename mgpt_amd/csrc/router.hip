@@ -888,6 +888,93 @@ __global__ __launch_bounds__(256) void router_logits_pc_kernel(
   }
 }
 
+// Logits with an expert per lane: a wave owns T tokens and 64 experts
+// (blockIdx.y the group of 64).  x[t][c] is the same for every lane, so it is
+// read with scalar loads and widened on the scalar unit, a batch of CB columns
+// ahead; W_r comes from its column quads wr4 = [C/4][E][4] (1 KB contiguous a
+// load), a batch ahead in registers.  The vector ALU then issues one product
+// and one add a term and nothing else, no LDS and no barrier; its rate is the
+// bound with several waves a SIMD, the latency of the scalar loads with one
+// (about 1000 cycles a batch; weights three batches ahead measured the same).
+// So T grows with the work.  The rounding sequence is the other kernels' (c ascending, one rounded
+// product and one rounded add per term, the bias last).  hist[e][block] is
+// cleared for router_softmax_wave_kernel.
+template <typename ActT, int T>
+__global__ __launch_bounds__(256) void router_logits_lane_kernel(
+    const ActT* __restrict__ x, const float4* __restrict__ wr4, const float* __restrict__ br, int N,
+    int C, int E, float* __restrict__ logits, int32_t* __restrict__ hist, int nb) {
+  constexpr int kPerDw = 4 / (int)sizeof(ActT);        // columns per dword of x
+  constexpr int CB = 32 * kPerDw / T < 32 ? 32 * kPerDw / T : 32;   // 32 dwords of x a batch
+  constexpr int kDw = CB / kPerDw;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), lane = lane_id();
+  const int tok0 = (blockIdx.x * 4 + w) * T;
+  const int e = blockIdx.y * kWave + lane, ee = min(e, E - 1);
+  if (tok0 >= N) return;
+  if (hist && tok0 % kRT == 0 && e < E) hist[(size_t)e * nb + tok0 / kRT] = 0;
+  const uint32_t* xr[T];
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+    xr[i] = reinterpret_cast<const uint32_t*>(x + (size_t)min(tok0 + i, N - 1) * C);
+  const float4* wp = wr4 + ee;
+  float acc[T];
+#pragma unroll
+  for (int i = 0; i < T; ++i) acc[i] = 0.0f;
+  const int nbat = C / CB;
+  auto load_x = [&](int j, uint32_t (&xs)[T][kDw]) __attribute__((always_inline)) {
+    const int d0 = min(j, nbat - 1) * kDw;
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+      for (int d = 0; d < kDw; ++d) xs[i][d] = xr[i][d0 + d];
+  };
+  auto load_w = [&](int j, float4 (&ws)[CB / 4]) __attribute__((always_inline)) {
+    const size_t q0 = (size_t)min(j, nbat - 1) * (CB / 4);
+#pragma unroll
+    for (int q = 0; q < CB / 4; ++q) ws[q] = wp[(q0 + q) * E];
+  };
+  auto add = [&](const uint32_t (&xs)[T][kDw], const float4 (&ws)[CB / 4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < CB; ++c) {
+      const float4& q = ws[c / 4];
+      const float wv = (c & 3) == 0 ? q.x : (c & 3) == 1 ? q.y : (c & 3) == 2 ? q.z : q.w;
+#pragma unroll
+      for (int i = 0; i < T; ++i) {
+        const uint32_t d = xs[i][c / kPerDw];
+        const float xv = __uint_as_float(kPerDw == 1 ? d : (c & 1) ? (d & 0xFFFF0000u) : (d << 16));
+        acc[i] = acc[i] + xv * wv;
+      }
+    }
+  };
+  uint32_t xs[2][T][kDw];
+  float4 ws[2][CB / 4];
+  load_x(0, xs[0]);
+  load_w(0, ws[0]);
+  auto step = [&](int j, auto s_c) __attribute__((always_inline)) {
+    constexpr int st = decltype(s_c)::value;
+    // Scalar loads return in any order, so a wait for one batch waits for all
+    // of them: batch j is waited for here, before batch j + 1 is requested.
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+      for (int d = 0; d < kDw; ++d) asm volatile("" : "+s"(xs[st][i][d]));
+    __builtin_amdgcn_sched_barrier(0);
+    load_x(j + 1, xs[st ^ 1]);
+    load_w(j + 1, ws[st ^ 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    add(xs[st], ws[st]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int j = 0; j < nbat; j += 2) {   // an even number of batches
+    step(j, IntC<0>{});
+    step(j + 1, IntC<1>{});
+  }
+  if (e >= E) return;
+  const float b = br[e];
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+    if (tok0 + i < N) logits[(size_t)(tok0 + i) * E + e] = acc[i] + b;
+}
+
 // Softmax, top-k and histogram for decode shapes: one wave per token, lane e
 // holding expert e (E <= 64), the row in LDS.  Every lane computes the
 // row's reductions itself, in the reference's order: the running max from
@@ -984,7 +1071,7 @@ __global__ __launch_bounds__(kSoftmaxWaves * 64) void router_softmax_wave_kernel
   softmax_topk_wave(l, valid, t, e, E, k, row, s_tab, topk_idx, topk_p, hist, nb, probs);
 }
 
-// Decode router for a single block of tokens (N <= 64, E > 16, no
+// Decode router for a single block of tokens (N <= 64, E <= 64, no
 // normalisation), logits and softmax in one launch.  A block owns one token
 // t: wave 0 runs the 64 chains acc = acc + p[c] (lane e = expert e, columns
 // ascending, then the bias: the reference's rounding sequence, as in the
@@ -1214,16 +1301,16 @@ __global__ __launch_bounds__(256) void router_decode_kernel(
 
 }  // namespace
 
-// logits == nullptr: the fused kernel.  Otherwise (E > 16, few tokens) the
-// split path through logits [N][E] (wr1 = W_r as [E][C]).  probs (nullable)
-// receives the clamped softmax [N][E] (the reference's cached_router_probs).
+// logits [N][E] (nullable: the fused kernel), for the paths that keep them in
+// memory; wr1: W_r as [E][C]; wr4 (nullable): W_r as column quads [C/4][E][4].
+// probs (nullable) receives the clamped softmax [N][E] (the reference's
+// cached_router_probs).
 // gamma (nullable): route on RMSNorm(x) * gamma instead of x, writing each
 // token's 1/rms to rstd [N]; cn: the mean's divisor (C, or the caller's width
 // when x's rows are zero-padded to C).
 //
-// wr4 (W_r as column quads [C/4][E][4]) set: the one-launch decode router,
-// for N <= 64, E > 16, no normalisation and C a multiple of 64 up to
-// kDecodeRouterMaxC; it writes no histogram (hist is unused).
+// In the decode range (router_decode_range) with wr4 set, one launch does it
+// all and writes no histogram (hist is unused).
 template <typename ActT>
 hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, const float* wr4,
                          const float* br, int N, int C, int E, int k, int32_t* topk_idx,
@@ -1232,12 +1319,34 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
   const RowNorm nrm{gamma, eps, cn};
   const int nb = (N + kRT - 1) / kRT;
   if (nb == 0) return hipSuccess;
+  const int eg = (E + kMaxExperts - 1) / kMaxExperts;
+  // The expert-per-lane logits, T tokens a wave by the number of (token, group
+  // of 64 experts) pairs (us of the router stage on MI355X, T = 1 / 2 / 4, C =
+  // 2048, E = 64: 1024 tokens 37 / 47 / 66, 2048 49 / 52 / 67, 4096 90 / 62 /
+  // 72, 8192 158 / 105 / 89).
+  auto lane_logits = [&]() {
+    const long pairs = (long)N * eg;
+    auto go = [&](auto kernel, int T) {
+      hipLaunchKernelGGL(kernel, dim3((N + 4 * T - 1) / (4 * T), eg), dim3(256), 0, stream, x,
+                         reinterpret_cast<const float4*>(wr4), br, N, C, E, logits, hist, nb);
+    };
+    if (pairs <= 2048)
+      go(router_logits_lane_kernel<ActT, 1>, 1);
+    else if (pairs <= 6144)
+      go(router_logits_lane_kernel<ActT, 2>, 2);
+    else
+      go(router_logits_lane_kernel<ActT, 4>, 4);
+  };
   if (E > kMaxExperts) {
     // wide: per-expert logits (the split kernels, any E), then the block
     // softmax / top-k over rows of up to kMaxExpertsWide
-    if (E > kMaxExpertsWide || !logits || wr4) return hipErrorInvalidValue;
-    const int eg = (E + kMaxExperts - 1) / kMaxExperts;
-    if (nb * eg >= 256 && router_experts_per_wave(E) == 4) {
+    if (E > kMaxExpertsWide || !logits) return hipErrorInvalidValue;
+    if (!gamma && wr4 && (long)N * eg >= 1024) {
+      // a wave a token and 64 experts from one wave per SIMD on (us with the
+      // kernels below: E = 128, C = 1024: 512 tokens 41 -> 37, 2048 94 -> 45,
+      // 8191 103 -> 91; 65 tokens 30 -> 36, which stay below)
+      lane_logits();
+    } else if (nb * eg >= 256 && router_experts_per_wave(E) == 4) {
       // enough (token block, 64 experts) blocks to fill the chip
       if (gamma)
         hipLaunchKernelGGL((router_logits_wide_kernel<ActT, true>), dim3(nb, eg), dim3(1024), 0,
@@ -1261,32 +1370,41 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
                          stream, logits, N, E, k, topk_idx, topk_p, hist, nb, probs);
     return hipGetLastError();
   }
-  if (wr4) {
-    if (N > kRT || E <= 16 || E > kMaxExperts || gamma || C % 64 || C > kDecodeRouterMaxC)
-      return hipErrorInvalidValue;
+  if (router_decode_range(N, C, E, gamma != nullptr) && wr4) {
     hipLaunchKernelGGL((router_decode_kernel<ActT>), dim3(N), dim3(256), 0, stream, x,
                        reinterpret_cast<const float4*>(wr4), br, N, C, E, k, topk_idx, topk_p,
                        probs);
     return hipGetLastError();
   }
-  if (logits && !gamma) {
-    // decode shapes without normalisation: products and chains on separate
-    // waves, then the softmax / top-k with one wave per token
-    hipLaunchKernelGGL((router_logits_pc_kernel<ActT>), dim3(nb, E), dim3(256), 0, stream, x, wr1,
-                       br, N, C, E, logits, hist, nb);
+  // Without normalisation the logits go through memory, with more blocks than
+  // the fused kernel's one per 64 tokens, while those do not fill the chip.
+  // Measured on MI355X (us of the router stage, separate product and chain
+  // waves / an expert per lane / fused):
+  //   E = 16, C = 1024: 512 tokens 16 / - / 27, 2048 19 / 28 / 27, 4096 28 / 33 / 28
+  //   E = 32, C = 1024: 1024 tokens 19 / 23 / 45, 2048 28 / 28 / 45, 4096 47 / 34 / 46,
+  //                     8192 - / 50 / 48
+  //   E = 64, C = 2048: 512 tokens 25 / 36 / 128, 1024 41 / 37 / 128, 2048 73 / 49 / 130,
+  //                     4096 134 / 62 / 132, 8192 - / 89 / 137, 32768 - / 257 / 287
+  //   E = 8, C = 512: 512 tokens 15 / - / 12
+  // An expert per lane costs 16 us and 4 us per 1000 tokens and 64 experts (C =
+  // 1024), the fused kernel 1.25 us per expert and round of 256 blocks.
+  const bool many = (long)N * E >= 57344;
+  const bool lane = many && wr4 && 4L * N + 16000 < 1250L * E * ((N + 16383) / 16384);
+  if (logits && !gamma && E > 8 && (lane || (E > 16 ? N < 4096 : !many))) {
+    if (lane)
+      lane_logits();
+    else
+      hipLaunchKernelGGL((router_logits_pc_kernel<ActT>), dim3(nb, E), dim3(256), 0, stream, x, wr1,
+                         br, N, C, E, logits, hist, nb);
     hipLaunchKernelGGL(router_softmax_wave_kernel, dim3((N + kSoftmaxWaves - 1) / kSoftmaxWaves),
                        dim3(kSoftmaxWaves * kWave), 0, stream, logits, N, E, k, topk_idx, topk_p,
                        hist, nb, probs);
     return hipGetLastError();
   }
-  if (logits) {
+  if (logits && gamma && E > 16 && N < 4096) {
     const dim3 lg(nb, (E + kSplitExperts - 1) / kSplitExperts), lb(kSplitExperts * kWave);
-    if (nrm.gamma)
-      hipLaunchKernelGGL((router_logits_kernel<ActT, true>), lg, lb, 0, stream, x, wr1, br, N, C,
-                         E, logits, nrm, rstd);
-    else
-      hipLaunchKernelGGL((router_logits_kernel<ActT, false>), lg, lb, 0, stream, x, wr1, br, N, C,
-                         E, logits, nrm, rstd);
+    hipLaunchKernelGGL((router_logits_kernel<ActT, true>), lg, lb, 0, stream, x, wr1, br, N, C, E,
+                       logits, nrm, rstd);
     hipLaunchKernelGGL(router_softmax_kernel, dim3(nb), dim3(MGPT_SOFTMAX_THREADS), 0, stream,
                        logits, N, E, k,
                        topk_idx, topk_p, hist, nb, probs);

@@ -1,0 +1,53 @@
+"""Every way the router forms its logits routes bit for bit like the oracle:
+the one-launch kernel at 1 to 64 experts, separate product and chain waves, an
+expert per lane (1, 2 and 4 tokens a wave, 1 to 8 groups of 64 experts) and the
+fused kernel, on both sides of each line between them, with token counts that
+leave blocks and waves partly filled, training (router probabilities) included.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as O
+from mgpt_amd import workload as wl
+from mgpt_amd.moe import MoELayer
+
+pytestmark = pytest.mark.gpu
+
+# (N, C, E, k, act)
+SHAPES = [
+    # one launch: up to 64 tokens, any width that is a multiple of 64
+    (1, 64, 1, 1, "f32"), (64, 64, 2, 2, "bf16"), (63, 128, 8, 2, "f32"), (17, 1024, 16, 2, "bf16"),
+    (64, 576, 9, 8, "bf16"), (5, 2048, 33, 3, "f32"),
+    # product and chain waves; fused below nine experts
+    (65, 128, 8, 2, "bf16"), (65, 192, 9, 2, "bf16"), (3583, 64, 16, 2, "bf16"), (3584, 64, 16, 2, "f32"),
+    (895, 128, 64, 6, "bf16"), (1791, 64, 32, 2, "f32"),
+    # an expert per lane: 1, 2 and 4 tokens a wave, and the fused kernel past it
+    (896, 128, 64, 6, "bf16"), (2049, 192, 60, 4, "bf16"), (2049, 64, 64, 1, "f32"),
+    (6147, 128, 64, 2, "bf16"), (4097, 64, 32, 2, "bf16"), (9001, 64, 32, 2, "bf16"),
+    (16383, 64, 57, 2, "bf16"), (16385, 64, 40, 2, "bf16"),
+    # more than 64 experts
+    (511, 64, 65, 4, "bf16"), (513, 128, 70, 4, "bf16"), (1030, 64, 128, 8, "f32"),
+    (3075, 64, 100, 3, "bf16"), (1025, 64, 512, 8, "bf16"), (127, 64, 300, 8, "bf16"),
+]
+
+
+@pytest.mark.parametrize("N,C,E,k,act", SHAPES)
+@pytest.mark.parametrize("train", [False, True])
+def test_routing_bit_exact(N, C, E, k, act, train):
+    cfg = wl.MoEConfig("paths", N, C, E, k, 8, act, act, "normal")
+    inp = wl.make_inputs(cfg, seed=N + E, bias_std=0.02)
+    # a router of ordinary fp32 weights: products that do round
+    inp.Wr[:] = wl.normal_f32(7, 3, C * E, std=0.05).reshape(C, E)
+    inp.x[min(3, N - 1), :] = 0.0   # equal logits up to the bias
+    layer = MoELayer(C, 8, E, k, act=act)
+    layer.load_parameters(inp.params())
+    x = torch.from_numpy(inp.x).to("cuda").to(layer.dtype)
+    layer.forward(x, train=train)
+    torch.cuda.synchronize()
+    r = {n: t.cpu().numpy() for n, t in layer.routing().items()}
+    ref = O.forward(inp, with_y=False)
+    assert np.array_equal(r["topk_idx"], ref["idx"])
+    assert np.array_equal(r["topk_p"], ref["topp"])
+    assert np.array_equal(r["counts"], ref["counts"])
+    assert np.array_equal(r["perm"], ref["perm"])
