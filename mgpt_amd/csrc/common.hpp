@@ -110,15 +110,22 @@ __device__ __forceinline__ void store_act(bf16_t* p, float v) { *p = f32_to_bf16
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & (kWave - 1)); }
 
-// Inclusive prefix sum over the 64 lanes of a wave.
+// Inclusive prefix sum over the 64 lanes of a wave (every lane active), by
+// DPP adds: within the rows of 16 lanes, then row 0's total into row 1 and row
+// 2's into row 3, then the lower half's into the upper half.  (Lane shuffles
+// are LDS round trips, six in a row; every GEMM block starts with two or three
+// of these scans.)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
 __device__ __forceinline__ int wave_incl_scan(int v) {
-  const int l = lane_id();
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    int t = __shfl_up(v, d, kWave);
-    if (l >= d) v += t;
-  }
-  return v;
+  v = dpp_add<0x111, 0xf>(v);   // row_shr:1
+  v = dpp_add<0x112, 0xf>(v);   // row_shr:2
+  v = dpp_add<0x114, 0xf>(v);   // row_shr:4
+  v = dpp_add<0x118, 0xf>(v);   // row_shr:8
+  v = dpp_add<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+  return dpp_add<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
 }
 
 __device__ __forceinline__ int wave_sum(int v) {

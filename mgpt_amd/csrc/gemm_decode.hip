@@ -4,16 +4,23 @@
 // about 8 rows per expert) make the expert GEMMs a weight stream: every
 // weight byte is used by at most 32 rows, so the bound is HBM bandwidth,
 // not MFMA.  This kernel is built for that bound:
-//  * Work items are (expert m-tile of <= 32 rows, 256 output features); a
-//    persistent block per CU walks them, and a direct-to-LDS ring of three
-//    stages (256 weight rows x 128 fp8 columns + 32 activation rows x 128
-//    bf16 columns, 40 KB) keeps two stages of loads in flight per CU across
-//    item boundaries.  The loads are inline asm the compiler does not track,
-//    with explicit waits (as in gemm_dma.hip).
-//  * 4 waves each own 64 features (a [32 gate | 32 up] pair for gate/up) x
-//    the 32 token rows: two v_mfma_f32_32x32x16_bf16 per 16 columns, the
-//    fp8 weights converted to bf16 in registers (exact: every e4m3 value is
-//    a bf16 value); the per-output-channel scale is applied in the epilogue.
+//  * Work items are (expert m-tile of <= 32 rows, 64 or 128 output features);
+//    two persistent blocks per CU walk them, so that one block's start, epilogue
+//    and waits are covered by the other's stream, each with a direct-to-LDS ring
+//    across item boundaries (a stage: 64 or 128 weight rows x 128 fp8 columns
+//    and 32 activation rows x 128 columns).  The loads are inline asm the
+//    compiler does not track, with explicit waits (as in gemm_dma.hip); a lane's
+//    addresses are formed once an item and stepped by additions.
+//  * Each wave owns 64 features (a [32 gate | 32 up] pair for gate/up) x the 32
+//    token rows: two v_mfma_f32_32x32x16_bf16 per 16 columns, the fp8 weights
+//    converted to bf16 in registers (exact: every e4m3 value is a bf16 value);
+//    the per-output-channel scale is applied in the epilogue.  A stage's LDS
+//    reads are all issued before its first MFMA.  Few tokens are bound by this
+//    chain (launch, routing, then a stage's reads, conversions and barrier), not
+//    by HBM; address arithmetic and reads waited for one by one had made a stage
+//    0.85 us where the weights take 0.4 (E = 64, C = 2048, H = 1408, 1 token:
+//    gate/up 22.2 -> 16.6 us, down 15.1 -> 10.8; 64 tokens, HBM-bound at 5.5
+//    TB/s: 69.8 -> 66.8, 37.4 -> 36.0).
 //  * K order within a stage: lane half h holds k = 64h + 8*ks + e for k-step
 //    ks (element e) in both operands, so a lane's weights for the stage are
 //    64 contiguous bytes of its row (four 16-byte LDS reads).
@@ -21,21 +28,18 @@
 // activations [rows][K], B = fp8 weights in stage tiles
 // [E][Npad/256][K/128][256][128] (pack.hip: tile_fp8_kernel) with scales
 // [E][Npad], SwiGLU or bias epilogue).
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace mgpt {
 namespace {
 
-constexpr int kDThreads = 256;
 constexpr int kDBM = 32;                     // token rows per item
-constexpr int kDBN = 256;                    // features per item
 constexpr int kDBK = 128;                    // columns per stage
-#ifndef MGPT_DECODE_STAGES
-#define MGPT_DECODE_STAGES 3
-#endif
-constexpr int kDStages = MGPT_DECODE_STAGES;   // ring depth (LDS: 40 KB a stage, 48 KB for fp32 rows)
-constexpr int kWBytes = kDBN * kDBK;         // 32 KB of fp8 weights
-constexpr int kDmaW = kWBytes / 1024 / 4;    // 8 weight blocks per wave
+constexpr int kTileN = 256;                  // features per tile of the weights' layout
+constexpr int kBlocksPerCu = 2;
+constexpr int kDmaW = 64 * kDBK / 1024;      // 8 weight blocks per wave (64 features) and stage
 
 typedef __attribute__((address_space(3))) char lds_char;
 
@@ -109,20 +113,20 @@ struct DScan {
     rows_incl = wave_incl_scan(cnt);
     tiles_incl = wave_incl_scan(tiles);
     tiles_excl = tiles_incl - tiles;
-    tm = __builtin_amdgcn_readfirstlane(__shfl(tiles_incl, kWave - 1, kWave));
+    tm = __builtin_amdgcn_readlane(tiles_incl, kWave - 1);
   }
-  __device__ __forceinline__ bool locate(int E, int nbx, int v, DItem* out) const {
+  __device__ __forceinline__ bool locate(int E, int nbx, int bn, int v, DItem* out) const {
     if (v >= tm * nbx) return false;
     const int mt = v / nbx;
     const int l = lane_id();
     const bool mine = (l < E) && (mt >= tiles_excl) && (mt < tiles_incl);
     const unsigned long long m = __ballot(mine);
-    const int owner = __ffsll((long long)m) - 1;
-    out->expert = __builtin_amdgcn_readfirstlane(owner);
-    out->row0 = __builtin_amdgcn_readfirstlane(
-        __shfl((rows_incl - cnt) + (mt - tiles_excl) * kDBM, owner, kWave));
-    out->row_end = __builtin_amdgcn_readfirstlane(__shfl(rows_incl, owner, kWave));
-    out->n0 = (v - mt * nbx) * kDBN;
+    const int owner = __builtin_amdgcn_readfirstlane(__ffsll((long long)m) - 1);
+    out->expert = owner;
+    out->row0 = __builtin_amdgcn_readlane(rows_incl - cnt, owner) +
+                (mt - __builtin_amdgcn_readlane(tiles_excl, owner)) * kDBM;
+    out->row_end = __builtin_amdgcn_readlane(rows_incl, owner);
+    out->n0 = (v - mt * nbx) * bn;
     return true;
   }
 };
@@ -200,8 +204,8 @@ __device__ __forceinline__ void decode_rank(const int32_t* __restrict__ topk_idx
 // GATHER (gate/up of at most 512 flat ids, bf16 rows): the activation rows
 // come straight from the caller's x through s_tok instead of from the
 // gathered copy A, and the routing is computed in the block (decode_rank).
-template <int EPI, bool GATHER, typename XT>
-__global__ __launch_bounds__(kDThreads) void gemm_decode_kernel(
+template <int EPI, bool GATHER, typename XT, int NW>
+__global__ __launch_bounds__(NW * 64) void gemm_decode_kernel(
     const XT* __restrict__ A, const fp8_t* __restrict__ B, const float* __restrict__ wscale,
     const float* __restrict__ bias0, const float* __restrict__ bias1,
     const int32_t* __restrict__ counts, int E, int K, int Npad, int n_store, int bias_ld,
@@ -212,21 +216,26 @@ __global__ __launch_bounds__(kDThreads) void gemm_decode_kernel(
   // kRowB bytes per stage row, staged as they are and converted to bf16 when
   // the fragments are read.
   constexpr int kXS = (int)sizeof(XT);
+  constexpr int BN = 64 * NW;                  // features per item
+  constexpr int kWBytes = BN * kDBK;
   constexpr int kAB = kDBM * kDBK * kXS;       // activation bytes per stage
   constexpr int kStage = kWBytes + kAB;
-  constexpr int kDA = kAB / 1024 / 4;          // activation blocks per wave
+  constexpr int kDA = kAB / 1024 / NW;         // activation blocks per wave
   constexpr int kDm = kDmaW + kDA;             // loads per wave and stage
   constexpr int kRowB = kDBK * kXS;            // LDS bytes per activation row
   constexpr int kRowsPerBlk = 1024 / kRowB;
   constexpr int kChunks = kRowB / 16;          // 16-byte chunks per row
   static_assert(kXS == 2 || kXS == 4, "bf16 or fp32 rows");
-  static_assert(kDStages * kStage + kGatherFlat * 4 <= 160 * 1024,
-                "the ring does not fit in LDS at this MGPT_DECODE_STAGES");
+  // ring depth: what LDS holds and the wait counter can count (63 loads)
+  constexpr int kLds = (160 * 1024 / kBlocksPerCu - (GATHER ? kGatherFlat * 4 + 1024 : 0)) / kStage;
+  constexpr int kCnt = 63 / kDm + 2;
+  constexpr int kDStages = kLds < kCnt ? kLds : kCnt;
+  static_assert(kDStages >= 2, "ring depth");
   __shared__ __attribute__((aligned(1024))) char smem[kDStages * kStage];
   __shared__ int s_tok[GATHER ? kGatherFlat : 1];
   __shared__ int s_cnt[GATHER ? kMaxExperts : 1], s_base[GATHER ? kMaxExperts : 1],
       s_run[GATHER ? kMaxExperts : 1];
-  const int nbx = Npad / kDBN;
+  const int nbx = (n_store + BN - 1) / BN;
   const int G = gridDim.x;
   const int32_t* cnts = counts;
   if constexpr (GATHER) {
@@ -238,66 +247,77 @@ __global__ __launch_bounds__(kDThreads) void gemm_decode_kernel(
   sc.init(cnts, E);
   int v = blockIdx.x;
   DItem cur;
-  if (!sc.locate(E, nbx, v, &cur)) return;
+  if (!sc.locate(E, nbx, BN, v, &cur)) return;
 
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
   const int lane = lane_id();
   const int lrow = lane & 31, lhalf = lane >> 5;
   const int KT = K / kDBK;
+  const size_t tiles_n = Npad / kTileN;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char*)smem;
 
   // DMA lane mapping.  Weights: 128-byte rows, wave w fills rows 64w ..
   // 64w+63 in 8 blocks of 8 rows; lane l covers row 8i + l/8, slot l%8 =
   // chunk ^ ((row >> 1) & 7).  Activations: kRowB-byte rows (256 for bf16,
-  // 512 for fp32), wave w fills rows 8w .. 8w+7 in kDA blocks of
-  // kRowsPerBlk rows; lane l covers row kRowsPerBlk*i + l/kChunks, slot
+  // 512 for fp32), wave w fills kDA blocks of kRowsPerBlk rows; lane l covers row kRowsPerBlk*i + l/kChunks, slot
   // l%kChunks = chunk ^ (row & (kChunks - 1)).  Activation rows past the
   // item's last token re-read that token (in bounds, never stored).
   // Weights are in the tiled layout [E][Npad/256][K/128][256][128]: a
-  // stage is one contiguous 32 KB block, rows 128 bytes apart.
-  const size_t wrow_g = (size_t)kDBK;       // fp8 bytes between weight rows of a stage
+  // stage's are one contiguous block, rows 128 bytes apart.
   const size_t arow_g = (size_t)K * kXS;    // bytes per activation row
   uint32_t woff[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int r = i * 8 + lane / 8;
-    woff[i] = (uint32_t)(lane / 8) * (uint32_t)wrow_g + (uint32_t)(((lane % 8) ^ ((r >> 1) & 7)) * 16);
+    woff[i] = (uint32_t)(lane / 8) * (uint32_t)kDBK + (uint32_t)(((lane % 8) ^ ((r >> 1) & 7)) * 16);
   }
-  auto dma_stage = [&](const DItem& it, int kt, int stage) __attribute__((always_inline)) {
-    const uint32_t st = lds0 + (uint32_t)(stage * kStage);
-    const char* wg = reinterpret_cast<const char*>(B) +
-                     (((size_t)it.expert * nbx + it.n0 / kDBN) * KT + kt) * (size_t)kWBytes +
-                     (size_t)(64 * w) * wrow_g;
-#pragma unroll
-    for (int i = 0; i < kDmaW; ++i)
-      dma16_stream(wg + (size_t)(8 * i) * wrow_g + woff[i & 1], st + (uint32_t)((w * kDmaW + i) * 1024));
-#pragma unroll
-    for (int i = 0; i < kDA; ++i) {
-      const int r = 8 * w + kRowsPerBlk * i + lane / kChunks;   // activation row in the tile
-      const int tok = min(it.row0 + r, it.row_end - 1);         // a slot
-      const int chunk = (lane % kChunks) ^ (r & (kChunks - 1));
-      const int src_row = GATHER ? s_tok[tok] : tok;
-      const char* ag = reinterpret_cast<const char*>(A) + (size_t)src_row * arow_g +
-                       (size_t)kt * kRowB + chunk * 16;
-      dma16(ag, st + (uint32_t)(kWBytes + (w * kDA + i) * 1024));
-    }
-  };
 
-  // DMA cursor (item dv, stage column block dkt), STAGES-1 stages ahead.
+  // DMA cursor: item dv at stage column block dkt, STAGES-1 stages ahead, with
+  // this lane's addresses of the stage (a row of weights 8i + lane / 8 is 1024 i
+  // bytes on; the addresses are formed once an item and stepped per stage: a
+  // stage's arithmetic is 64-bit adds only).
   DItem dit = cur;
   int dv = v, dkt = 0, dstage = 0;
   bool dvalid = true;
   int ahead = 0;   // stages issued and not yet waited for
+  const char* wp[2];
+  const char* ap[kDA];
+  auto enter_item = [&]() __attribute__((always_inline)) {
+    const char* wg = reinterpret_cast<const char*>(B) +
+                     ((size_t)dit.expert * tiles_n + dit.n0 / kTileN) * KT * (size_t)(kTileN * kDBK) +
+                     (size_t)(dit.n0 % kTileN + 64 * w) * kDBK;
+    wp[0] = wg + woff[0];
+    wp[1] = wg + woff[1];
+#pragma unroll
+    for (int i = 0; i < kDA; ++i) {
+      const int r = (w * kDA + i) * kRowsPerBlk + lane / kChunks;   // activation row in the tile
+      const int tok = min(dit.row0 + r, dit.row_end - 1);           // a slot
+      const int src_row = GATHER ? s_tok[tok] : tok;
+      ap[i] = reinterpret_cast<const char*>(A) + (size_t)src_row * arow_g +
+              (((lane % kChunks) ^ (r & (kChunks - 1))) << 4);
+    }
+  };
+  enter_item();
   auto advance = [&]() __attribute__((always_inline)) {
     if (dvalid) {
-      dma_stage(dit, dkt, dstage);
+      const uint32_t st = lds0 + (uint32_t)(dstage * kStage);
+#pragma unroll
+      for (int i = 0; i < kDmaW; ++i)
+        dma16_stream(wp[i & 1] + 1024 * i, st + (uint32_t)((w * kDmaW + i) * 1024));
+#pragma unroll
+      for (int i = 0; i < kDA; ++i) dma16(ap[i], st + (uint32_t)(kWBytes + (w * kDA + i) * 1024));
+      wp[0] += kTileN * kDBK;
+      wp[1] += kTileN * kDBK;
+#pragma unroll
+      for (int i = 0; i < kDA; ++i) ap[i] += kRowB;
       ++ahead;
     }
     dstage = dstage + 1 == kDStages ? 0 : dstage + 1;
     if (++dkt == KT) {
       dkt = 0;
       dv += G;
-      if (dvalid) dvalid = sc.locate(E, nbx, dv, &dit);
+      if (dvalid) dvalid = sc.locate(E, nbx, BN, dv, &dit);
+      if (dvalid) enter_item();
     }
   };
   // Barrier before consuming stage c: it landed, with the stages issued
@@ -319,20 +339,30 @@ __global__ __launch_bounds__(kDThreads) void gemm_decode_kernel(
     const int chunk = 4 * lhalf + q;
     return *reinterpret_cast<const uint4*>(st + row * kDBK + ((chunk ^ wswz) << 4));
   };
-  auto afrag = [&](const char* st, int ks) -> bf16x8 {
+  struct ARaw {
+    uint4 v[kXS / 2];
+  };
+  auto aread = [&](const char* st, int ks) -> ARaw {
     const int c = 8 * lhalf + ks;   // columns 8c .. 8c+7 of the stage
     const char* row = st + kWBytes + lrow * kRowB;
+    ARaw r;
     if constexpr (kXS == 2) {
-      return *reinterpret_cast<const bf16x8*>(row + ((c ^ (lrow & 15)) << 4));
+      r.v[0] = *reinterpret_cast<const uint4*>(row + ((c ^ (lrow & 15)) << 4));
+    } else {
+      r.v[0] = *reinterpret_cast<const uint4*>(row + (((2 * c) ^ (lrow & 31)) << 4));
+      r.v[kXS / 2 - 1] = *reinterpret_cast<const uint4*>(row + (((2 * c + 1) ^ (lrow & 31)) << 4));
+    }
+    return r;
+  };
+  auto abf16 = [&](const ARaw& r) -> bf16x8 {
+    if constexpr (kXS == 2) {
+      return __builtin_bit_cast(bf16x8, r.v[0]);
     } else {
       // two 16-byte chunks of fp32 rounded to bf16 by v_cvt_pk_bf16_f32
       // (nearest even, fp32 denormals kept: the rounding f32_to_bf16 does in
       // software for the permute's gather, at 4 instructions a fragment)
       typedef float f32x8 __attribute__((ext_vector_type(8)));
-      const float4 a = *reinterpret_cast<const float4*>(row + (((2 * c) ^ (lrow & 31)) << 4));
-      const float4 b = *reinterpret_cast<const float4*>(row + (((2 * c + 1) ^ (lrow & 31)) << 4));
-      const f32x8 v = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-      return __builtin_convertvector(v, bf16x8);
+      return __builtin_convertvector(__builtin_bit_cast(f32x8, r), bf16x8);
     }
   };
 
@@ -343,7 +373,7 @@ __global__ __launch_bounds__(kDThreads) void gemm_decode_kernel(
 
   for (;;) {
     DItem nxt;
-    const bool have_next = sc.locate(E, nbx, v + G, &nxt);
+    const bool have_next = sc.locate(E, nbx, BN, v + G, &nxt);
     f32x16 acc[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -351,19 +381,27 @@ __global__ __launch_bounds__(kDThreads) void gemm_decode_kernel(
       for (int e = 0; e < 16; ++e) acc[j][e] = 0.0f;
     for (int kt = 0; kt < KT; ++kt) {
       const char* st = smem + cstage * kStage;
-      // 8 k-steps: weights as 4 chunks of 16 fp8 per row (2 k-steps each)
+      // every LDS read of the stage first (one wave a SIMD: nothing else hides
+      // their latency), then 8 k-steps: weights as 4 chunks of 16 fp8 per row
+      // (2 k-steps each)
+      uint4 wv[2][4];
+      ARaw av[8];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const uint4 w0 = wfrag(st, 0, q), w1 = wfrag(st, 1, q);
+        wv[0][q] = wfrag(st, 0, q);
+        wv[1][q] = wfrag(st, 1, q);
+        av[2 * q] = aread(st, 2 * q);
+        av[2 * q + 1] = aread(st, 2 * q + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int ks = 2 * q + h;
-          const bf16x8 b = afrag(st, ks);
-          const bf16x8 a0 = h ? fp8x8_to_bf16x8(w0.z, w0.w) : fp8x8_to_bf16x8(w0.x, w0.y);
-          const bf16x8 a1 = h ? fp8x8_to_bf16x8(w1.z, w1.w) : fp8x8_to_bf16x8(w1.x, w1.y);
-          acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b, acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b, acc[1], 0, 0, 0);
-        }
+      for (int ks = 0; ks < 8; ++ks) {
+        const uint4 w0 = wv[0][ks / 2], w1 = wv[1][ks / 2];
+        const bf16x8 b = abf16(av[ks]);
+        const bf16x8 a0 = (ks & 1) ? fp8x8_to_bf16x8(w0.z, w0.w) : fp8x8_to_bf16x8(w0.x, w0.y);
+        const bf16x8 a1 = (ks & 1) ? fp8x8_to_bf16x8(w1.z, w1.w) : fp8x8_to_bf16x8(w1.x, w1.y);
+        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b, acc[1], 0, 0, 0);
       }
       cstage = cstage + 1 == kDStages ? 0 : cstage + 1;
       // next stage (after the block's last one this waits for nothing new)
@@ -426,16 +464,16 @@ __global__ __launch_bounds__(kDThreads) void gemm_decode_kernel(
   }
 }
 
-// Persistent launch, one block per CU.  Requires K % 128 == 0, Npad % 256 ==
-// 0 and n_store % 64 == 0; max_mtiles bounds sum_e ceil(count_e / 32).
+// Persistent launch, two blocks per CU.  Requires K % 128 == 0, Npad % 256 ==
+// 0 and n_store % 64 == 0; rows: all rows of the E segments.
 template <int EPI, bool GATHER, typename XT>
 hipError_t launch_decode(const XT* A, const fp8_t* B, const float* wscale, const float* bias0,
                          const float* bias1, const int32_t* counts, int E, int K, int Npad,
-                         int n_store, int bias_ld, bf16_t* out, int ldo, int max_mtiles,
-                         const int32_t* topk_idx, int nflat, int k, int32_t* counts_out,
-                         int32_t* perm, int32_t* slot_of, hipStream_t stream) {
-  if (max_mtiles <= 0) return hipSuccess;
-  if (K % kDBK != 0 || Npad % kDBN != 0 || n_store % 64 != 0) return hipErrorInvalidValue;
+                         int n_store, int bias_ld, bf16_t* out, int ldo, int rows,
+                         const int32_t* topk_idx, int k, int32_t* counts_out, int32_t* perm,
+                         int32_t* slot_of, hipStream_t stream) {
+  if (rows <= 0) return hipSuccess;
+  if (K % kDBK != 0 || Npad % kTileN != 0 || n_store % 64 != 0) return hipErrorInvalidValue;
   static int num_cus = 0;
   if (num_cus == 0) {
     int dev = 0;
@@ -443,15 +481,25 @@ hipError_t launch_decode(const XT* A, const fp8_t* B, const float* wscale, const
     if (e == hipSuccess) e = hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e != hipSuccess || num_cus <= 0) num_cus = 256;
   }
-#ifndef MGPT_DECODE_BLOCKS_PER_CU
-#define MGPT_DECODE_BLOCKS_PER_CU 1
-#endif
-  const int items = max_mtiles * (Npad / kDBN);
-  const int slots = MGPT_DECODE_BLOCKS_PER_CU * num_cus;
-  const int grid = items < slots ? items : slots;
-  hipLaunchKernelGGL((gemm_decode_kernel<EPI, GATHER, XT>), dim3(grid), dim3(kDThreads), 0, stream, A,
-                     B, wscale, bias0, bias1, counts, E, K, Npad, n_store, bias_ld, out, ldo,
-                     topk_idx, nflat, k, counts_out, perm, slot_of);
+  // An item of 64 features (one wave) where those give no CU more than one,
+  // else of 128 (two waves); E or fewer tiles of rows is the estimate while they
+  // average 16 rows.  us on MI355X for 256 features and one block a CU / 128 /
+  // 64: down, E = 64, C = 2048, H = 1408, 1 token 15.2 / 12.0 / 10.8 (256 items
+  // of 64), 64 tokens 36.9 / 36.0 / 40.1 (2048); E = 16, C = 1024, H = 2816, 37
+  // tokens 23.3 / 19.8 / 16.3 (256); gate/up of the former, 1 token 20.1 / 16.6 /
+  // 17.4 (352), 64 tokens 67.1 / 66.8 / 79.6 (2816).
+  const long est = (long)rows <= 16L * E ? std::min<long>(E, rows) : rows / 32 + E;
+  const bool narrow = est * ((n_store + 63) / 64) <= num_cus;
+  auto launch = [&](auto kernel, int NW) {
+    const long items = (long)(rows / 32 + std::min(E, rows)) * ((n_store + 64 * NW - 1) / (64 * NW));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<long>(items, kBlocksPerCu * num_cus)), dim3(64 * NW),
+                       0, stream, A, B, wscale, bias0, bias1, counts, E, K, Npad, n_store, bias_ld, out,
+                       ldo, topk_idx, rows, k, counts_out, perm, slot_of);
+  };
+  if (narrow)
+    launch(gemm_decode_kernel<EPI, GATHER, XT, 1>, 1);
+  else
+    launch(gemm_decode_kernel<EPI, GATHER, XT, 2>, 2);
   return hipGetLastError();
 }
 
@@ -461,10 +509,10 @@ template <int EPI>
 hipError_t launch_gemm_decode(const bf16_t* A, const fp8_t* B, const float* wscale,
                               const float* bias0, const float* bias1, const int32_t* counts, int E,
                               int K, int Npad, int n_store, int bias_ld, bf16_t* out, int ldo,
-                              int max_mtiles, hipStream_t stream) {
+                              int rows, hipStream_t stream) {
   return launch_decode<EPI, false, bf16_t>(A, B, wscale, bias0, bias1, counts, E, K, Npad, n_store,
-                                   bias_ld, out, ldo, max_mtiles, nullptr, 0, 0, nullptr, nullptr,
-                                   nullptr, stream);
+                                   bias_ld, out, ldo, rows, nullptr, 0, nullptr, nullptr, nullptr,
+                                   stream);
 }
 
 template hipError_t launch_gemm_decode<kEpiGateUp>(const bf16_t*, const fp8_t*, const float*,
@@ -485,23 +533,22 @@ template <typename XT>
 hipError_t launch_gemm_decode_gather(const XT* x, const fp8_t* B, const float* wscale,
                                      const float* bias0, const float* bias1, const int32_t* topk_idx,
                                      int nflat, int k, int E, int K, int Npad, int n_store,
-                                     int bias_ld, bf16_t* out, int ldo, int max_mtiles,
-                                     int32_t* counts, int32_t* perm, int32_t* slot_of,
+                                     int bias_ld, bf16_t* out, int ldo, int32_t* counts, int32_t* perm, int32_t* slot_of,
                                      hipStream_t stream) {
   if (nflat > kGatherFlat || E > kMaxExperts || k < 1) return hipErrorInvalidValue;
   return launch_decode<kEpiGateUp, true, XT>(x, B, wscale, bias0, bias1, nullptr, E, K, Npad, n_store,
-                                         bias_ld, out, ldo, max_mtiles, topk_idx, nflat, k, counts,
-                                         perm, slot_of, stream);
+                                         bias_ld, out, ldo, nflat, topk_idx, k, counts, perm,
+                                         slot_of, stream);
 }
 template hipError_t launch_gemm_decode_gather<bf16_t>(const bf16_t*, const fp8_t*, const float*,
                                                        const float*, const float*, const int32_t*,
                                                        int, int, int, int, int, int, int, bf16_t*,
-                                                       int, int, int32_t*, int32_t*, int32_t*,
+                                                       int, int32_t*, int32_t*, int32_t*,
                                                        hipStream_t);
 template hipError_t launch_gemm_decode_gather<float>(const float*, const fp8_t*, const float*,
                                                       const float*, const float*, const int32_t*,
                                                       int, int, int, int, int, int, int, bf16_t*,
-                                                      int, int, int32_t*, int32_t*, int32_t*,
+                                                      int, int32_t*, int32_t*, int32_t*,
                                                       hipStream_t);
 
 }  // namespace mgpt

@@ -76,8 +76,7 @@ hipError_t launch_pad_row(const float*, int, float*, int, hipStream_t);
 template <typename XT>
 hipError_t launch_gemm_decode_gather(const XT*, const fp8_t*, const float*, const float*,
                                      const float*, const int32_t*, int, int, int, int, int, int,
-                                     int, bf16_t*, int, int, int32_t*, int32_t*, int32_t*,
-                                     hipStream_t);
+                                     int, bf16_t*, int, int32_t*, int32_t*, int32_t*, hipStream_t);
 hipError_t launch_pack_router(const float*, const float*, int, int, int, int, float*, float*, float*,
                               float*, float*, hipStream_t);
 template <int EPI>
@@ -311,14 +310,14 @@ struct mgpt_moe {
   }
   // fp8 weights on the decode kernel's tiled copies, up to 64 rows per expert on
   // average.  Its 32-row tiles read the weights once per 32 rows of an expert,
-  // so past 40 rows the 256-row tiles of gemm_stream.hip are faster where the
+  // so past 48 rows the 256-row tiles of gemm_stream.hip are faster where the
   // gate/up product has enough of them, two a CU (us for both expert products
   // on MI355X, E = 64, C = 2048, H = 1408: 33 rows per expert 175 against 185,
   // 45 rows 201 against 191, 60 rows 234 against 195; E = 16, C = 1024, H =
   // 2816, 1.4 tiles a CU: 60 rows 80 against 82; a layer of E = 16, C = 512, H =
   // 1376, 0.7 a CU: 56 rows 61 against 68).
   bool fp8_decode(int N) const {
-    const size_t rows = (size_t)E * ((2 * Hp + 255) / 256) >= (size_t)2 * num_cus ? 40 : 64;
+    const size_t rows = (size_t)E * ((2 * Hp + 255) / 256) >= (size_t)2 * num_cus ? 48 : 64;
     return wgu_t && !wide() && (size_t)N * k < rows * E;
   }
   size_t w_bytes() const { return wdt == MGPT_DTYPE_FP8_E4M3 ? 1 : (wdt == MGPT_DTYPE_BF16 ? 2 : 4); }
@@ -897,17 +896,16 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
     if (h->fp8_decode(N)) {
       // weight streaming: the persistent direct-to-LDS decode kernel on the
       // tiled copies
-      const int mt = (int)((A + 31) / 32) + E;
       if (gather_decode)
         HIP_TRY(launch_gemm_decode_gather<IoT>(xi, (const fp8_t*)h->wgu_t, h->sgu, h->bg, h->bu, idx,
-                                               (int)A, k, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, mt, counts,
+                                               (int)A, k, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, counts,
                                                perm, slot_of, st));
       else
         HIP_TRY(launch_gemm_decode<kEpiGateUp>(xg, (const fp8_t*)h->wgu_t, h->sgu, h->bg, h->bu,
-                                               counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, mt, st));
+                                               counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, (int)A, st));
       HIP_TRY(mark(3));
       HIP_TRY(launch_gemm_decode<kEpiDown>(hb, (const fp8_t*)h->wd_t, h->sd, h->bd, nullptr, counts,
-                                           E, Hp, Cp, C, Cp, ob, C, mt, st));
+                                           E, Hp, Cp, C, Cp, ob, C, (int)A, st));
     } else if (fp8) {
       // 256 x 256 tiles, except where the decode kernel's shape rules do not
       // hold (width, more than 64 experts) and rows are few
