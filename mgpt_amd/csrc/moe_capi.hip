@@ -310,14 +310,14 @@ struct mgpt_moe {
   }
   // fp8 weights on the decode kernel's tiled copies, up to 64 rows per expert on
   // average.  Its 32-row tiles read the weights once per 32 rows of an expert,
-  // so past 48 rows the 256-row tiles of gemm_stream.hip are faster where the
+  // so past 40 rows the 256-row tiles of gemm_stream.hip are faster where the
   // gate/up product has enough of them, two a CU (us for both expert products
   // on MI355X, E = 64, C = 2048, H = 1408: 33 rows per expert 175 against 185,
   // 45 rows 201 against 191, 60 rows 234 against 195; E = 16, C = 1024, H =
   // 2816, 1.4 tiles a CU: 60 rows 80 against 82; a layer of E = 16, C = 512, H =
   // 1376, 0.7 a CU: 56 rows 61 against 68).
   bool fp8_decode(int N) const {
-    const size_t rows = (size_t)E * ((2 * Hp + 255) / 256) >= (size_t)2 * num_cus ? 48 : 64;
+    const size_t rows = (size_t)E * ((2 * Hp + 255) / 256) >= (size_t)2 * num_cus ? 40 : 64;
     return wgu_t && !wide() && (size_t)N * k < rows * E;
   }
   size_t w_bytes() const { return wdt == MGPT_DTYPE_FP8_E4M3 ? 1 : (wdt == MGPT_DTYPE_BF16 ? 2 : 4); }
