@@ -279,9 +279,9 @@ int mgpt_moe_expert_counts(mgpt_moe* h, int32_t* host_counts, int num_experts);
  * [4] combine; if n > 5, ms[5] receives the number of forwards averaged.
  * (Inference steps with fp8 weights, no gamma, bf16 or fp32 rows, an
  * embed_dim padded to a multiple of 128 (its tiled weight copy exists only
- * then) and at most 512 flat ids N*k, below 64*E (40*E for
- * layers of many wide experts), route inside the gate/up GEMM: [1] is then
- * only the gap between two events and [2] includes the routing.  Other decode steps run the permute and split their stages as
+ * then) and at most 512 flat ids N*k, below 64*E, route inside the gate/up
+ * GEMM: [1] is then only the gap between two events and [2] includes the
+ * routing.  Other decode steps run the permute and split their stages as
  * usual.)
  * enable: 0 off, 1 every stage boundary, 2 only the two boundaries of the
  * gate/up GEMM (the other launches keep their spacing; stage_times then

@@ -308,18 +308,16 @@ struct mgpt_moe {
     return act == MGPT_DTYPE_BF16 && wdt == MGPT_DTYPE_BF16 && gemm_tile == 256 &&
            (size_t)N * k >= (size_t)64 * E;
   }
-  // fp8 weights on the decode kernel's tiled copies, up to 64 rows per expert on
-  // average.  Its 32-row tiles read the weights once per 32 rows of an expert,
-  // so past 40 rows the 256-row tiles of gemm_stream.hip are faster where the
-  // gate/up product has enough of them, two a CU (us for both expert products
-  // on MI355X, E = 64, C = 2048, H = 1408: 33 rows per expert 175 against 185,
-  // 45 rows 201 against 191, 60 rows 234 against 195; E = 16, C = 1024, H =
-  // 2816, 1.4 tiles a CU: 60 rows 80 against 82; a layer of E = 16, C = 512, H =
-  // 1376, 0.7 a CU: 56 rows 61 against 68).
-  bool fp8_decode(int N) const {
-    const size_t rows = (size_t)E * ((2 * Hp + 255) / 256) >= (size_t)2 * num_cus ? 40 : 64;
-    return wgu_t && !wide() && (size_t)N * k < rows * E;
-  }
+  // fp8 weights on the decode kernel's tiled copies, below 64 rows per expert on
+  // average.  Its 32-row tiles read the weights once per 32 rows of an expert; the
+  // 256-row tiles of gemm_stream.hip do so once, but leave the chip idle where the
+  // down product has few of them and follow a skewed routing worse.  MI355X, us
+  // of the forward, decode against 256-row tiles (even; skewed routing):
+  // E = 32, C = 1024, H = 4096: 44 rows an expert 156 / 201; 137 / 206, 62 rows
+  // 190 / 206; 177 / 222.  E = 32, C = 1792, H = 2400: 44 rows 189 / 193; 177 /
+  // 200, 62 rows 226 / 200; 222 / 209.  E = 64, C = 2048, H = 1408: 44 rows 239 /
+  // 243; 233 / 253, 62 rows 279 / 254; 282 / 272.
+  bool fp8_decode(int N) const { return wgu_t && !wide() && (size_t)N * k < (size_t)64 * E; }
   size_t w_bytes() const { return wdt == MGPT_DTYPE_FP8_E4M3 ? 1 : (wdt == MGPT_DTYPE_BF16 ? 2 : 4); }
   // h (SwiGLU output) is kept in the activation dtype.
   // stream_part: with the weight-streaming GEMMs' partial tiles (bf16 weights,
