@@ -34,6 +34,10 @@ constexpr int kMaxTopK = 8;
 constexpr int kRouterTokens = 64;
 __host__ __device__ inline int router_tokens_per_block(int /*E*/) { return kRouterTokens; }
 
+// Tokens up to which the permute counts the ids itself (no histogram): each of
+// its blocks reads all of them, at most 2048, in place of a counting launch.
+constexpr int kPermuteCountTokens = 256;
+
 // Widest row the one-launch decode router takes (x[t] is widened into LDS as
 // fp32, 32 KB at this width).
 constexpr int kDecodeRouterMaxC = 8192;

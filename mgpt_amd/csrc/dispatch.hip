@@ -193,16 +193,19 @@ __global__ __launch_bounds__(256) void permute_kernel(
       s_tot[e] = counts[e];
     }
   } else if (!hist) {
-    // a single router block routed without a histogram (nb == 1): count its
-    // ids (LDS integer atomics; counts do not depend on their order)
+    // few tokens, no histogram: count the ids, all and those of the router
+    // blocks before this one (LDS integer atomics; counts do not depend on
+    // their order)
     for (int e = tid; e < E; e += 256) {
       s_pre[e] = 0;
       s_tot[e] = 0;
     }
     __syncthreads();
-    for (int f = tid; f < nflat; f += 256) {
-      const int e = topk_idx[flat0 + f];
-      if (e >= 0 && e < E) atomicAdd(&s_tot[e], 1);
+    for (int f = tid; f < N * k; f += 256) {
+      const int e = topk_idx[f];
+      if (e < 0 || e >= E) continue;
+      atomicAdd(&s_tot[e], 1);
+      if (f < (int)flat0) atomicAdd(&s_pre[e], 1);
     }
   } else {
     // Per expert: the assignments of the router blocks before this one and
@@ -353,7 +356,7 @@ hipError_t launch_permute(const InT* x, const int32_t* topk_idx, const int32_t* 
   const int nb = (N + TB - 1) / TB;
   if (nb == 0) return hipSuccess;
   const bool fold = E * nb <= kFoldScan;
-  if (!hist && nb != 1) return hipErrorInvalidValue;   // counting the ids needs one block
+  if (!hist && N > kPermuteCountTokens) return hipErrorInvalidValue;
   if (E > kMaxExpertsWide) return hipErrorInvalidValue;
   if (!fold)
     hipLaunchKernelGGL(expert_scan_kernel, dim3(E), dim3(256), 0, stream, hist, nb, base, counts);

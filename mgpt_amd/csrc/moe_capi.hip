@@ -288,11 +288,6 @@ struct mgpt_moe {
   bool padded() const { return Cx != C; }
   // more experts than a wave has lanes: the forward's generic paths only
   bool wide() const { return E > kMaxExperts; }
-  // one router block of tokens: logits and softmax in one launch, and the
-  // permute counts the ids itself (no histogram)
-  bool router_one_launch(int N, bool norm) const {
-    return wr4 && router_decode_range(N, C, E, norm);
-  }
   // Where the router may keep its logits [N][E]: a region of their own for few
   // tokens and many experts (E > 16), else the expert outputs' region, which
   // is written only after them, if they fit there.
@@ -859,7 +854,6 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
   float* probs = train ? (float*)(ws + L.probs) : nullptr;
   ActT* gu = train ? (ActT*)(ws + L.gu) : nullptr;
   float* rstd = gamma ? (float*)(ws + L.rstd) : nullptr;
-  const bool one_launch = h->router_one_launch(N, gamma != nullptr);
   HIP_TRY(launch_router<IoT>(xi, h->wr_g, h->wr1, h->wr4, h->br, N, C, E,
                              k, idx, topp, hist, logits,
                              probs, gamma, blk.eps, Cx, rstd, st));
@@ -871,8 +865,8 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
   const bool gather_decode = !train && !gamma && h->fp8_decode(N) &&
                              A <= (size_t)kRouterTokens * kMaxTopK;
   if (!gather_decode)
-    HIP_TRY((launch_permute<IoT, ActT>(xi, idx, one_launch ? nullptr : hist, base, N, C, E, k,
-                                       counts, perm, slot_of, xg, rstd, gamma, st)));
+    HIP_TRY((launch_permute<IoT, ActT>(xi, idx, N <= kPermuteCountTokens ? nullptr : hist, base, N,
+                                       C, E, k, counts, perm, slot_of, xg, rstd, gamma, st)));
   HIP_TRY(mark(2));
   if constexpr (sizeof(ActT) == 4) {
     HIP_TRY(launch_gemm_f32<kEpiGateUp>(xg, (const float*)h->wgu, h->bg, h->bu, counts, E, C, 2 * Hp,

@@ -745,8 +745,7 @@ __global__ __launch_bounds__(1024) void router_softmax_wide_kernel(
 // buffer.  The chain wave then issues one add and a quarter of an LDS read
 // per column instead of a product, an add and two half reads; the rounding
 // sequence (one rounded product, one rounded add per term) is unchanged.
-// Loads run two chunks ahead in registers.  hist[e][block] is cleared for
-// router_softmax_wave_kernel.  Measured at cfg5 (64 tokens, C = 2048, E =
+// Loads run two chunks ahead in registers.  Measured at cfg5 (64 tokens, C = 2048, E =
 // 64): 15 us, against 23 us for four experts' chains per block with each
 // wave forming its own products; the chains alone (products skipped) take
 // 10.8 us, 2048 dependent fp32 adds of about 11 cycles each, which no
@@ -779,7 +778,7 @@ template <> struct PcPiece<float> {
 template <typename ActT>
 __global__ __launch_bounds__(256) void router_logits_pc_kernel(
     const ActT* __restrict__ x, const float* __restrict__ wr1, const float* __restrict__ br,
-    int N, int C, int E, float* __restrict__ logits, int32_t* __restrict__ hist, int nb) {
+    int N, int C, int E, float* __restrict__ logits) {
   __shared__ float4 s_p[2][kRT * kPcLD / 4];
   const int tid = threadIdx.x;
   const int lane = lane_id();
@@ -787,7 +786,6 @@ __global__ __launch_bounds__(256) void router_logits_pc_kernel(
   const int tok0 = blockIdx.x * kRT;
   const int e = blockIdx.y;
   const int last_row = min(kRT, N - tok0) - 1;
-  if (e == 0 && tid < E) hist[(size_t)tid * nb + blockIdx.x] = 0;
   const int nch = (C + kPcCB - 1) / kPcCB;
   auto cols = [&](int ch) { return min(kPcCB, C - ch * kPcCB); };   // a multiple of 64
   if (w == 0) {
@@ -897,12 +895,11 @@ __global__ __launch_bounds__(256) void router_logits_pc_kernel(
 // bound with several waves a SIMD, the latency of the scalar loads with one
 // (about 1000 cycles a batch; weights three batches ahead measured the same).
 // So T grows with the work.  The rounding sequence is the other kernels' (c ascending, one rounded
-// product and one rounded add per term, the bias last).  hist[e][block] is
-// cleared for router_softmax_wave_kernel.
+// product and one rounded add per term, the bias last).
 template <typename ActT, int T>
 __global__ __launch_bounds__(256) void router_logits_lane_kernel(
     const ActT* __restrict__ x, const float4* __restrict__ wr4, const float* __restrict__ br, int N,
-    int C, int E, float* __restrict__ logits, int32_t* __restrict__ hist, int nb) {
+    int C, int E, float* __restrict__ logits) {
   constexpr int kPerDw = 4 / (int)sizeof(ActT);        // columns per dword of x
   constexpr int CB = 32 * kPerDw / T < 32 ? 32 * kPerDw / T : 32;   // 32 dwords of x a batch
   constexpr int kDw = CB / kPerDw;
@@ -910,7 +907,6 @@ __global__ __launch_bounds__(256) void router_logits_lane_kernel(
   const int tok0 = (blockIdx.x * 4 + w) * T;
   const int e = blockIdx.y * kWave + lane, ee = min(e, E - 1);
   if (tok0 >= N) return;
-  if (hist && tok0 % kRT == 0 && e < E) hist[(size_t)e * nb + tok0 / kRT] = 0;
   const uint32_t* xr[T];
 #pragma unroll
   for (int i = 0; i < T; ++i)
@@ -975,7 +971,7 @@ __global__ __launch_bounds__(256) void router_logits_lane_kernel(
     if (tok0 + i < N) logits[(size_t)(tok0 + i) * E + e] = acc[i] + b;
 }
 
-// Softmax, top-k and histogram for decode shapes: one wave per token, lane e
+// Softmax and top-k for decode shapes: one wave per token, lane e
 // holding expert e (E <= 64), the row in LDS.  Every lane computes the
 // row's reductions itself, in the reference's order: the running max from
 // element 0 with a strict '>' (NaN-aware as the reference is), then after the
@@ -983,17 +979,12 @@ __global__ __launch_bounds__(256) void router_logits_lane_kernel(
 // clamped probabilities under (p descending, id ascending) -- the order the
 // reference's insertion top-k with a strict '>' produces -- is the number of
 // experts before it; ranks below k are the choices, written at their rank,
-// and counted into hist[e][token / 64] with integer atomics
-// (router_logits_pc_kernel cleared those entries).  No shuffles or merge
-// rounds: four passes over the row in LDS, latency hidden across lanes.
-// The softmax / top-k of one token on one wave (lane e = expert e, l its
-// logit), with the row in LDS (row[e] = l for every lane already stored and
-// visible to the wave).  hist == nullptr: no histogram (the caller's
-// permute counts the ids itself).
+// for router_count_kernel (one router block: the permute) to count.  No
+// shuffles or merge rounds: four passes over the row in LDS, latency hidden
+// across lanes.
 // The softmax / top-k of one token on one wave (lane e = expert e, l its
 // logit), with the row in LDS: row[e] = l for e < E and -inf for the lanes
-// past E, stored by every lane and visible to the wave.  hist == nullptr: no
-// histogram (the caller's permute counts the ids itself).
+// past E, stored by every lane and visible to the wave.
 //
 // Every pass reads the whole row (kMaxExperts floats, 16-byte aligned) as
 // quads, all reads before the arithmetic, and runs over all kMaxExperts
@@ -1005,7 +996,6 @@ __device__ __forceinline__ void softmax_topk_wave(float l, bool valid, int t, in
                                                   int k, float* row, const uint64_t* tab,
                                                   int32_t* __restrict__ topk_idx,
                                                   float* __restrict__ topk_p,
-                                                  int32_t* __restrict__ hist, int nb,
                                                   float* __restrict__ probs) {
   constexpr int kQ = kMaxExperts / 4;
   const float4* row4 = reinterpret_cast<const float4*>(row);
@@ -1050,14 +1040,13 @@ __device__ __forceinline__ void softmax_topk_wave(float l, bool valid, int t, in
   if (rank < k) {
     topk_idx[(size_t)t * k + rank] = e;
     topk_p[(size_t)t * k + rank] = p;
-    if (hist) atomicAdd(&hist[(size_t)e * nb + t / kRT], 1);
   }
 }
 
 constexpr int kSoftmaxWaves = 4;   // tokens per block
 __global__ __launch_bounds__(kSoftmaxWaves * 64) void router_softmax_wave_kernel(
     const float* __restrict__ logits, int N, int E, int k, int32_t* __restrict__ topk_idx,
-    float* __restrict__ topk_p, int32_t* __restrict__ hist, int nb, float* __restrict__ probs) {
+    float* __restrict__ topk_p, float* __restrict__ probs) {
   __shared__ __align__(16) float s_row[kSoftmaxWaves][kMaxExperts];
   __shared__ uint64_t s_tab[32];
   const int w = threadIdx.x / kWave, e = lane_id();
@@ -1068,7 +1057,28 @@ __global__ __launch_bounds__(kSoftmaxWaves * 64) void router_softmax_wave_kernel
   const float l = (valid && e < E) ? logits[(size_t)t * E + e] : 0.0f;
   row[e] = e < E ? l : -INFINITY;
   __syncthreads();
-  softmax_topk_wave(l, valid, t, e, E, k, row, s_tab, topk_idx, topk_p, hist, nb, probs);
+  softmax_topk_wave(l, valid, t, e, E, k, row, s_tab, topk_idx, topk_p, probs);
+}
+
+// hist[e][block] of one router block's ids, counted in LDS.  A launch of its
+// own: counted by the softmax kernel's waves with global atomics instead, the
+// ids of a batch meet on a few cache lines (16 router blocks share one of
+// hist's), at 80 ns each.  MI355X, the router stage: E = 60, C = 1024, top-2,
+// 1024 tokens 26 -> 20 us, 2048 37 -> 26, 4096 41 -> 28.
+__global__ __launch_bounds__(256) void router_count_kernel(const int32_t* __restrict__ topk_idx,
+                                                           int N, int E, int k,
+                                                           int32_t* __restrict__ hist, int nb) {
+  __shared__ int s_hist[kMaxExperts];
+  const int tid = threadIdx.x, b = blockIdx.x;
+  if (tid < kMaxExperts) s_hist[tid] = 0;
+  __syncthreads();
+  const int nflat = min(kRT, N - b * kRT) * k;
+  for (int f = tid; f < nflat; f += 256) {
+    const int e = topk_idx[(size_t)b * kRT * k + f];
+    if (e >= 0 && e < E) atomicAdd(&s_hist[e], 1);
+  }
+  __syncthreads();
+  if (tid < E) hist[(size_t)tid * nb + b] = s_hist[tid];
 }
 
 // Decode router for a single block of tokens (N <= 64, E <= 64, no
@@ -1295,7 +1305,7 @@ __global__ __launch_bounds__(256) void router_decode_kernel(
   s_row[e] = mine ? l : -INFINITY;
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  softmax_topk_wave(l, t < N, t, e, E, k, s_row, s_tab, topk_idx, topk_p, nullptr, 1, probs);
+  softmax_topk_wave(l, t < N, t, e, E, k, s_row, s_tab, topk_idx, topk_p, probs);
 }
 
 
@@ -1328,7 +1338,7 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
     const long pairs = (long)N * eg;
     auto go = [&](auto kernel, int T) {
       hipLaunchKernelGGL(kernel, dim3((N + 4 * T - 1) / (4 * T), eg), dim3(256), 0, stream, x,
-                         reinterpret_cast<const float4*>(wr4), br, N, C, E, logits, hist, nb);
+                         reinterpret_cast<const float4*>(wr4), br, N, C, E, logits);
     };
     if (pairs <= 2048)
       go(router_logits_lane_kernel<ActT, 1>, 1);
@@ -1361,7 +1371,7 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
                          rstd);
     else
       hipLaunchKernelGGL((router_logits_pc_kernel<ActT>), dim3(nb, E), dim3(256), 0, stream, x,
-                         wr1, br, N, C, E, logits, hist, nb);
+                         wr1, br, N, C, E, logits);
     if (E <= 256)
       hipLaunchKernelGGL(router_softmax_wide_kernel<256>, dim3(nb), dim3(1024), 0, stream, logits,
                          N, E, k, topk_idx, topk_p, hist, nb, probs);
@@ -1377,28 +1387,43 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
     return hipGetLastError();
   }
   // Without normalisation the logits go through memory, with more blocks than
-  // the fused kernel's one per 64 tokens, while those do not fill the chip.
-  // Measured on MI355X (us of the router stage, separate product and chain
-  // waves / an expert per lane / fused):
-  //   E = 16, C = 1024: 512 tokens 16 / - / 27, 2048 19 / 28 / 27, 4096 28 / 33 / 28
-  //   E = 32, C = 1024: 1024 tokens 19 / 23 / 45, 2048 28 / 28 / 45, 4096 47 / 34 / 46,
-  //                     8192 - / 50 / 48
-  //   E = 64, C = 2048: 512 tokens 25 / 36 / 128, 1024 41 / 37 / 128, 2048 73 / 49 / 130,
-  //                     4096 134 / 62 / 132, 8192 - / 89 / 137, 32768 - / 257 / 287
-  //   E = 8, C = 512: 512 tokens 15 / - / 12
-  // An expert per lane costs 16 us and 4 us per 1000 tokens and 64 experts (C =
-  // 1024), the fused kernel 1.25 us per expert and round of 256 blocks.
+  // the fused kernel's one per 64 tokens, where that is faster.  MI355X, us of
+  // router and permute, top-2, fused (E > 16 below 4096 tokens: split) / here:
+  //   E = 12: C = 128 15 / 15 everywhere; C = 256 256 tokens 17.4 / 15.1, 2048 18.3
+  //     / 18.1; C = 1024 512 tokens 34 / 21, 2048 37 / 26, 4096 37 / 34
+  //   E = 32: C = 256 1024 tokens 30 / 20, 3072 40 / 24, 4096 28 / 25, 8192 30 / 30;
+  //     C = 1024 1024 tokens 36 / 27, 3072 53 / 37, 4096 55 / 38, 8192 60 / 59
+  //   E = 64: C = 256 1024 tokens 33 / 18, 4096 34 / 27; C = 2048 512 tokens 33 /
+  //     32, 2048 87 / 54, 4096 137 / 58, 8192 151 / 99
+  // An expert per lane is priced at 10 us and (0.9 + 0.0036 C) us per 1000 tokens,
+  // the fused kernel at 10 us and (0.011 + 0.00073 E) C us per round of 256
+  // blocks.  Up to 16 experts, product and chain waves win while the fused
+  // kernel's chains are long against the tokens (E N below 64 C: the limit is
+  // 1024 tokens at E = 16, C = 256 and about 3500 from C = 1024 on).
   const bool many = (long)N * E >= 57344;
-  const bool lane = many && wr4 && 4L * N + 16000 < 1250L * E * ((N + 16383) / 16384);
-  if (logits && !gamma && E > 8 && (lane || (E > 16 ? N < 4096 : !many))) {
+  const float lane_us = 10.0f + N * (0.9e-3f + 3.6e-6f * C);
+  const float fused_us = (10.0f + C * (0.011f + 0.73e-3f * E)) * ((nb + 255) / 256);
+  const bool lane = wr4 && many && E > 16 && (N < 4096 || lane_us < fused_us);
+  const bool pc = E > 16 ? N < 4096 : E > 8 && C >= 256 && (long)N * E < std::min(57344L, 64L * C);
+  if (logits && !gamma && (lane || pc)) {
     if (lane)
       lane_logits();
     else
       hipLaunchKernelGGL((router_logits_pc_kernel<ActT>), dim3(nb, E), dim3(256), 0, stream, x, wr1,
-                         br, N, C, E, logits, hist, nb);
+                         br, N, C, E, logits);
+    // up to 16 experts, four tokens share a wave and the block counts its ids: 2
+    // us less than a wave per token and the counting launch; from 17 on 1 us more
+    if (E <= 16) {
+      hipLaunchKernelGGL(router_softmax_kernel, dim3(nb), dim3(MGPT_SOFTMAX_THREADS), 0, stream,
+                         logits, N, E, k, topk_idx, topk_p, hist, nb, probs);
+      return hipGetLastError();
+    }
     hipLaunchKernelGGL(router_softmax_wave_kernel, dim3((N + kSoftmaxWaves - 1) / kSoftmaxWaves),
                        dim3(kSoftmaxWaves * kWave), 0, stream, logits, N, E, k, topk_idx, topk_p,
-                       hist, nb, probs);
+                       probs);
+    if (N > kPermuteCountTokens)
+      hipLaunchKernelGGL(router_count_kernel, dim3(nb), dim3(256), 0, stream, topk_idx, N, E, k,
+                         hist, nb);
     return hipGetLastError();
   }
   if (logits && gamma && E > 16 && N < 4096) {

@@ -26,6 +26,10 @@ SHAPES = [
     (896, 128, 64, 6, "bf16"), (2049, 192, 60, 4, "bf16"), (2049, 64, 64, 1, "f32"),
     (6147, 128, 64, 2, "bf16"), (4097, 64, 32, 2, "bf16"), (9001, 64, 32, 2, "bf16"),
     (16383, 64, 57, 2, "bf16"), (16385, 64, 40, 2, "bf16"),
+    # ids counted by the permute (up to 256 tokens) and by a launch of its own
+    (190, 64, 33, 8, "bf16"), (256, 256, 16, 2, "bf16"), (256, 64, 512, 8, "f32"), (257, 64, 17, 8, "bf16"),
+    # the width's part in the rule up to 16 experts
+    (1023, 256, 16, 2, "bf16"), (1025, 256, 16, 2, "f32"), (1819, 320, 10, 3, "bf16"), (900, 192, 9, 2, "bf16"),
     # more than 64 experts
     (511, 64, 65, 4, "bf16"), (513, 128, 70, 4, "bf16"), (1030, 64, 128, 8, "f32"),
     (3075, 64, 100, 3, "bf16"), (1025, 64, 512, 8, "bf16"), (127, 64, 300, 8, "bf16"),
