@@ -43,11 +43,11 @@ constexpr int kPermuteCountTokens = 256;
 constexpr int kDecodeRouterMaxC = 8192;
 
 // The calls that the one-launch decode router takes: one router block of
-// tokens, a wave of experts, plain rows (us of the router stage on MI355X with
+// tokens, a wave of experts (us of the router stage on MI355X with
 // the fused kernel and with this one, 24 tokens: E = 8, C = 512 11.2 -> 8.5; E =
 // 16, C = 1024 25.6 -> 11.0; E = 16, C = 2048 46 -> 16).
-__host__ __device__ inline bool router_decode_range(int N, int C, int E, bool norm) {
-  return N <= kRouterTokens && E <= kMaxExperts && !norm && C % 64 == 0 && C <= kDecodeRouterMaxC;
+__host__ __device__ inline bool router_decode_range(int N, int C, int E) {
+  return N <= kRouterTokens && E <= kMaxExperts && C % 64 == 0 && C <= kDecodeRouterMaxC;
 }
 
 // Router experts per wave (the router block has ceil(E / RE) <= 16 waves);

@@ -39,7 +39,7 @@ namespace mgpt {
 template <typename ActT>
 hipError_t launch_router(const ActT*, const float*, const float*, const float*, const float*, int,
                          int, int, int, int32_t*, float*, int32_t*, float*, float*, const float*,
-                         float, int, float*, hipStream_t);
+                         float, int, float*, float*, hipStream_t);
 hipError_t launch_expf_probe(const float*, float*, int, hipStream_t);
 template <typename InT, typename ActT>
 hipError_t launch_permute(const InT*, const int32_t*, const int32_t*, int32_t*, int, int, int,
@@ -854,9 +854,11 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
   float* probs = train ? (float*)(ws + L.probs) : nullptr;
   ActT* gu = train ? (ActT*)(ws + L.gu) : nullptr;
   float* rstd = gamma ? (float*)(ws + L.rstd) : nullptr;
+  // the router's normalised fp32 rows, where the permuted rows and h come later
+  float* xn = gamma && (size_t)N * C * 4 <= L.obuf - L.xg ? (float*)(ws + L.xg) : nullptr;
   HIP_TRY(launch_router<IoT>(xi, h->wr_g, h->wr1, h->wr4, h->br, N, C, E,
                              k, idx, topp, hist, logits,
-                             probs, gamma, blk.eps, Cx, rstd, st));
+                             probs, gamma, blk.eps, Cx, rstd, xn, st));
   HIP_TRY(mark(1));
   // A decode step of at most 512 flat ids (N * k) with fp8 weights (no
   // training caches): the gate/up weight-streaming GEMM routes the ids

@@ -1081,8 +1081,73 @@ __global__ __launch_bounds__(256) void router_count_kernel(const int32_t* __rest
   if (tid < E) hist[(size_t)tid * nb + b] = s_hist[tid];
 }
 
-// Decode router for a single block of tokens (N <= 64, E <= 64, no
-// normalisation), logits and softmax in one launch.  A block owns one token
+// A row's 1/rms from its squares in LDS (C of them, a multiple of 64): the sum
+// in column order, one rounded add a term, then r = 1/sqrt(ms/cn + eps) as in
+// logit_chains.  Every lane of the wave computes it.
+__device__ __forceinline__ float row_rstd(const float4* sq, int C, const RowNorm& nrm) {
+  float ms = 0.0f;
+  for (int q0 = 0; q0 < C / 4; q0 += 16) {
+    float4 v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = sq[q0 + u];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      ms = ms + v[u].x;
+      ms = ms + v[u].y;
+      ms = ms + v[u].z;
+      ms = ms + v[u].w;
+    }
+  }
+  return __fdiv_rn(1.0f, sqrt_rn(__fdiv_rn(ms, (float)nrm.cn) + nrm.eps));
+}
+
+// Widest row of router_rownorm_kernel (64 KB of LDS for four rows' squares).
+constexpr int kRowNormMaxC = 4096;
+
+// Normalised rows xn = (x * r) * gamma in fp32, the values the router's products
+// take, and r: a wave per token, its squares in LDS.  The other router kernels
+// then run on xn as on any fp32 rows.
+template <typename ActT>
+__global__ __launch_bounds__(256) void router_rownorm_kernel(const ActT* __restrict__ x, int N,
+                                                             int C, RowNorm nrm,
+                                                             float* __restrict__ rstd,
+                                                             float* __restrict__ xn) {
+  extern __shared__ __align__(16) float4 s_sq[];   // [4 waves][C / 4]
+  const int w = threadIdx.x / kWave, lane = lane_id();
+  const int t = blockIdx.x * 4 + w;
+  if (t >= N) return;
+  constexpr int kPer = 16 / (int)sizeof(ActT);
+  float4* sq = s_sq + (size_t)w * (C / 4);
+  const ActT* xr = x + (size_t)t * C;
+  for (int c = lane * kPer; c < C; c += kWave * kPer) {
+    const uint4 q = *reinterpret_cast<const uint4*>(xr + c);
+#pragma unroll
+    for (int h = 0; h < kPer; h += 4) {
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = widen<ActT>(q, h + i);
+      sq[(c + h) / 4] = make_float4(v[0] * v[0], v[1] * v[1], v[2] * v[2], v[3] * v[3]);
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  const float r = row_rstd(sq, C, nrm);
+  if (lane == 0) rstd[t] = r;
+  for (int c = lane * kPer; c < C; c += kWave * kPer) {
+    const uint4 q = *reinterpret_cast<const uint4*>(xr + c);
+#pragma unroll
+    for (int h = 0; h < kPer; h += 4) {
+      const float* g = nrm.gamma + c + h;
+      *reinterpret_cast<float4*>(xn + (size_t)t * C + c + h) =
+          make_float4((widen<ActT>(q, h) * r) * g[0], (widen<ActT>(q, h + 1) * r) * g[1],
+                      (widen<ActT>(q, h + 2) * r) * g[2], (widen<ActT>(q, h + 3) * r) * g[3]);
+    }
+  }
+}
+
+// Decode router for a single block of tokens (N <= 64, E <= 64), logits and
+// softmax in one launch (NORM: on the normalised row, whose 1/rms each block
+// forms first).  A block owns one token
 // t: wave 0 runs the 64 chains acc = acc + p[c] (lane e = expert e, columns
 // ascending, then the bias: the reference's rounding sequence, as in the
 // other router kernels) and then the softmax / top-k of the token with
@@ -1113,11 +1178,11 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // return zeros (none are issued here).
 constexpr int kBufWord3 = 0x00020000;
 
-template <typename ActT>
+template <typename ActT, bool NORM>
 __global__ __launch_bounds__(256) void router_decode_kernel(
     const ActT* __restrict__ x, const float4* __restrict__ wr4, const float* __restrict__ br,
     int N, int C, int E, int k, int32_t* __restrict__ topk_idx, float* __restrict__ topk_p,
-    float* __restrict__ probs) {
+    float* __restrict__ probs, RowNorm nrm, float* __restrict__ rstd) {
   __shared__ float4 s_x[kDecodeRouterMaxC / 4];          // x[t] widened to fp32
   __shared__ float4 s_p[3][kMaxExperts * kDrPLD / 4];    // products [e][column]
   __shared__ __align__(16) float s_row[kMaxExperts];
@@ -1172,27 +1237,48 @@ __global__ __launch_bounds__(256) void router_decode_kernel(
 #pragma unroll
       for (int j = 0; j < kDrPS - 1; ++j) load(j, wv[j]);
     }
+    auto widened = [&](int pp, float (&v)[8]) __attribute__((always_inline)) {
+      if constexpr (sizeof(ActT) == 2) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = widen<ActT>(xv[pp], i);
+      } else {
+        v[0] = xv[pp].x; v[1] = xv[pp].y; v[2] = xv[pp].z; v[3] = xv[pp].w;
+        v[4] = xv2[pp].x; v[5] = xv2[pp].y; v[6] = xv2[pp].z; v[7] = xv2[pp].w;
+      }
+    };
+    float r = 1.0f;
+    if constexpr (NORM) {
+      // the squares into the (still unused) product buffers, then every wave
+      // adds them up in column order for itself
+      float4* sq = s_p[0];
+#pragma unroll
+      for (int pp = 0; pp < kXP; ++pp) {
+        const int c = 8 * tid + 8 * 256 * pp;
+        if (c >= C) continue;
+        float v[8];
+        widened(pp, v);
+        sq[c / 4] = make_float4(v[0] * v[0], v[1] * v[1], v[2] * v[2], v[3] * v[3]);
+        sq[c / 4 + 1] = make_float4(v[4] * v[4], v[5] * v[5], v[6] * v[6], v[7] * v[7]);
+      }
+      barrier();
+      r = row_rstd(sq, C, nrm);
+      if (tid == 0) rstd[t] = r;
+    }
 #pragma unroll
     for (int pp = 0; pp < kXP; ++pp) {
       const int c = 8 * tid + 8 * 256 * pp;
-      if (c < C) {
-        float4 lo, hi;
-        if constexpr (sizeof(ActT) == 2) {
-          const uint4 v = xv[pp];
-          lo = make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u),
-                           __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xFFFF0000u));
-          hi = make_float4(__uint_as_float(v.z << 16), __uint_as_float(v.z & 0xFFFF0000u),
-                           __uint_as_float(v.w << 16), __uint_as_float(v.w & 0xFFFF0000u));
-        } else {
-          lo = xv[pp];
-          hi = xv2[pp];
-        }
-        s_x[c / 4] = lo;
-        s_x[c / 4 + 1] = hi;
+      if (c >= C) continue;
+      float v[8];
+      widened(pp, v);
+      if constexpr (NORM) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = (v[i] * r) * nrm.gamma[c + i];
       }
+      s_x[c / 4] = make_float4(v[0], v[1], v[2], v[3]);
+      s_x[c / 4 + 1] = make_float4(v[4], v[5], v[6], v[7]);
     }
   }
-  barrier();   // x[t] and the table are in LDS
+  barrier();   // x[t] and the table are in LDS (and, with NORM, the squares read)
 
   if (w > 0) {
     // step j: request W_r of step j + kDrPS - 1 into its stage, then form
@@ -1315,6 +1401,7 @@ __global__ __launch_bounds__(256) void router_decode_kernel(
 // memory; wr1: W_r as [E][C]; wr4 (nullable): W_r as column quads [C/4][E][4].
 // probs (nullable) receives the clamped softmax [N][E] (the reference's
 // cached_router_probs).
+// xn (nullable): room for [N][C] fp32 normalised rows.
 // gamma (nullable): route on RMSNorm(x) * gamma instead of x, writing each
 // token's 1/rms to rstd [N]; cn: the mean's divisor (C, or the caller's width
 // when x's rows are zero-padded to C).
@@ -1325,7 +1412,8 @@ template <typename ActT>
 hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, const float* wr4,
                          const float* br, int N, int C, int E, int k, int32_t* topk_idx,
                          float* topk_p, int32_t* hist, float* logits, float* probs,
-                         const float* gamma, float eps, int cn, float* rstd, hipStream_t stream) {
+                         const float* gamma, float eps, int cn, float* rstd, float* xn,
+                         hipStream_t stream) {
   const RowNorm nrm{gamma, eps, cn};
   const int nb = (N + kRT - 1) / kRT;
   if (nb == 0) return hipSuccess;
@@ -1347,10 +1435,21 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
     else
       go(router_logits_lane_kernel<ActT, 4>, 4);
   };
+  // Normalised rows by way of the paths for plain rows.
+  auto normalised = [&]() {
+    hipLaunchKernelGGL(router_rownorm_kernel<ActT>, dim3((N + 3) / 4), dim3(256), (size_t)C * 16, stream,
+                       x, N, C, nrm, rstd, xn);
+    return launch_router<float>(xn, wr_g, wr1, wr4, br, N, C, E, k, topk_idx, topk_p, hist, logits, probs,
+                                nullptr, 0.0f, C, nullptr, nullptr, stream);
+  };
+  const bool can_norm = gamma && xn && C <= kRowNormMaxC;
   if (E > kMaxExperts) {
     // wide: per-expert logits (the split kernels, any E), then the block
     // softmax / top-k over rows of up to kMaxExpertsWide
     if (E > kMaxExpertsWide || !logits) return hipErrorInvalidValue;
+    // (E = 128, C = 1024, us as above: 64 tokens 55 / 36, 2048 159 / 62, 8192 113 /
+    // 114, 16500 270 / 210)
+    if (can_norm && (C <= 2048 || N < 4096)) return normalised();
     if (!gamma && wr4 && (long)N * eg >= 1024) {
       // a wave a token and 64 experts from one wave per SIMD on (us with the
       // kernels below: E = 128, C = 1024: 512 tokens 41 -> 37, 2048 94 -> 45,
@@ -1380,10 +1479,15 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
                          stream, logits, N, E, k, topk_idx, topk_p, hist, nb, probs);
     return hipGetLastError();
   }
-  if (router_decode_range(N, C, E, gamma != nullptr) && wr4) {
-    hipLaunchKernelGGL((router_decode_kernel<ActT>), dim3(N), dim3(256), 0, stream, x,
-                       reinterpret_cast<const float4*>(wr4), br, N, C, E, k, topk_idx, topk_p,
-                       probs);
+  if (router_decode_range(N, C, E) && wr4) {
+    auto decode = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(N), dim3(256), 0, stream, x, reinterpret_cast<const float4*>(wr4),
+                         br, N, C, E, k, topk_idx, topk_p, probs, nrm, rstd);
+    };
+    if (gamma)
+      decode(router_decode_kernel<ActT, true>);
+    else
+      decode(router_decode_kernel<ActT, false>);
     return hipGetLastError();
   }
   // Without normalisation the logits go through memory, with more blocks than
@@ -1400,12 +1504,35 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
   // blocks.  Up to 16 experts, product and chain waves win while the fused
   // kernel's chains are long against the tokens (E N below 64 C: the limit is
   // 1024 tokens at E = 16, C = 256 and about 3500 from C = 1024 on).
+  //   E = 8: C = 512 65 tokens 16.9 / 15.2, 2048 20 / 19; C = 1024 1024 28 / 22; C =
+  //     2048 2048 43 / 29, 6000 52 / 59
   const bool many = (long)N * E >= 57344;
   const float lane_us = 10.0f + N * (0.9e-3f + 3.6e-6f * C);
   const float fused_us = (10.0f + C * (0.011f + 0.73e-3f * E)) * ((nb + 255) / 256);
   const bool lane = wr4 && many && E > 16 && (N < 4096 || lane_us < fused_us);
-  const bool pc = E > 16 ? N < 4096 : E > 8 && C >= 256 && (long)N * E < std::min(57344L, 64L * C);
-  if (logits && !gamma && (lane || pc)) {
+  const long NE = (long)N * E;
+  const bool pc = E > 16  ? N < 4096
+                  : E > 8 ? C >= 256 && NE < std::min(57344L, 64L * C)
+                          : E > 4 && C >= 512 && NE < 32768;
+  const bool mid = logits && (lane || pc);
+  // With normalisation those paths run on rows normalised once (xn), where that
+  // is faster than the fused kernel or router_logits_kernel, which form the
+  // norm in every wave.  MI355X, us of router and permute, before / here:
+  //   E = 8: C = 1024 65 tokens 40 / 25, 1024 43 / 30; C = 512 2048 28 / 26, 3072
+  //     30 / 31
+  //   E = 16: C = 1024 65 tokens 46 / 26, 2048 50 / 38; C = 2048 2048 86 / 53
+  //   E = 20: C = 1024 1024 tokens 51 / 35, 3072 54 / 56; C = 256 2048 26 / 28
+  //   E = 32: C = 1024 2048 tokens 53 / 46, 3072 86 / 57, 4096 65 / 61, 6000 68 / 70
+  //   E = 64: C = 512 2048 tokens 55 / 35, 6000 55 / 51, 8192 57 / 62; C = 2048 1024
+  //     tokens 86 / 56, 3072 214 / 89, 4096 152 / 93
+  // (past 256 blocks router_logits_kernel needs another round).
+  const bool norm_mid =
+      mid && (E <= 16    ? NE < 48L * std::min(C, 1024)
+              : N < 4096 ? C >= 256 && (nb * ((E + kSplitExperts - 1) / kSplitExperts) > 256 ||
+                                        N <= (C >= 512 ? 2048 : 1024))
+                         : E * C >= 30000 && N <= (E > 32 ? 6144 : 4096));
+  if (can_norm && norm_mid) return normalised();
+  if (mid && !gamma) {
     if (lane)
       lane_logits();
     else
@@ -1462,11 +1589,12 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
 template hipError_t launch_router<float>(const float*, const float*, const float*, const float*,
                                          const float*, int, int, int, int, int32_t*, float*,
                                          int32_t*, float*, float*, const float*, float, int,
-                                         float*, hipStream_t);
+                                         float*, float*, hipStream_t);
 template hipError_t launch_router<bf16_t>(const bf16_t*, const float*, const float*,
                                           const float*, const float*, int, int, int, int,
                                           int32_t*, float*, int32_t*, float*, float*,
-                                          const float*, float, int, float*, hipStream_t);
+                                          const float*, float, int, float*, float*,
+                                          hipStream_t);
 
 // Device expf over a buffer (tests compare it with the host's glibc expf).
 __global__ void expf_probe_kernel(const float* __restrict__ in, float* __restrict__ out, int n) {

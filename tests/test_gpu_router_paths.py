@@ -55,3 +55,46 @@ def test_routing_bit_exact(N, C, E, k, act, train):
     assert np.array_equal(r["topk_p"], ref["topp"])
     assert np.array_equal(r["counts"], ref["counts"])
     assert np.array_equal(r["perm"], ref["perm"])
+
+
+# (N, C, E, k, act, H): normalised rows
+NORM_SHAPES = [
+    # one launch, the block's own 1/rms
+    (1, 64, 1, 1, "f32", 8), (64, 1024, 16, 2, "bf16", 8), (33, 4160, 8, 2, "bf16", 8), (64, 192, 64, 8, "f32", 8),
+    # rows normalised once, on both sides of the lines of its rule
+    (65, 1024, 16, 2, "bf16", 8), (3071, 1024, 16, 2, "bf16", 8), (3072, 1024, 16, 2, "bf16", 8),
+    (258, 512, 8, 2, "f32", 8), (1025, 256, 20, 2, "bf16", 8), (2049, 512, 64, 6, "bf16", 8),
+    (4095, 512, 60, 2, "bf16", 8), (4097, 576, 64, 2, "bf16", 8), (6145, 512, 64, 2, "bf16", 8),
+    # no room for the rows (top-1, few hidden units), rows too wide for their kernel
+    (300, 2048, 16, 1, "bf16", 8), (100, 4160, 16, 2, "bf16", 8),
+    # more than 64 experts
+    (65, 64, 65, 4, "bf16", 8), (513, 128, 128, 8, "f32", 8), (1030, 64, 300, 3, "bf16", 8),
+    # a width that the library pads
+    (70, 200, 16, 2, "bf16", 8), (20, 200, 16, 2, "f32", 8),
+]
+
+
+@pytest.mark.parametrize("N,C,E,k,act,H", NORM_SHAPES)
+def test_normalised_routing_bit_exact(N, C, E, k, act, H):
+    """The same for the fused block's routing on RMSNorm(x) * gamma, with its
+    1/rms, from a gamma that is only 4-byte aligned."""
+    cfg = wl.MoEConfig("paths", N, C, E, k, H, act, act, "normal")
+    inp = wl.make_inputs(cfg, seed=N + E, bias_std=0.02)
+    inp.Wr[:] = wl.normal_f32(7, 3, C * E, std=0.05).reshape(C, E)
+    inp.x[min(3, N - 1), :] = 0.0
+    layer = MoELayer(C, H, E, k, act=act)
+    layer.load_parameters(inp.params())
+    x1 = inp.x.copy()
+    gamma = (np.float32(1.0) + wl.normal_f32(9, 5, C, std=0.2)).astype(np.float32)
+    g = torch.zeros(C + 1, device="cuda")[1:].copy_(torch.from_numpy(gamma))
+    layer.forward_block(torch.from_numpy(x1).to("cuda").to(layer.dtype), g, 1e-5)
+    torch.cuda.synchronize()
+    r = {n: t.cpu().numpy() for n, t in layer.routing().items()}
+    xn, rstd = O.rmsnorm_scaled(x1, gamma, 1e-5)
+    inp.x[:] = xn
+    ref = O.forward(inp, with_y=False)
+    assert np.array_equal(layer.rstd().cpu().numpy(), rstd.reshape(-1))
+    assert np.array_equal(r["topk_idx"], ref["idx"])
+    assert np.array_equal(r["topk_p"], ref["topp"])
+    assert np.array_equal(r["counts"], ref["counts"])
+    assert np.array_equal(r["perm"], ref["perm"])
