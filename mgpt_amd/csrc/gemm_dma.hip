@@ -121,6 +121,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
   int t = (G % kNumXcd == 0) ? (blockIdx.x % kNumXcd) * (G / kNumXcd) + blockIdx.x / kNumXcd
                              : blockIdx.x;
   const int KT = K / 64;
+  if (gridDim.y > 1) {   // a group of 64 experts per grid row
+    const int g0 = (int)blockIdx.y * kMaxExperts;
+    E = min(kMaxExperts, E - g0);
+    e_base += g0;
+    B += (size_t)g0 * Npad * K;
+    if (bias0) bias0 += (size_t)g0 * bias_ld;
+    if (bias1) bias1 += (size_t)g0 * bias_ld;
+  }
   SegScan<256> sc;
   sc.init(counts, E, e_base);
   SplitPlan plan;
@@ -372,37 +380,38 @@ hipError_t launch_gemm_dma(const bf16_t* A, const bf16_t* B, const float* bias0,
     return hipErrorInvalidValue;
   if (K / 64 < kMinSplitSlabs) partials = nullptr;   // no split, no reduce launch
   const int tiles = max_mtiles * (Npad / kBN);
+  // More than 64 experts: groups of 64, the weights and biases from the group's
+  // first expert on; the rows come in expert order, so each group's follow the
+  // earlier groups'.  One launch takes all groups as rows of its grid, so that
+  // the CUs that a group's last round leaves idle go on with the next group;
+  // that round is then not split (us of gate/up + down on MI355X with a launch
+  // and a split reduction per group and so: E = 128, C = 1024, H = 704, 511 rows
+  // an expert 233 + 161 -> 226 + 154; E = 256, C = 768, H = 512, 200 rows 192 +
+  // 107 -> 151 + 94).
+  const int groups = (E + kMaxExperts - 1) / kMaxExperts;
+  if (groups > 1) partials = nullptr;
   // (with split tiles every CU has work, also where there are fewer tiles)
   const int grid = partials || tiles >= num_cus ? num_cus : tiles;
-  // More than 64 experts: one launch (and split reduce) per group of 64, the
-  // weights and biases from the group's first expert on; the rows come in
-  // expert order, so each group's follow the earlier groups'.
-  for (int e0 = 0; e0 < E; e0 += kMaxExperts) {
-    const int Eg = std::min(kMaxExperts, E - e0);
-    const bf16_t* Bg = B + (size_t)e0 * Npad * K;
-    const float* b0 = bias0 ? bias0 + (size_t)e0 * bias_ld : nullptr;
-    const float* b1 = bias1 ? bias1 + (size_t)e0 * bias_ld : nullptr;
-    // the gate/up epilogue's pre-activation stores are compiled only into
-    // the training instance (fewer live registers in the inference one)
-    auto launch = [&](auto save_c) {
-      hipLaunchKernelGGL((gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value>),
-                         dim3(grid), dim3(kRingWaves * kWave), 0, stream, A, Bg, b0, b1, counts,
-                         Eg, e0, K, Npad, n_store, bias_ld, out, ldo, partials, save, save_ld);
-    };
-    if constexpr (EPI == kEpiGateUp) {
-      if (save)
-        launch(std::true_type{});
-      else
-        launch(std::false_type{});
-    } else {
+  // the gate/up epilogue's pre-activation stores are compiled only into
+  // the training instance (fewer live registers in the inference one)
+  auto launch = [&](auto save_c) {
+    hipLaunchKernelGGL((gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value>),
+                       dim3(grid, groups), dim3(kRingWaves * kWave), 0, stream, A, B, bias0, bias1,
+                       counts, E, 0, K, Npad, n_store, bias_ld, out, ldo, partials, save, save_ld);
+  };
+  if constexpr (EPI == kEpiGateUp) {
+    if (save)
+      launch(std::true_type{});
+    else
       launch(std::false_type{});
-    }
-    if constexpr (EPI != kEpiSwigluBwd) {
-      if (partials)
-        hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI, Waves<kRingWaves>>), dim3(8 * grid),
-                           dim3(256), 0, stream, partials, nullptr, b0, b1, counts, Eg, e0, K, Npad,
-                           Npad / kBN, n_store, bias_ld, out, ldo, grid, kMinSplitSlabs);
-    }
+  } else {
+    launch(std::false_type{});
+  }
+  if constexpr (EPI != kEpiSwigluBwd) {
+    if (partials)
+      hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI, Waves<kRingWaves>>), dim3(8 * grid),
+                         dim3(256), 0, stream, partials, nullptr, bias0, bias1, counts, E, 0, K, Npad,
+                         Npad / kBN, n_store, bias_ld, out, ldo, grid, kMinSplitSlabs);
   }
   return hipGetLastError();
 }

@@ -78,9 +78,9 @@ struct Tile {
 constexpr int kGroupM = 4;   // m-tiles per group of the tile order
 
 // Per-expert segment bookkeeping, computed once per wave from counts[] (lane
-// e holds expert e_base + e of the launch's group of E <= 64 experts; more
-// experts run one launch per group, whose rows start after the earlier
-// groups' rows), so that locating a tile needs no memory access and no
+// e holds expert e_base + e of the block's group of E <= 64 experts; more
+// experts take a grid row, or a launch, per group, whose rows start after the
+// earlier groups' rows), so that locating a tile needs no memory access and no
 // barrier.
 template <int BM>
 struct SegScan {

@@ -117,6 +117,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
   int t = (G % kNumXcd == 0) ? (blockIdx.x % kNumXcd) * (G / kNumXcd) + blockIdx.x / kNumXcd
                              : blockIdx.x;
   const int KT = K / 64;
+  if (gridDim.y > 1) {   // a group of 64 experts per grid row
+    const int g0 = (int)blockIdx.y * kMaxExperts;
+    E = min(kMaxExperts, E - g0);
+    e_base += g0;
+    B += (size_t)g0 * Npad * K;
+    if (wscale) wscale += (size_t)g0 * Npad;
+    if (bias0) bias0 += (size_t)g0 * bias_ld;
+    if (bias1) bias1 += (size_t)g0 * bias_ld;
+  }
   SegScan<BM> sc;
   sc.init(counts, E, e_base);
   SplitPlan plan;
@@ -381,15 +390,20 @@ hipError_t launch_gemm_stream(const bf16_t* A, const WT* B, const float* wscale,
     return hipErrorInvalidValue;
   const int BM = small ? 64 : 256, BN = small ? 128 : 256;
   const int nt = EPI == kEpiGateUp ? Npad / BN : (n_store + BN - 1) / BN;
-  // more than 64 experts: one launch per group of 64 (as in gemm_dma.hip)
+  // at most this many tiles (an expert with rows has one more than its whole
+  // ones at most)
+  const int KT = K / 64;
+  const bool split = partials && small && !save && KT >= kStreamMinSlabs &&
+                     2 * ((long)(rows / BM) + (long)std::min<size_t>(E, rows)) * nt <= num_cus;
+  // More than 64 experts: groups of 64.  Whole tiles: one launch, a group per
+  // grid row (as in gemm_dma.hip; us of gate/up + down, E = 128, C = 512, H = 256,
+  // 16 rows an expert 28 + 22 -> 25 + 19; E = 256, C = 512, H = 512, 24 rows 91 +
+  // 57 -> 81 + 46); split ones: a launch and a reduction each.
   for (int e0 = 0; e0 < E; e0 += kMaxExperts) {
-    const int Eg = std::min(kMaxExperts, E - e0);
-    // at most this many tiles (an expert with rows has one more than its
-    // whole ones at most)
-    const long tiles = ((long)(rows / BM) + (long)std::min<size_t>(Eg, rows)) * nt;
-    const int KT = K / 64;
-    float* part = partials;
-    if (!small || save || KT < kStreamMinSlabs || 2 * tiles > num_cus) part = nullptr;
+    const int groups = split ? 1 : (E + kMaxExperts - 1) / kMaxExperts;
+    const int Eg = split ? std::min(kMaxExperts, E - e0) : E;
+    const long tiles = ((long)(rows / BM) + (long)std::min<size_t>(std::min(E, kMaxExperts), rows)) * nt;
+    float* part = split ? partials : nullptr;
     // (with split tiles every CU has work, also where there are fewer tiles)
     const int grid = part ? num_cus : (int)std::min<long>(tiles, num_cus);
     const WT* Bg = B + (size_t)e0 * Npad * K;
@@ -397,7 +411,7 @@ hipError_t launch_gemm_stream(const bf16_t* A, const WT* B, const float* wscale,
     const float* b0 = bias0 ? bias0 + (size_t)e0 * bias_ld : nullptr;
     const float* b1 = bias1 ? bias1 + (size_t)e0 * bias_ld : nullptr;
     auto launch = [&](auto kernel, int threads) {
-      hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, A, Bg, sg, b0, b1, counts, Eg, e0,
+      hipLaunchKernelGGL(kernel, dim3(grid, groups), dim3(threads), 0, stream, A, Bg, sg, b0, b1, counts, Eg, e0,
                          K, Npad, nt, n_store, bias_ld, out, ldo, part, save, save_ld);
     };
     if constexpr (kFp8) {
@@ -422,6 +436,7 @@ hipError_t launch_gemm_stream(const bf16_t* A, const WT* B, const float* wscale,
                            0, stream, part, sg, b0, b1, counts, Eg, e0, K, Npad, nt, n_store, bias_ld,
                            out, ldo, grid, kStreamMinSlabs);
     }
+    if (!split) break;
   }
   return hipGetLastError();
 }

@@ -26,6 +26,9 @@ SHAPES = [
     (255, 128, 1, 1, 128, "fp8"), (257, 128, 1, 1, 192, "fp8"), (300, 192, 3, 2, 160, "fp8"),
     (40, 192, 3, 2, 160, "fp8"), (600, 256, 8, 3, 1408, "fp8"), (260, 128, 80, 3, 96, "fp8"),
     (9, 128, 70, 2, 96, "fp8"),
+    # groups of 64 experts as rows of one grid: split and whole tiles, 256-row tiles
+    (2, 64, 130, 2, 2112, "bf16"), (700, 64, 130, 1, 64, "bf16"), (2400, 64, 70, 2, 96, "bf16"),
+    (4300, 128, 130, 2, 64, "bf16"), (2500, 128, 70, 2, 96, "fp8"),
 ]
 
 
