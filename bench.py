@@ -78,21 +78,21 @@ def stage_of(kernel_name: str):
         return "router_wgrad"
     if "rmsnorm_bwd" in short or "rmsnorm_dgamma" in short:
         return "ln2_bwd"
-    m = re.search(r"wgrad(?:_tr)?_kernel<(?:[^,>]*, )?(\d)>", short)
+    m = re.search(r"wgrad_(?:tr|f32)_kernel<(\d)[,>]", short)
     if m:
         return ("wgrad_down", "wgrad_gateup")[int(m.group(1))]
-    if re.search(r"router_(?:topk|logits|softmax|decode)", short):
+    if re.search(r"router_(?:topk|logits|softmax|decode|rownorm|count)", short):
         return "router_topk"
     if "permute_kernel" in short:
         return "permute"
     if re.search(r"combine\d?_kernel", short):
         return "combine"
-    m = re.search(r"gemm_(?:dma|ring5|decode|split_reduce)_kernel<(\d)[,>]", short)
+    m = re.search(r"gemm_(?:ring5|stream|f32|decode|split_reduce)_kernel<(\d)[,>]", short)
     if m:
         return ("gemm_gateup", "gemm_down", "gemm_dact_swiglu_bwd")[int(m.group(1))]
     m = re.search(r"grouped_gemm_kernel<([^>]*)>", short)
     if m:
-        epi = int(m.group(1).split(",")[6])
+        epi = int(m.group(1).split(",")[4])
         return ("gemm_gateup", "gemm_down", "gemm_dact_swiglu_bwd")[epi]
     if "MulFunctor" in kernel_name:
         return "calib_copy"

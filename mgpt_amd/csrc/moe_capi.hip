@@ -35,7 +35,7 @@
 #include "common.hpp"
 
 namespace mgpt {
-// kernels (router.hip, dispatch.hip, gemm.hip, combine.hip, pack.hip)
+// kernels (router.hip, dispatch.hip, combine.hip, pack.hip and the gemm_*.hip)
 template <typename ActT>
 hipError_t launch_router(const ActT*, const float*, const float*, const float*, const float*, int,
                          int, int, int, int32_t*, float*, int32_t*, float*, float*, const float*,
