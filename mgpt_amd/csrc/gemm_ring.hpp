@@ -57,9 +57,14 @@ __device__ __forceinline__ float uniform_load(const float* p) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(*p)));
 }
 
+// silu(g) * u and the sigmoid, by the hardware reciprocal (1 ulp) or divided.
+// The reciprocal form multiplies g by u first, so a product past fp32's range
+// (|g u| > 3.4e38) gives infinity, or NaN where the reciprocal is 0; the divided
+// one makes g small first.
 __device__ __forceinline__ float silu_mul_fast(float g, float u) {
   return g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
 }
+__device__ __forceinline__ float silu_mul(float g, float u) { return (g / (1.0f + __expf(-g))) * u; }
 
 // Four floats -> four bf16 (round to nearest even) in 8 bytes.
 __device__ __forceinline__ uint2 pack4_bf16(float a, float b, float c, float d) {
@@ -207,8 +212,9 @@ __device__ __forceinline__ void load_group32(const bf16_t* base, uint2 (&q)[4], 
 // 8*(v/4) + 4*(lane/32) + v%4 (four consecutive features per group v/4) and
 // token column lane%32.  Biases are read at wave-uniform addresses (scalar
 // loads): a vector load here would make the compiler wait for the DMA loads
-// it does not track as well.
-template <int EPI, typename W, bool kSave, bool kTight = false>
+// it does not track as well.  kStream (gemm_stream.hip): one sub-tile at a
+// time, and silu and the sigmoid divided.
+template <int EPI, typename W, bool kSave, bool kStream = false>
 __device__ __forceinline__ void store_tile(const f32x16 (&acc)[W::TN][W::TM],
                                            const Tile& cur, int wn, int wm, int lrow, int lhalf,
                                            int n_store, bf16_t* out, int ldo, bf16_t* save,
@@ -224,12 +230,13 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[W::TN][W::TM],
         const int row = tok_base + i * 32;
         const f32x16 ga = acc_fetch<W>(acc[2 * gi][i]);
         const f32x16 ua = acc_fetch<W>(acc[2 * gi + 1][i]);
+        auto act = [](float gv, float uv) { return kStream ? silu_mul(gv, uv) : silu_mul_fast(gv, uv); };
         uint2 q[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int v = 4 * g;
-          q[g] = pack4_bf16(silu_mul_fast(ga[v + 0], ua[v + 0]), silu_mul_fast(ga[v + 1], ua[v + 1]),
-                            silu_mul_fast(ga[v + 2], ua[v + 2]), silu_mul_fast(ga[v + 3], ua[v + 3]));
+          q[g] = pack4_bf16(act(ga[v + 0], ua[v + 0]), act(ga[v + 1], ua[v + 1]),
+                            act(ga[v + 2], ua[v + 2]), act(ga[v + 3], ua[v + 3]));
         }
         store_group32(out + (size_t)row * ldo + hb, q, lhalf, row < cur.row_end);
         if constexpr (kSave) {
@@ -245,7 +252,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[W::TN][W::TM],
           store_group32(save + (size_t)row * save_ld + pc, sg, lhalf, row < cur.row_end);
           store_group32(save + (size_t)row * save_ld + pc + 32, su, lhalf, row < cur.row_end);
         }
-        if constexpr (kTight) __builtin_amdgcn_sched_barrier(0);   // one sub-tile at a time
+        if constexpr (kStream) __builtin_amdgcn_sched_barrier(0);   // one sub-tile at a time
       }
       // one column group at a time: keeps the scheduler from hoisting every
       // accumulator read (TN * TM * 16 values) ahead of the stores
@@ -292,7 +299,8 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[W::TN][W::TM],
               const float gv = __uint_as_float((q & 1) ? (gw & 0xFFFF0000u) : (gw << 16));
               const float uv = __uint_as_float((q & 1) ? (uw & 0xFFFF0000u) : (uw << 16));
               const float d = a[4 * g + q];
-              const float sig = __builtin_amdgcn_rcpf(1.0f + __expf(-gv));
+              const float den = 1.0f + __expf(-gv);
+              const float sig = kStream ? 1.0f / den : __builtin_amdgcn_rcpf(den);
               du[q] = d * (gv * sig);
               dg[q] = (d * uv) * (sig * (1.0f + gv * (1.0f - sig)));
             }

@@ -72,3 +72,22 @@ def test_training_through_few_rows(N, C, E, k, H):
     for name, a in zip(("dx",) + tuple(O.GRAD_NAMES), got):
         b = np.asarray(ref[name], np.float64).reshape(a.shape)
         assert np.linalg.norm(a - b) <= 2e-2 * np.linalg.norm(b) + 1e-12, name
+
+
+@pytest.mark.parametrize("N,C,E,k,H,weights", [(24, 128, 4, 2, 256, "bf16"), (1, 64, 70, 2, 64, "bf16"),
+                                               (600, 128, 4, 2, 192, "fp8"), (40, 192, 3, 2, 160, "fp8")])
+def test_gate_times_up_past_the_range(N, C, E, k, H, weights):
+    """silu(g) * u where g * u overflows but the result does not: g = -1e20 and
+    u = 1e20 give -0, so each expert returns its output bias."""
+    gen = torch.Generator().manual_seed(N)
+    p = [torch.randn(C, E, generator=gen), torch.zeros(1, E)]
+    for e in range(E):
+        p += [torch.zeros(C, H), torch.full((1, H), -1e20), torch.zeros(C, H), torch.full((1, H), 1e20),
+              torch.randn(H, C, generator=gen), torch.full((1, C), 1.0 + e % 4)]
+    layer = MoELayer(C, H, E, k, act="bf16", weights=weights)
+    layer.load_parameters([t.cuda() for t in p])
+    y = layer.forward(torch.randn(N, C, generator=gen).cuda().bfloat16()).float().cpu()
+    r = layer.routing()
+    want = (r["topk_p"].cpu() * (1.0 + (r["topk_idx"].cpu() % 4))).sum(1, keepdim=True).expand(N, C)
+    # a bf16 rounding of the output
+    assert (y - want).abs().max() <= 2.0 ** -8 * want.abs().max()
