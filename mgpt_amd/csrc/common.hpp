@@ -191,6 +191,14 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ counts, in
   return out->expert >= 0;
 }
 
+// Where column k of a row of fp8 weights [E][Npad][K] sits: within each 64
+// columns, the sixteen bytes 16p + 32h .. hold columns 32p + 8h .. +7 and 32p + 16 +
+// 8h .. +7, a lane half's (h) operands of the k-steps 2p and 2p + 1 of a matrix
+// instruction that contracts 16 consecutive columns.
+__host__ __device__ __forceinline__ int fp8_col(int k) {
+  return (k & ~63) | ((k & 8) << 2) | ((k & 32) >> 1) | ((k & 16) >> 1) | (k & 7);
+}
+
 // A batch of gradient additions dst_j[r][c] += src[off_j + r * lds_j + c]
 // (launch_add_jobs; passed by value as a kernel argument).
 // 96 tensors a launch keep the argument block under 3 KB (a layer of 8

@@ -15,9 +15,10 @@
 //    256) instead of 64 KB, so both operands lead by two slabs in 144 KB; the
 //    64 x 128 tiles take 24 KB (bf16) or 16 KB (fp8) a slab, with 112 to 120 KB
 //    of loads in flight a CU, which a weight stream from HBM needs.
-//  * Within a slab, lane half h and k-step ks stand for columns 32h + 8ks ..
-//    +7 in both operands, so a lane's fp8 weights of two k-steps are one
-//    16-byte LDS read; they become bf16 in registers (exact).  fp8 rows are 64
+//  * A k-step ks contracts columns 16ks .. 16ks+15 of the slab, lane half h
+//    columns 16ks + 8h .. +7, as in the other bf16 products (the same sums, bit
+//    for bit); the packed fp8 rows keep a lane's weights of two k-steps in one
+//    16-byte LDS read (fp8_col); they become bf16 in registers (exact).  fp8 rows are 64
 //    bytes: 16-byte chunk c of row r sits at slot c ^ ((r >> 2) & 3), which
 //    spreads the 16 lanes served together over all banks.
 //  * Scales and biases are applied after the contraction from scalar loads (a
@@ -226,7 +227,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
   bf16x8 wf[2][kFp8 ? 1 : kTN];   // bf16 weights by k-step
   uint4 wr[2][kFp8 ? kTN : 1];    // fp8 weights by pair of k-steps
   auto frags = [&](int stage, int ks) __attribute__((always_inline)) {
-    const int cofs = ((4 * lhalf + ks) ^ swz) << 4;
+    const int cofs = ((2 * ks + lhalf) ^ swz) << 4;
 #pragma unroll
     for (int i = 0; i < kTM; ++i)
       xf[ks & 1][i] = *reinterpret_cast<const bf16x8*>(x_base + stage * kStage + i * 32 * kARow + cofs);

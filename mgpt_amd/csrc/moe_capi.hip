@@ -1596,7 +1596,7 @@ int mgpt_moe_export_fp8(const mgpt_moe* h, int expert, int which, uint8_t* q_hos
     for (int n = 0; n < H; ++n) {
       const int prow = (n / 32) * 64 + (n % 32) + 32 * which;
       scale_host[n] = s[prow];
-      for (int c = 0; c < Cx; ++c) q_host[(size_t)c * H + n] = q[(size_t)prow * C + c];
+      for (int c = 0; c < Cx; ++c) q_host[(size_t)c * H + n] = q[(size_t)prow * C + fp8_col(c)];
     }
   } else {
     std::vector<uint8_t> q((size_t)Cp * Hp);
@@ -1607,7 +1607,7 @@ int mgpt_moe_export_fp8(const mgpt_moe* h, int expert, int which, uint8_t* q_hos
                       hipMemcpyDeviceToHost));
     for (int c = 0; c < Cx; ++c) {
       scale_host[c] = s[c];
-      for (int n = 0; n < H; ++n) q_host[(size_t)n * Cx + c] = q[(size_t)c * Hp + n];
+      for (int n = 0; n < H; ++n) q_host[(size_t)n * Cx + c] = q[(size_t)c * Hp + fp8_col(n)];
     }
   }
   return MGPT_OK;

@@ -64,7 +64,8 @@ __device__ __forceinline__ uint8_t f32_to_e4m3(float v) {
   return (uint8_t)(code | ((sign && code) ? 0x80u : 0u));
 }
 
-// Row-wise quantisation of src [rows][K] fp32 -> q [rows][K] e4m3, scale[rows].
+// Row-wise quantisation of src [rows][K] fp32 -> q [rows][K] e4m3 (columns at
+// fp8_col), scale[rows].
 __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* __restrict__ src, int K,
                                                             uint8_t* __restrict__ q,
                                                             float* __restrict__ scale) {
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* __restr
   __syncthreads();
   const float amax = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
   const float s = amax > 0.0f ? amax / 448.0f : 1.0f;
-  for (int k = threadIdx.x; k < K; k += 256) q[r * K + k] = f32_to_e4m3(row[k] / s);
+  for (int k = threadIdx.x; k < K; k += 256) q[r * K + fp8_col(k)] = f32_to_e4m3(row[k] / s);
   if (threadIdx.x == 0) scale[r] = s;
 }
 
@@ -243,10 +244,11 @@ __global__ __launch_bounds__(256) void copy_cols_kernel(const T* __restrict__ sr
     dst[r * ldd + c] = c < ncopy ? src[r * lds + c] : T(0);
 }
 
-// fp8 weights [E][Npad][K] -> the decode stream's tiles
+// fp8 weights [E][Npad][K] (columns at fp8_col) -> the decode stream's tiles
 // [E][Npad/256][K/128][256][128]: every 256-row x 128-column stage the decode
-// GEMM loads is one contiguous 32 KB block.  One thread per 16-byte chunk.
-__global__ __launch_bounds__(256) void tile_fp8_kernel(const uint4* __restrict__ src, int Npad,
+// GEMM loads is one contiguous 32 KB block, columns in their own order.  One
+// thread per 16-byte chunk.
+__global__ __launch_bounds__(256) void tile_fp8_kernel(const uint8_t* __restrict__ src, int Npad,
                                                        int K, size_t chunks,
                                                        uint4* __restrict__ dst) {
   const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -258,7 +260,10 @@ __global__ __launch_bounds__(256) void tile_fp8_kernel(const uint4* __restrict__
   const int n = (int)(row % Npad);
   const int KT = K / 128;
   const size_t tile = (e * (size_t)(Npad / 256) + n / 256) * KT + c16 / 8;
-  dst[(tile * 256 + n % 256) * 8 + c16 % 8] = src[q];
+  const uint8_t* r = src + row * K;
+  const uint2 lo = *reinterpret_cast<const uint2*>(r + fp8_col(16 * c16));
+  const uint2 hi = *reinterpret_cast<const uint2*>(r + fp8_col(16 * c16 + 8));
+  dst[(tile * 256 + n % 256) * 8 + c16 % 8] = make_uint4(lo.x, lo.y, hi.x, hi.y);
 }
 
 // dst_j[r][c] += src[off_j + r * lds_j + c]: the handle's gradients added
@@ -293,8 +298,7 @@ hipError_t launch_tile_fp8(const uint8_t* src, int E, int Npad, int K, uint8_t* 
   if (Npad % 256 != 0 || K % 128 != 0) return hipErrorInvalidValue;
   const size_t chunks = (size_t)E * Npad * (K / 16);
   hipLaunchKernelGGL(tile_fp8_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, stream,
-                     reinterpret_cast<const uint4*>(src), Npad, K, chunks,
-                     reinterpret_cast<uint4*>(dst));
+                     src, Npad, K, chunks, reinterpret_cast<uint4*>(dst));
   return hipGetLastError();
 }
 

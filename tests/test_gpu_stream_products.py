@@ -91,3 +91,36 @@ def test_gate_times_up_past_the_range(N, C, E, k, H, weights):
     want = (r["topk_p"].cpu() * (1.0 + (r["topk_idx"].cpu() % 4))).sum(1, keepdim=True).expand(N, C)
     # a bf16 rounding of the output
     assert (y - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+
+
+# every expert gets rows in both calls: few rows (64 x 128 tiles; fp8 from 32 rows an
+# expert on 256 x 256 ones) against at least 64 an expert in 128 x 128 tiles
+@pytest.mark.parametrize("N,C,E,k,H,weights", [(40, 192, 4, 2, 160, "bf16"),
+                                               (40, 192, 4, 2, 160, "fp8"), (300, 192, 4, 2, 160, "fp8"),
+                                               (400, 512, 8, 3, 704, "fp8")])
+def test_same_bits_as_the_128_row_tiles(N, C, E, k, H, weights, monkeypatch):
+    """One order of sums, one form of the epilogue: the products equal those of the
+    register-staged 128 x 128 tiles bit for bit.  fp8 weights lie on the e4m3 grid with
+    power-of-two scales, so the same values are exact in bf16 and the scales commute
+    with every rounding."""
+    gen = torch.Generator().manual_seed(N + C)
+
+    def weight(i, o):
+        q = (torch.randn(i, o, generator=gen) * 20).to(torch.float8_e4m3fn).float()
+        q[0] = 448.0   # the channel's largest: scale 2^-9
+        return q * 2.0 ** -9
+
+    p = [torch.randn(C, E, generator=gen) * 0.1, torch.zeros(1, E)]
+    for _ in range(E):
+        p += [weight(C, H), torch.randn(1, H, generator=gen), weight(C, H), torch.randn(1, H, generator=gen),
+              weight(H, C), torch.randn(1, C, generator=gen)]
+    p = [t.cuda() for t in p]
+    x = torch.randn(N, C, generator=gen).cuda().bfloat16()
+    layer = MoELayer(C, H, E, k, act="bf16", weights=weights)
+    layer.load_parameters(p)
+    y = layer.forward(x)
+    monkeypatch.setenv("MGPT_MOE_GEMM_TILE", "128")
+    tiles = MoELayer(C, H, E, k, act="bf16")
+    tiles.load_parameters(p)
+    many = x.repeat(-(-64 * E // (N * k)), 1)
+    assert torch.equal(y, tiles.forward(many)[:N])
