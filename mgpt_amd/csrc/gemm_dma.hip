@@ -410,8 +410,8 @@ hipError_t launch_gemm_dma(const bf16_t* A, const bf16_t* B, const float* bias0,
   if constexpr (EPI != kEpiSwigluBwd) {
     if (partials)
       hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI, Waves<kRingWaves>>), dim3(8 * grid),
-                         dim3(256), 0, stream, partials, nullptr, bias0, bias1, counts, E, 0, K, Npad,
-                         Npad / kBN, n_store, bias_ld, out, ldo, grid, kMinSplitSlabs);
+                         dim3(256), 0, stream, partials, bias0, bias1, counts, E, 0, K, Npad / kBN,
+                         n_store, bias_ld, out, ldo, grid);
   }
   return hipGetLastError();
 }

@@ -347,13 +347,11 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[W::TN][W::TM],
 constexpr int kMinSplitSlabs = 24;
 struct SplitPlan {
   int full, rem, s, items;
-  // min_slabs: tiles of fewer slabs stay whole
-  __device__ __forceinline__ void init(int T, int G, int KT, bool enable,
-                                       int min_slabs = kMinSplitSlabs) {
+  __device__ __forceinline__ void init(int T, int G, int KT, bool enable) {
     full = (T / G) * G;
     rem = T - full;
     s = 1;
-    if (enable && rem > 0 && KT >= min_slabs) {
+    if (enable && rem > 0 && KT >= kMinSplitSlabs) {
       s = min(min(G / rem, 8), KT);
       if (s < 2) s = 1;
     }
@@ -398,15 +396,12 @@ __device__ __forceinline__ bool locate_work(const SegScan<BM>& sc, const SplitPl
 // iteration: the s float4 loads of a quad are independent, so each thread
 // keeps them all in flight, and the quads of all split tiles are spread over
 // the whole grid.  The (GEMM thread, slot) -> (token, feature) mapping is
-// the one store_tile applies to the GEMM's accumulators.  wscale (fp8 weights,
-// else null): the per-channel scales, applied before the bias.
+// the one store_tile applies to the GEMM's accumulators.
 template <int EPI, typename W>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(
-    const float* __restrict__ partials, const float* __restrict__ wscale,
-    const float* __restrict__ bias0,
+    const float* __restrict__ partials, const float* __restrict__ bias0,
     const float* __restrict__ bias1, const int32_t* __restrict__ counts, int E, int e_base, int K,
-    int Npad, int nbx, int n_store, int bias_ld, bf16_t* __restrict__ out, int ldo, int G,
-    int min_slabs) {
+    int nbx, int n_store, int bias_ld, bf16_t* __restrict__ out, int ldo, int G) {
   constexpr int kPartialFloats = W::kBM * W::kBN;
   constexpr int kTM = W::TM, kT = W::kThreads;
   constexpr bool kGU = EPI == kEpiGateUp;
@@ -416,7 +411,7 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(
   SegScan<W::kBM> sc;
   sc.init(counts, E, e_base);
   SplitPlan plan;
-  plan.init(sc.tm * nbx, G, KT, true, min_slabs);
+  plan.init(sc.tm * nbx, G, KT, true);
   if (plan.s == 1) return;
   const int total = plan.rem * kQuads;
   // kQuads is a multiple of 256, so r (and the tile) is uniform per block
@@ -442,11 +437,6 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(
       }
       const int hb = (tile.n0 + wn * W::WTN) / 2 + 32 * j;
       const int f = hb + 8 * g + 4 * lhalf;
-      if (wscale) {   // packed rows: 32 gate, then 32 up
-        const float* s = wscale + (size_t)tile.expert * Npad + 2 * hb + 8 * g + 4 * lhalf;
-        ga.x *= s[0]; ga.y *= s[1]; ga.z *= s[2]; ga.w *= s[3];
-        ua.x *= s[32]; ua.y *= s[33]; ua.z *= s[34]; ua.w *= s[35];
-      }
       const float* bg = bias0 + (size_t)tile.expert * bias_ld + f;
       const float* bu = bias1 + (size_t)tile.expert * bias_ld + f;
       *reinterpret_cast<uint2*>(out + (size_t)row * ldo + f) =
@@ -464,10 +454,6 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(
         a.x += x.x; a.y += x.y; a.z += x.z; a.w += x.w;
       }
       const int f = cb + 8 * g + 4 * lhalf;
-      if (wscale) {
-        const float* s = wscale + (size_t)tile.expert * Npad + f;
-        a.x *= s[0]; a.y *= s[1]; a.z *= s[2]; a.w *= s[3];
-      }
       float b[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       if (bias0) {
         const float* bp = bias0 + (size_t)tile.expert * bias_ld + f;

@@ -26,11 +26,6 @@
 //  * Few rows take 64 x 128 tiles (4 waves): the narrower they are, the more
 //    evenly a step's few tiles spread over the CUs (16 experts of H = 2816:
 //    704 gate/up tiles are 2.75 rounds, 352 of 256 columns 1.4, paid as 2).
-//  * Where the tiles do not reach half the CUs and the contraction is long,
-//    they are split along K like gemm_dma's last round (us for the down product
-//    with and without, its reduction included, E = 16, C = 1024, H = 2816: 1
-//    token 14.8 / 22.7, 4 tokens 18.5 / 24.7, 24 tokens 27.2 / 29.7; H = 1408:
-//    24 tokens 19.3 / 17.5, so a contraction of 22 slabs stays whole).
 //
 // Measured on MI355X, stage times with cold weights, against the register-staged
 // 32 x 256 (bf16) and 128 x 128 (fp8) tiles used before, gate/up + down us:
@@ -64,8 +59,6 @@ __device__ __forceinline__ bf16x8 fp8x8_to_bf16x8(uint32_t lo, uint32_t hi) {
   __builtin_memcpy(&r, w, 16);
   return r;
 }
-
-constexpr int kStreamMinSlabs = 32;   // shorter contractions stay whole
 
 // acc = acc * scale + bias, per output feature (register v of a 32x32 tile
 // holds feature 8*(v/4) + 4*lhalf + v%4 of the tile, a token per lane);
@@ -102,8 +95,8 @@ template <int EPI, typename WT, int NW, int BM, int BN, int ST, bool kSave>
 __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
     const bf16_t* __restrict__ A, const WT* __restrict__ B, const float* __restrict__ wscale,
     const float* __restrict__ bias0, const float* __restrict__ bias1,
-    const int32_t* __restrict__ counts, int E, int e_base, int K, int Npad, int nbx,
-    int n_store, int bias_ld, bf16_t* out, int ldo, float* __restrict__ partials, bf16_t* save, int save_ld) {
+    const int32_t* __restrict__ counts, int E, int K, int Npad, int nbx,
+    int n_store, int bias_ld, bf16_t* out, int ldo, bf16_t* save, int save_ld) {
   using W = Waves<NW, BM, BN>;
   constexpr int kTN = W::TN, kTM = W::TM;
   constexpr bool kFp8 = sizeof(WT) == 1;
@@ -118,10 +111,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
   int t = (G % kNumXcd == 0) ? (blockIdx.x % kNumXcd) * (G / kNumXcd) + blockIdx.x / kNumXcd
                              : blockIdx.x;
   const int KT = K / 64;
+  int e_base = 0;
   if (gridDim.y > 1) {   // a group of 64 experts per grid row
     const int g0 = (int)blockIdx.y * kMaxExperts;
     E = min(kMaxExperts, E - g0);
-    e_base += g0;
+    e_base = g0;
     B += (size_t)g0 * Npad * K;
     if (wscale) wscale += (size_t)g0 * Npad;
     if (bias0) bias0 += (size_t)g0 * bias_ld;
@@ -129,10 +123,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
   }
   SegScan<BM> sc;
   sc.init(counts, E, e_base);
-  SplitPlan plan;
-  plan.init(sc.tm * nbx, G, KT, partials != nullptr, kStreamMinSlabs);
-  Work cur;
-  if (!locate_work<BN>(sc, plan, E, nbx, KT, t, &cur)) return;
+  Tile cur;
+  if (!locate_tile<BN>(sc, E, nbx, t, &cur)) return;
 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = lane_id();
@@ -158,19 +150,19 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
   const uint32_t lds_a = (uint32_t)(uintptr_t)(lds_char*)smem + (uint32_t)(w * kDA * 1024);
   const uint32_t lds_b = (uint32_t)(uintptr_t)(lds_char*)smem + (uint32_t)(kABytes + w * kDB * 1024);
 
-  // Cursor over slabs (work item dwk, slab dkt, ring stage dstage).  Past the
+  // Cursor over slabs (tile dtl, slab dkt, ring stage dstage).  Past the
   // end of the block's work it repeats the last slab (in bounds, into a freed
   // stage), so every slab issues the same loads and waits the same way.
-  Work dwk = cur;
-  int dt = t, dkt = cur.k0, dstage = 0;
+  Tile dtl = cur;
+  int dt = t, dkt = 0, dstage = 0;
   bool dvalid = true;
   const char *dga, *dgb;
   uint32_t ga_off[kDA];
   auto enter_item = [&]() __attribute__((always_inline)) {
-    dga = reinterpret_cast<const char*>(A + (size_t)dwk.tile.row0 * K);
-    dgb = reinterpret_cast<const char*>(B + ((size_t)dwk.tile.expert * Npad + dwk.tile.n0) * K);
+    dga = reinterpret_cast<const char*>(A + (size_t)dtl.row0 * K);
+    dgb = reinterpret_cast<const char*>(B + ((size_t)dtl.expert * Npad + dtl.n0) * K);
     // (few rows: those past the segment re-read its last one, in L1)
-    const int rows = dwk.tile.row_end - dwk.tile.row0;
+    const int rows = dtl.row_end - dtl.row0;
 #pragma unroll
     for (int i = 0; i < kDA; ++i)
       ga_off[i] = a_off[i] + (uint32_t)(BM <= 64 ? min(a_row[i], rows - 1) : a_row[i]) * (uint32_t)(K * 2);
@@ -184,13 +176,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
     uda = lds_a + (uint32_t)(dstage * kStage);
     udb = lds_b + (uint32_t)(dstage * kStage);
     dstage = dstage + 1 == ST ? 0 : dstage + 1;
-    if (dvalid && ++dkt == dwk.k1) {
+    if (dvalid && ++dkt == KT) {
       dt += G;
-      Work nx;
-      dvalid = locate_work<BN>(sc, plan, E, nbx, KT, dt, &nx);
+      Tile nx;
+      dvalid = locate_tile<BN>(sc, E, nbx, dt, &nx);
       if (dvalid) {
-        dwk = nx;
-        dkt = dwk.k0;
+        dtl = nx;
+        dkt = 0;
       } else {
         --dkt;
       }
@@ -259,8 +251,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
   frags(0, 0);
 
   for (;;) {
-    Work nxt;
-    const bool have_next = locate_work<BN>(sc, plan, E, nbx, KT, t + G, &nxt);
+    Tile nxt;
+    const bool have_next = locate_tile<BN>(sc, E, nbx, t + G, &nxt);
     f32x16 acc[kTN][kTM];
 #pragma unroll
     for (int j = 0; j < kTN; ++j)
@@ -273,7 +265,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
     auto kloop = [&](auto mt_c) __attribute__((always_inline)) {
       constexpr int MT = decltype(mt_c)::value;
       constexpr int kMfma = kTN * MT;
-      for (int kt = cur.k0; kt < cur.k1; ++kt) {
+      for (int kt = 0; kt < KT; ++kt) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
           if (ks < 3) {
@@ -310,7 +302,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
         }
       }
     };
-    const int wrows = cur.tile.row_end - (cur.tile.row0 + wm * W::WTM);
+    const int wrows = cur.row_end - (cur.row0 + wm * W::WTM);
     const int mt_live = wrows <= 0 ? 0 : min(kTM, (wrows + 31) / 32);
     if constexpr (kTM == 4) {
       switch (mt_live) {
@@ -329,38 +321,25 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
       else kloop(IntC<1>{});
     }
     if (mt_live > 0) {
-      if (cur.sidx < 0) {
-        // the lane recomputed rather than kept live across the k loop (the 256-
-        // row tiles run at the register limit)
-        int lane_now;
-        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_now));
-        const int lrow = lane_now & 31, lhalf = lane_now >> 5;
-        const size_t e = cur.tile.expert;
-        const int nw = cur.tile.n0 + wn * W::WTN;
-        if constexpr (EPI == kEpiGateUp) {
-          const int hb = nw / 2;   // [32 gate | 32 up] of units hb .. hb+31
-          affine<W>(acc, 0, kFp8 ? wscale + e * Npad + nw : nullptr, bias0 + e * bias_ld + hb, lhalf);
-          affine<W>(acc, 1, kFp8 ? wscale + e * Npad + nw + 32 : nullptr, bias1 + e * bias_ld + hb, lhalf);
-        } else if constexpr (EPI == kEpiDown) {
-#pragma unroll
-          for (int j = 0; j < kTN; ++j)
-            if (kFp8 || bias0)
-              affine<W>(acc, j, kFp8 ? wscale + e * Npad + nw + 32 * j : nullptr,
-                        bias0 ? bias0 + e * bias_ld + nw + 32 * j : nullptr, lhalf);
-        }
-        store_tile<EPI, W, kSave, true>(acc, cur.tile, wn, wm, lrow, lhalf, n_store, out, ldo, save, save_ld);
-      } else {
-        float4* P = reinterpret_cast<float4*>(partials + (size_t)cur.sidx * (BM * BN)) + tid;
+      // the lane recomputed rather than kept live across the k loop (the 256-
+      // row tiles run at the register limit)
+      int lane_now;
+      asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_now));
+      const int lrow = lane_now & 31, lhalf = lane_now >> 5;
+      const size_t e = cur.expert;
+      const int nw = cur.n0 + wn * W::WTN;
+      if constexpr (EPI == kEpiGateUp) {
+        const int hb = nw / 2;   // [32 gate | 32 up] of units hb .. hb+31
+        affine<W>(acc, 0, kFp8 ? wscale + e * Npad + nw : nullptr, bias0 + e * bias_ld + hb, lhalf);
+        affine<W>(acc, 1, kFp8 ? wscale + e * Npad + nw + 32 : nullptr, bias1 + e * bias_ld + hb, lhalf);
+      } else if constexpr (EPI == kEpiDown) {
 #pragma unroll
         for (int j = 0; j < kTN; ++j)
-#pragma unroll
-          for (int i = 0; i < kTM; ++i)
-#pragma unroll
-            for (int v4 = 0; v4 < 4; ++v4)
-              P[((j * kTM + i) * 4 + v4) * W::kThreads] =
-                  make_float4(acc[j][i][4 * v4], acc[j][i][4 * v4 + 1], acc[j][i][4 * v4 + 2],
-                              acc[j][i][4 * v4 + 3]);
+          if (kFp8 || bias0)
+            affine<W>(acc, j, kFp8 ? wscale + e * Npad + nw + 32 * j : nullptr,
+                      bias0 ? bias0 + e * bias_ld + nw + 32 * j : nullptr, lhalf);
       }
+      store_tile<EPI, W, kSave, true>(acc, cur, wn, wm, lrow, lhalf, n_store, out, ldo, save, save_ld);
     }
     if (!have_next) break;
     t += G;
@@ -372,16 +351,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
 }  // namespace
 
 // Persistent launch, one block per CU.  Tiles of 64 rows x 128 features
-// (small) or 256 x 256.  partials (num_cus x 64 x 128 floats, small tiles
-// only, or null): the split last round's.  save: the training pre-activations
-// (gate/up: written; SwiGLU backward: read, bf16 weights only).  K % 64 == 0,
-// Npad % 256 == 0, n_store % 64 == 0; A has 256 rows of slack.
+// (small) or 256 x 256.  save: the training pre-activations (gate/up: written;
+// SwiGLU backward: read, bf16 weights only).  K % 64 == 0, Npad % 256 == 0,
+// n_store % 64 == 0; A has 256 rows of slack.
 template <int EPI, typename WT>
 hipError_t launch_gemm_stream(const bf16_t* A, const WT* B, const float* wscale, const float* bias0,
                               const float* bias1, const int32_t* counts, int E, int K, int Npad,
                               int n_store, int bias_ld, bf16_t* out, int ldo, size_t rows, bool small,
-                              float* partials, int num_cus, bf16_t* save, int save_ld,
-                              hipStream_t stream) {
+                              int num_cus, bf16_t* save, int save_ld, hipStream_t stream) {
   constexpr bool kFp8 = sizeof(WT) == 1;
   if (rows == 0) return hipSuccess;
   if (E <= 0 || E > kMaxExpertsWide || K % 64 || Npad % 256 || n_store % 64 || num_cus <= 0 ||
@@ -391,53 +368,33 @@ hipError_t launch_gemm_stream(const bf16_t* A, const WT* B, const float* wscale,
     return hipErrorInvalidValue;
   const int BM = small ? 64 : 256, BN = small ? 128 : 256;
   const int nt = EPI == kEpiGateUp ? Npad / BN : (n_store + BN - 1) / BN;
+  // More than 64 experts: one launch, a group of 64 per grid row (as in
+  // gemm_dma.hip; us of gate/up + down, E = 128, C = 512, H = 256, 16 rows an
+  // expert 28 + 22 -> 25 + 19; E = 256, C = 512, H = 512, 24 rows 91 + 57 -> 81 + 46).
+  const int groups = (E + kMaxExperts - 1) / kMaxExperts;
   // at most this many tiles (an expert with rows has one more than its whole
   // ones at most)
-  const int KT = K / 64;
-  const bool split = partials && small && !save && KT >= kStreamMinSlabs &&
-                     2 * ((long)(rows / BM) + (long)std::min<size_t>(E, rows)) * nt <= num_cus;
-  // More than 64 experts: groups of 64.  Whole tiles: one launch, a group per
-  // grid row (as in gemm_dma.hip; us of gate/up + down, E = 128, C = 512, H = 256,
-  // 16 rows an expert 28 + 22 -> 25 + 19; E = 256, C = 512, H = 512, 24 rows 91 +
-  // 57 -> 81 + 46); split ones: a launch and a reduction each.
-  for (int e0 = 0; e0 < E; e0 += kMaxExperts) {
-    const int groups = split ? 1 : (E + kMaxExperts - 1) / kMaxExperts;
-    const int Eg = split ? std::min(kMaxExperts, E - e0) : E;
-    const long tiles = ((long)(rows / BM) + (long)std::min<size_t>(std::min(E, kMaxExperts), rows)) * nt;
-    float* part = split ? partials : nullptr;
-    // (with split tiles every CU has work, also where there are fewer tiles)
-    const int grid = part ? num_cus : (int)std::min<long>(tiles, num_cus);
-    const WT* Bg = B + (size_t)e0 * Npad * K;
-    const float* sg = wscale ? wscale + (size_t)e0 * Npad : nullptr;
-    const float* b0 = bias0 ? bias0 + (size_t)e0 * bias_ld : nullptr;
-    const float* b1 = bias1 ? bias1 + (size_t)e0 * bias_ld : nullptr;
-    auto launch = [&](auto kernel, int threads) {
-      hipLaunchKernelGGL(kernel, dim3(grid, groups), dim3(threads), 0, stream, A, Bg, sg, b0, b1, counts, Eg, e0,
-                         K, Npad, nt, n_store, bias_ld, out, ldo, part, save, save_ld);
-    };
-    if constexpr (kFp8) {
-      if (small)
-        launch(gemm_stream_kernel<EPI, fp8_t, 4, 64, 128, 8, false>, 256);
+  const long tiles = ((long)(rows / BM) + (long)std::min<size_t>(std::min(E, kMaxExperts), rows)) * nt;
+  const int grid = (int)std::min<long>(tiles, num_cus);
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(grid, groups), dim3(threads), 0, stream, A, B, wscale, bias0, bias1,
+                       counts, E, K, Npad, nt, n_store, bias_ld, out, ldo, save, save_ld);
+  };
+  if constexpr (kFp8) {
+    if (small)
+      launch(gemm_stream_kernel<EPI, fp8_t, 4, 64, 128, 8, false>, 256);
+    else
+      launch(gemm_stream_kernel<EPI, fp8_t, 8, 256, 256, 3, false>, 512);
+  } else {
+    if (!small) return hipErrorInvalidValue;   // gemm_dma.hip's
+    if constexpr (EPI == kEpiGateUp) {
+      if (save)
+        launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, true>, 256);
       else
-        launch(gemm_stream_kernel<EPI, fp8_t, 8, 256, 256, 3, false>, 512);
-    } else {
-      if (!small) return hipErrorInvalidValue;   // gemm_dma.hip's
-      if constexpr (EPI == kEpiGateUp) {
-        if (save)
-          launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, true>, 256);
-        else
-          launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, false>, 256);
-      } else {
         launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, false>, 256);
-      }
+    } else {
+      launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, false>, 256);
     }
-    if constexpr (EPI != kEpiSwigluBwd) {
-      if (part)
-        hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI, Waves<4, 64, 128>>), dim3(2 * grid), dim3(256),
-                           0, stream, part, sg, b0, b1, counts, Eg, e0, K, Npad, nt, n_store, bias_ld,
-                           out, ldo, grid, kStreamMinSlabs);
-    }
-    if (!split) break;
   }
   return hipGetLastError();
 }
@@ -445,7 +402,7 @@ hipError_t launch_gemm_stream(const bf16_t* A, const WT* B, const float* wscale,
 #define MGPT_INST_STREAM(EPI, WT)                                                                   \
   template hipError_t launch_gemm_stream<EPI, WT>(                                                  \
       const bf16_t*, const WT*, const float*, const float*, const float*, const int32_t*, int, int, \
-      int, int, int, bf16_t*, int, size_t, bool, float*, int, bf16_t*, int, hipStream_t);
+      int, int, int, bf16_t*, int, size_t, bool, int, bf16_t*, int, hipStream_t);
 MGPT_INST_STREAM(kEpiGateUp, bf16_t)
 MGPT_INST_STREAM(kEpiDown, bf16_t)
 MGPT_INST_STREAM(kEpiSwigluBwd, bf16_t)

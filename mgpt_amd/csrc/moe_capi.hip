@@ -59,7 +59,7 @@ hipError_t launch_pack_transpose(const float*, int, int, float*, int, int, int, 
 template <int EPI, typename WT>
 hipError_t launch_gemm_stream(const bf16_t*, const WT*, const float*, const float*, const float*,
                               const int32_t*, int, int, int, int, int, bf16_t*, int, size_t, bool,
-                              float*, int, bf16_t*, int, hipStream_t);
+                              int, bf16_t*, int, hipStream_t);
 template <int EPI>
 hipError_t launch_gemm_f32(const float*, const float*, const float*, const float*, const int32_t*,
                            int, int, int, int, int, float*, int, size_t, float*, int, int,
@@ -145,7 +145,6 @@ namespace {
 
 constexpr size_t kAlign = 256;
 constexpr size_t kGemmPartialBytes = 512 * 128 * 4;   // one 256x256 fp32 tile
-constexpr size_t kStreamPartialBytes = 64 * 128 * 4;   // one 64x128 fp32 tile
 constexpr int kRowPad = 256;   // rows of slack after activation buffers (GEMM tile overrun)
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -315,9 +314,7 @@ struct mgpt_moe {
   bool fp8_decode(int N) const { return wgu_t && !wide() && (size_t)N * k < (size_t)64 * E; }
   size_t w_bytes() const { return wdt == MGPT_DTYPE_FP8_E4M3 ? 1 : (wdt == MGPT_DTYPE_BF16 ? 2 : 4); }
   // h (SwiGLU output) is kept in the activation dtype.
-  // stream_part: with the weight-streaming GEMMs' partial tiles (bf16 weights,
-  // few rows per expert; those GEMMs also run without)
-  Layout layout(int N, bool train = false, bool stream_part = true) const {
+  Layout layout(int N, bool train = false) const {
     Layout L{};
     const size_t A = (size_t)N * k;
     const size_t TB = router_tokens_per_block(E);
@@ -343,10 +340,7 @@ struct mgpt_moe {
     L.hbuf = take((A + kRowPad) * Hp * act_bytes());
     L.obuf = take((A + kRowPad) * C * act_bytes());
     // fp32 partial tiles of the large-M GEMMs' split last round (one per CU)
-    // (one 64-row tile per CU for the weight-streaming ones)
-    L.partials = take(uses_gemm_dma(N) ? (size_t)num_cus * kGemmPartialBytes
-                      : wdt == MGPT_DTYPE_BF16 && stream_part ? (size_t)num_cus * kStreamPartialBytes
-                                                              : 0);
+    L.partials = take(uses_gemm_dma(N) ? (size_t)num_cus * kGemmPartialBytes : 0);
     L.rstd = take((size_t)N * 4);
     const size_t pad_rows = padded() ? (size_t)N * C * io_bytes() : 0;
     L.xpad = take(pad_rows);
@@ -801,9 +795,9 @@ struct BlockArgs {
 
 // IoT: the caller's x and y; ActT: the gathered rows, h and expert outputs.
 template <typename IoT, typename ActT>
-int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train, bool stream_part,
+int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
                  hipStream_t st, BlockArgs blk = BlockArgs()) {
-  const Layout L = h->layout(N, train, stream_part);
+  const Layout L = h->layout(N, train);
   const int C = h->C, Cx = h->Cx, E = h->E, k = h->k, Hp = h->Hp, Cp = h->Cp;
   const size_t A = (size_t)N * k;
   int32_t* idx = (int32_t*)(ws + L.topk_idx);
@@ -905,21 +899,20 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
       // hold (width, more than 64 experts) and rows are few
       HIP_TRY((launch_gemm_stream<kEpiGateUp, fp8_t>(
           xg, (const fp8_t*)h->wgu, h->sgu, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, A,
-          A < (size_t)32 * E, nullptr, h->num_cus, nullptr, 0, st)));
+          A < (size_t)32 * E, h->num_cus, nullptr, 0, st)));
       HIP_TRY(mark(3));
       HIP_TRY((launch_gemm_stream<kEpiDown, fp8_t>(hb, (const fp8_t*)h->wd, h->sd, h->bd, nullptr,
                                                    counts, E, Hp, Cp, C, Cp, ob, C, A,
-                                                   A < (size_t)32 * E || narrow_down, nullptr, h->num_cus,
+                                                   A < (size_t)32 * E || narrow_down, h->num_cus,
                                                    nullptr, 0, st)));
     } else if (few) {
       // few rows per expert: the weights are the larger operand
-      float* sp = stream_part ? part : nullptr;
       HIP_TRY((launch_gemm_stream<kEpiGateUp, bf16_t>(
           xg, (const bf16_t*)h->wgu, nullptr, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, A,
-          true, sp, h->num_cus, (bf16_t*)gu, 2 * Hp, st)));
+          true, h->num_cus, (bf16_t*)gu, 2 * Hp, st)));
       HIP_TRY(mark(3));
       HIP_TRY((launch_gemm_stream<kEpiDown, bf16_t>(hb, (const bf16_t*)h->wd, nullptr, h->bd, nullptr,
-                                                    counts, E, Hp, Cp, C, Cp, ob, C, A, true, sp,
+                                                    counts, E, Hp, Cp, C, Cp, ob, C, A, true,
                                                     h->num_cus, nullptr, 0, st)));
     } else if (h->gemm_tile == 256) {
       // bf16 weights, prefill-shaped segments: 256x256 direct-to-LDS kernel.
@@ -933,7 +926,7 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
       HIP_TRY(mark(3));
       if (narrow_down)
         HIP_TRY((launch_gemm_stream<kEpiDown, bf16_t>(hb, (const bf16_t*)h->wd, nullptr, h->bd, nullptr,
-                                                      counts, E, Hp, Cp, C, Cp, ob, C, A, true, part,
+                                                      counts, E, Hp, Cp, C, Cp, ob, C, A, true,
                                                       h->num_cus, nullptr, 0, st)));
       else
         HIP_TRY(launch_gemm_dma<kEpiDown>(hb, (const bf16_t*)h->wd, h->bd, nullptr, counts, E, Hp,
@@ -1112,11 +1105,11 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
   } else if (small_m(h, N)) {
     HIP_TRY((launch_gemm_stream<kEpiSwigluBwd, bf16_t>(
         (const bf16_t*)dgo, (const bf16_t*)wdb, nullptr, nullptr, nullptr, counts, E, C, h->Hq, Hp, 0,
-        (bf16_t*)gu, 2 * Hp, A, true, nullptr, h->num_cus, (bf16_t*)gu, 2 * Hp, st)));
+        (bf16_t*)gu, 2 * Hp, A, true, h->num_cus, (bf16_t*)gu, 2 * Hp, st)));
     HIP_TRY(mark(2));
     HIP_TRY((launch_gemm_stream<kEpiDown, bf16_t>(
         (const bf16_t*)gu, (const bf16_t*)wgub, nullptr, nullptr, nullptr, counts, E, 2 * Hp, Cp, C, 0,
-        (bf16_t*)ob, C, A, true, (float*)(ws + L.partials), h->num_cus, nullptr, 0, st)));
+        (bf16_t*)ob, C, A, true, h->num_cus, nullptr, 0, st)));
   } else {
     const int mt = (A + 127) / 128 + E;
     HIP_TRY((launch_grouped_gemm<128, 128, 2, 2, kEpiSwigluBwd>(
@@ -1148,18 +1141,17 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
 
 // The forward for the handle's (boundary, compute) dtype pair.
 int dispatch_forward(mgpt_moe* h, const void* x, void* y, int N, char* ws, bool train,
-                     hipStream_t st, BlockArgs blk, bool stream_part = true) {
+                     hipStream_t st, BlockArgs blk) {
   if (h->act == MGPT_DTYPE_F32)
-    return forward_impl<float, float>(h, (const float*)x, (float*)y, N, ws, train, stream_part, st, blk);
+    return forward_impl<float, float>(h, (const float*)x, (float*)y, N, ws, train, st, blk);
   if (h->io == MGPT_DTYPE_F32)
-    return forward_impl<float, bf16_t>(h, (const float*)x, (float*)y, N, ws, train, stream_part, st, blk);
-  return forward_impl<bf16_t, bf16_t>(h, (const bf16_t*)x, (bf16_t*)y, N, ws, train, stream_part, st, blk);
+    return forward_impl<float, bf16_t>(h, (const float*)x, (float*)y, N, ws, train, st, blk);
+  return forward_impl<bf16_t, bf16_t>(h, (const bf16_t*)x, (bf16_t*)y, N, ws, train, st, blk);
 }
 
 // Shared argument checks of the forward entry points.
 int check_forward_args(const mgpt_moe* h, const void* x, const void* y, int num_tokens,
-                       const void* workspace, size_t workspace_bytes, bool train,
-                       bool stream_part = true) {
+                       const void* workspace, size_t workspace_bytes, bool train) {
   if (!h) return fail(MGPT_ERR_INVALID_ARGUMENT, "null handle");
   if (!h->loaded) return fail(MGPT_ERR_NOT_READY, "parameters not loaded");
   if (num_tokens < 0) return fail(MGPT_ERR_INVALID_ARGUMENT, "negative num_tokens");
@@ -1169,7 +1161,7 @@ int check_forward_args(const mgpt_moe* h, const void* x, const void* y, int num_
     return fail(MGPT_ERR_INVALID_ARGUMENT, "x and y must be 16-byte aligned");
   if ((uintptr_t)workspace % kAlign != 0)
     return fail(MGPT_ERR_INVALID_ARGUMENT, "workspace must be %zu-byte aligned", kAlign);
-  const size_t need = h->layout(num_tokens, train, stream_part).total;
+  const size_t need = h->layout(num_tokens, train).total;
   if (workspace_bytes < need)
     return fail(MGPT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu bytes < required %zu",
                 workspace_bytes, need);
@@ -1233,10 +1225,7 @@ int mgpt_moe_forward(mgpt_moe* h, const void* x, void* y, int num_tokens, void* 
 int mgpt_moe_forward_noalloc(mgpt_moe* h, const void* x, void* y, int num_tokens, void* stream) {
   if (!h) return fail(MGPT_ERR_INVALID_ARGUMENT, "null handle");
   if (num_tokens < 0) return fail(MGPT_ERR_INVALID_ARGUMENT, "negative num_tokens");
-  // the weight-streaming GEMMs' partial tiles only where the scratch has room
-  // for them too
-  const bool stream_part = h->layout(num_tokens).total <= (size_t)MGPT_MOE_NOALLOC_SCRATCH_BYTES;
-  const size_t need = h->layout(num_tokens, false, stream_part).total;
+  const size_t need = h->layout(num_tokens).total;
   if (need > (size_t)MGPT_MOE_NOALLOC_SCRATCH_BYTES)
     return fail(MGPT_ERR_WORKSPACE_TOO_SMALL,
                 "%d tokens need %zu workspace bytes; the built-in scratch holds %zu "
@@ -1244,13 +1233,12 @@ int mgpt_moe_forward_noalloc(mgpt_moe* h, const void* x, void* y, int num_tokens
                 num_tokens, need, (size_t)MGPT_MOE_NOALLOC_SCRATCH_BYTES);
   void* ws = nullptr;
   if (int rc = scratch_address(h->device, &ws)) return rc;
-  if (int rc = check_forward_args(h, x, y, num_tokens, ws, MGPT_MOE_NOALLOC_SCRATCH_BYTES, false,
-                                  stream_part))
+  if (int rc = check_forward_args(h, x, y, num_tokens, ws, MGPT_MOE_NOALLOC_SCRATCH_BYTES, false))
     return rc;
   if (num_tokens == 0) return MGPT_OK;
   HIP_TRY(hipSetDevice(h->device));
   return dispatch_forward(h, x, y, num_tokens, (char*)ws, false, (hipStream_t)stream,
-                          BlockArgs(), stream_part);
+                          BlockArgs());
 }
 
 int mgpt_moe_forward_block(mgpt_moe* h, const void* x, const float* gamma, float eps, void* out,

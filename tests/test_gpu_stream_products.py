@@ -2,11 +2,11 @@
 they take: bf16 weights under 64 rows per expert (and narrow down products
 above), fp8 weights outside the decode kernel's range.  Segments that end
 inside, at and one past a 64- or 256-row tile, one token, contractions of one
-slab and of enough slabs to be split along K, widths that are not a multiple of
-128, more experts than a launch takes, and training through the 64-row tiles.
-Against the oracle at the layer's bars (bf16 2e-2, fp8 6e-2 of the fp32 path,
-which rounds the rows and products in between), and against the same rows one
-token at a time, which other tiles and splits compute, at a few bf16 roundings.
+slab and of 64, widths that are not a multiple of 128, more experts than a wave
+has lanes, and training through the 64-row tiles.  Against the oracle at the
+layer's bars (bf16 2e-2, fp8 6e-2 of the fp32 path, which rounds the rows and
+products in between), against the same rows one token at a time, which other
+tiles compute, at a few bf16 roundings, and bit for bit against the 128 x 128 tiles.
 """
 import numpy as np
 import pytest
@@ -26,7 +26,7 @@ SHAPES = [
     (255, 128, 1, 1, 128, "fp8"), (257, 128, 1, 1, 192, "fp8"), (300, 192, 3, 2, 160, "fp8"),
     (40, 192, 3, 2, 160, "fp8"), (600, 256, 8, 3, 1408, "fp8"), (260, 128, 80, 3, 96, "fp8"),
     (9, 128, 70, 2, 96, "fp8"),
-    # groups of 64 experts as rows of one grid: split and whole tiles, 256-row tiles
+    # groups of 64 experts as rows of one grid: 64- and 256-row tiles
     (2, 64, 130, 2, 2112, "bf16"), (700, 64, 130, 1, 64, "bf16"), (2400, 64, 70, 2, 96, "bf16"),
     (4300, 128, 130, 2, 64, "bf16"), (2500, 128, 70, 2, 96, "fp8"),
 ]
@@ -95,7 +95,7 @@ def test_gate_times_up_past_the_range(N, C, E, k, H, weights):
 
 # every expert gets rows in both calls: few rows (64 x 128 tiles; fp8 from 32 rows an
 # expert on 256 x 256 ones) against at least 64 an expert in 128 x 128 tiles
-@pytest.mark.parametrize("N,C,E,k,H,weights", [(40, 192, 4, 2, 160, "bf16"),
+@pytest.mark.parametrize("N,C,E,k,H,weights", [(40, 192, 4, 2, 160, "bf16"), (24, 1024, 16, 2, 2816, "bf16"),
                                                (40, 192, 4, 2, 160, "fp8"), (300, 192, 4, 2, 160, "fp8"),
                                                (400, 512, 8, 3, 704, "fp8")])
 def test_same_bits_as_the_128_row_tiles(N, C, E, k, H, weights, monkeypatch):
