@@ -62,33 +62,33 @@ __device__ __forceinline__ bf16x8 fp8x8_to_bf16x8(uint32_t lo, uint32_t hi) {
 
 // acc = acc * scale + bias, per output feature (register v of a 32x32 tile
 // holds feature 8*(v/4) + 4*lhalf + v%4 of the tile, a token per lane);
-// scale null: 1, bias null: none.
+// scale null: 1, bias null: none.  An array's 32 values are requested at once (8
+// at a time in the 256-row tiles, which run at the register limit).
 template <typename W>
 __device__ __forceinline__ void affine(f32x16 (&acc)[W::TN][W::TM], int j, const float* scale,
                                        const float* bias, int lhalf) {
+  constexpr int kBatch = W::TM >= 4 ? 8 : 32;
+  auto each = [&](const float* p, int f0, auto op) __attribute__((always_inline)) {
+    typedef const __attribute__((address_space(4))) float* cptr;   // scalar loads
+    const cptr u = (cptr)(uintptr_t)(p + f0);
+    float t[kBatch];
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
+    for (int f = 0; f < kBatch; ++f) t[f] = u[f];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int f = 8 * g + q;
-      float s = 1.0f, b = 0.0f;
-      if (scale) {
-        const float s0 = uniform_load(scale + f), s1 = uniform_load(scale + f + 4);
-        s = lhalf ? s1 : s0;
-      }
-      if (bias) {
-        const float b0 = uniform_load(bias + f), b1 = uniform_load(bias + f + 4);
-        b = lhalf ? b1 : b0;
-      }
+    for (int f = 0; f < kBatch; ++f) {
+      if (f & 4) continue;   // the other half's
+      const int v = (f0 + f) / 8 * 4 + f % 4;
+      const float x = lhalf ? t[f + 4] : t[f];
 #pragma unroll
-      for (int i = 0; i < W::TM; ++i) {
-        float a = acc[j][i][4 * g + q];
-        if (scale) a = a * s;
-        acc[j][i][4 * g + q] = a + b;
-      }
-      // one feature at a time (keeps the scalar loads from piling up)
-      if (q & 1) __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < W::TM; ++i) acc[j][i][v] = op(acc[j][i][v], x);
     }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int f0 = 0; f0 < 32; f0 += kBatch) {
+    if (scale) each(scale, f0, [](float a, float x) { return a * x; });
+    if (bias) each(bias, f0, [](float a, float x) { return a + x; });
+  }
 }
 
 template <int EPI, typename WT, int NW, int BM, int BN, int ST, bool kSave>
