@@ -6,15 +6,19 @@
 // Same contract as gemm_dma.hip (A = expert-contiguous bf16 rows [rows][K],
 // B = packed weights [E][Npad][K], bf16 or e4m3 with per-output-channel
 // scales; gate/up, down and SwiGLU-backward epilogues) and the same frame:
-// a persistent block per CU walks BM x BN tiles in an order that shares
-// operand panels within an XCD, operands go HBM -> LDS by untracked
+// a persistent block per CU (two of 64-row tiles) walks BM x BN tiles in an order
+// that shares operand panels within an XCD, operands go HBM -> LDS by untracked
 // 1 KB loads, waves of 64 features x BM/2 tokens run
 // v_mfma_f32_32x32x16_bf16 on D = W . X^T.  What differs:
 //  * The ring holds ST stages, each a whole 64-column slab (BM rows of A, BN
 //    rows of B), ST - 1 slabs ahead.  With fp8 weights a slab is 48 KB (BM =
 //    256) instead of 64 KB, so both operands lead by two slabs in 144 KB; the
-//    64 x 128 tiles take 24 KB (bf16) or 16 KB (fp8) a slab, with 112 to 120 KB
-//    of loads in flight a CU, which a weight stream from HBM needs.
+//    64 x 128 tiles take 24 KB (bf16) or 16 KB (fp8) a slab and a ring of 72 or
+//    80 KB, so that two blocks share a CU: one's start, epilogue and last slabs
+//    are covered by the other's stream, with 96 to 128 KB of loads in flight a CU.
+//    (One block with twice the ring, us of the forward: 96 experts of C = H = 512,
+//    48 tokens, bf16 65 / 50 with two; 512 experts, 71 tokens, k = 6, H = 1376, fp8
+//    400 / 266; the 24-token step below 64 / 61; no shape slower.)
 //  * A k-step ks contracts columns 16ks .. 16ks+15 of the slab, lane half h
 //    columns 16ks + 8h .. +7, as in the other bf16 products (the same sums, bit
 //    for bit); the packed fp8 rows keep a lane's weights of two k-steps in one
@@ -27,14 +31,13 @@
 //    evenly a step's few tiles spread over the CUs (16 experts of H = 2816:
 //    704 gate/up tiles are 2.75 rounds, 352 of 256 columns 1.4, paid as 2).
 //
-// Measured on MI355X, stage times with cold weights, against the register-staged
-// 32 x 256 (bf16) and 128 x 128 (fp8) tiles used before, gate/up + down us:
-// bf16, C = 1024, H = 2816, E = 16, k = 2: 1 token 33 + 38 -> 14 + 15, 24
-// tokens 51 + 62 -> 43 + 27, 300 tokens 80 + 65 -> 46 + 34; C = 2048, H = 1408,
-// E = 64, k = 8 (1.1 GB of weights): 64 tokens 201 + 110 -> 164 + 75 (4.6 TB/s),
-// 400 tokens 310 + 193 -> 175 + 86.  fp8, the latter layer: 600 tokens 209 + 142
-// -> 128 + 73, 1999 tokens 356 + 236 -> 220 + 136 (840 TFLOP/s in gate/up),
-// 4096 tokens 585 + 389 -> 382 + 229.
+// Measured on MI355X, stage times, against the register-staged 32 x 256 (bf16, fp8) and
+// 128 x 128 (fp8) tiles used before, gate/up + down us: bf16, C = 1024, H = 2816, E =
+// 16, k = 2: 1 token 33 + 38 -> 12 + 19, 24 tokens 47 + 60 -> 34 + 26, 300 tokens 67 +
+// 61 -> 36 + 28; C = 2048, H = 1408, E = 64, k = 8 (1.1 GB of weights): 64 tokens 190 +
+// 107 -> 160 + 67 (4.9 TB/s), 400 tokens 305 + 196 -> 175 + 82.  fp8, the latter layer:
+// 600 tokens 202 + 138 -> 117 + 64, 1999 tokens 345 + 226 -> 194 + 114 (950 TFLOP/s in
+// gate/up), 4096 tokens 555 + 390 -> 343 + 216.
 #include <type_traits>
 
 #include "gemm_ring.hpp"
@@ -108,8 +111,18 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
   __shared__ __attribute__((aligned(1024))) char smem[ST * kStage];
 
   const int G = gridDim.x;
-  int t = (G % kNumXcd == 0) ? (blockIdx.x % kNumXcd) * (G / kNumXcd) + blockIdx.x / kNumXcd
-                             : blockIdx.x;
+  // Which tiles an XCD (own L2) takes.  256-row tiles: contiguous runs, which share
+  // operand panels.  64-row tiles share little beyond the (at most four) m-tiles of a
+  // weight panel and are often fewer than the blocks, so runs of four tiles are dealt
+  // to the XCDs in turn, which leaves none of them idle.
+  constexpr int kRun = 4;
+  const int xcd = blockIdx.x % kNumXcd, in_xcd = blockIdx.x / kNumXcd;
+  int t = blockIdx.x;
+  if (BM > 64) {
+    if (G % kNumXcd == 0) t = xcd * (G / kNumXcd) + in_xcd;
+  } else if (G % (kRun * kNumXcd) == 0) {
+    t = (in_xcd / kRun * kNumXcd + xcd) * kRun + in_xcd % kRun;
+  }
   const int KT = K / 64;
   int e_base = 0;
   if (gridDim.y > 1) {   // a group of 64 experts per grid row
@@ -350,7 +363,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
 
 }  // namespace
 
-// Persistent launch, one block per CU.  Tiles of 64 rows x 128 features
+// Persistent launch, one block per CU (two of the small tiles).  Tiles of 64 rows x 128 features
 // (small) or 256 x 256.  save: the training pre-activations (gate/up: written;
 // SwiGLU backward: read, bf16 weights only).  K % 64 == 0, Npad % 256 == 0,
 // n_store % 64 == 0; A has 256 rows of slack.
@@ -369,31 +382,32 @@ hipError_t launch_gemm_stream(const bf16_t* A, const WT* B, const float* wscale,
   const int BM = small ? 64 : 256, BN = small ? 128 : 256;
   const int nt = EPI == kEpiGateUp ? Npad / BN : (n_store + BN - 1) / BN;
   // More than 64 experts: one launch, a group of 64 per grid row (as in
-  // gemm_dma.hip; us of gate/up + down, E = 128, C = 512, H = 256, 16 rows an
-  // expert 28 + 22 -> 25 + 19; E = 256, C = 512, H = 512, 24 rows 91 + 57 -> 81 + 46).
+  // gemm_dma.hip; us of gate/up + down, E = 128, C = 512, H = 256, 16 rows an expert 16 +
+  // 11, E = 256, C = 512, H = 512, 24 rows 63 + 34; with a launch a group and one block a
+  // CU 28 + 22 and 91 + 57).
   const int groups = (E + kMaxExperts - 1) / kMaxExperts;
   // at most this many tiles (an expert with rows has one more than its whole
   // ones at most)
   const long tiles = ((long)(rows / BM) + (long)std::min<size_t>(std::min(E, kMaxExperts), rows)) * nt;
-  const int grid = (int)std::min<long>(tiles, num_cus);
+  const int grid = (int)std::min<long>((tiles + 31) / 32 * 32, small ? 2 * num_cus : num_cus);
   auto launch = [&](auto kernel, int threads) {
     hipLaunchKernelGGL(kernel, dim3(grid, groups), dim3(threads), 0, stream, A, B, wscale, bias0, bias1,
                        counts, E, K, Npad, nt, n_store, bias_ld, out, ldo, save, save_ld);
   };
   if constexpr (kFp8) {
     if (small)
-      launch(gemm_stream_kernel<EPI, fp8_t, 4, 64, 128, 8, false>, 256);
+      launch(gemm_stream_kernel<EPI, fp8_t, 4, 64, 128, 5, false>, 256);
     else
       launch(gemm_stream_kernel<EPI, fp8_t, 8, 256, 256, 3, false>, 512);
   } else {
     if (!small) return hipErrorInvalidValue;   // gemm_dma.hip's
     if constexpr (EPI == kEpiGateUp) {
       if (save)
-        launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, true>, 256);
+        launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 3, true>, 256);
       else
-        launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, false>, 256);
+        launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 3, false>, 256);
     } else {
-      launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 6, false>, 256);
+      launch(gemm_stream_kernel<EPI, bf16_t, 4, 64, 128, 3, false>, 256);
     }
   }
   return hipGetLastError();
