@@ -4,11 +4,11 @@
 // about 8 rows per expert) make the expert GEMMs a weight stream: every
 // weight byte is used by at most 32 rows, so the bound is HBM bandwidth,
 // not MFMA.  This kernel is built for that bound:
-//  * Work items are (expert m-tile of <= 32 rows, 64 or 128 output features);
-//    two persistent blocks per CU walk them, so that one block's start, epilogue
-//    and waits are covered by the other's stream, each with a direct-to-LDS ring
-//    across item boundaries (a stage: 64 or 128 weight rows x 128 fp8 columns
-//    and 32 activation rows x 128 columns).  The loads are inline asm the
+//  * Work items are (expert m-tile of <= 32 rows, 64, 128 or 256 output features);
+//    two persistent blocks per CU (one of 256 features) walk them, so that one
+//    block's start, epilogue and waits are covered by the other's stream, each
+//    with a direct-to-LDS ring across item boundaries (a stage: the item's weight
+//    rows x 128 fp8 columns and 32 activation rows x 128 columns).  The loads are inline asm the
 //    compiler does not track, with explicit waits (as in gemm_dma.hip); a lane's
 //    addresses are formed once an item and stepped by additions.
 //  * Each wave owns 64 features (a [32 gate | 32 up] pair for gate/up) x the 32
@@ -29,6 +29,7 @@
 // [E][Npad/256][K/128][256][128] (pack.hip: tile_fp8_kernel) with scales
 // [E][Npad], SwiGLU or bias epilogue).
 #include <algorithm>
+#include <cmath>
 
 #include "common.hpp"
 
@@ -38,7 +39,7 @@ namespace {
 constexpr int kDBM = 32;                     // token rows per item
 constexpr int kDBK = 128;                    // columns per stage
 constexpr int kTileN = 256;                  // features per tile of the weights' layout
-constexpr int kBlocksPerCu = 2;
+constexpr int blocks_per_cu(int nw) { return nw == 4 ? 1 : 2; }   // nw waves a block
 constexpr int kDmaW = 64 * kDBK / 1024;      // 8 weight blocks per wave (64 features) and stage
 
 typedef __attribute__((address_space(3))) char lds_char;
@@ -123,10 +124,21 @@ struct DScan {
     const unsigned long long m = __ballot(mine);
     const int owner = __builtin_amdgcn_readfirstlane(__ffsll((long long)m) - 1);
     out->expert = owner;
-    out->row0 = __builtin_amdgcn_readlane(rows_incl - cnt, owner) +
-                (mt - __builtin_amdgcn_readlane(tiles_excl, owner)) * kDBM;
+    // The expert's T x nbx items in runs of eight feature blocks, row tiles next: the
+    // hardware deals blocks round-robin to the eight XCDs (each with its own L2), so
+    // the T items that read the same weights run on one XCD at about the same time.
+    const int T = __builtin_amdgcn_readlane(tiles_incl - tiles_excl, owner);
+    const int u = v - __builtin_amdgcn_readlane(tiles_excl, owner) * nbx;
+    int tile = 0, n = u;
+    if (T > 1) {
+      const int run = u / (kNumXcd * T), left = u - run * (kNumXcd * T);
+      const int g = min(kNumXcd, nbx - run * kNumXcd);
+      tile = left / g;
+      n = run * kNumXcd + left - tile * g;
+    }
+    out->row0 = __builtin_amdgcn_readlane(rows_incl - cnt, owner) + tile * kDBM;
     out->row_end = __builtin_amdgcn_readlane(rows_incl, owner);
-    out->n0 = (v - mt * nbx) * bn;
+    out->n0 = n * bn;
     return true;
   }
 };
@@ -227,7 +239,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_decode_kernel(
   constexpr int kChunks = kRowB / 16;          // 16-byte chunks per row
   static_assert(kXS == 2 || kXS == 4, "bf16 or fp32 rows");
   // ring depth: what LDS holds and the wait counter can count (63 loads)
-  constexpr int kLds = (160 * 1024 / kBlocksPerCu - (GATHER ? kGatherFlat * 4 + 1024 : 0)) / kStage;
+  constexpr int kLds = (160 * 1024 / blocks_per_cu(NW) - (GATHER ? kGatherFlat * 4 + 1024 : 0)) / kStage;
   constexpr int kCnt = 63 / kDm + 2;
   constexpr int kDStages = kLds < kCnt ? kLds : kCnt;
   static_assert(kDStages >= 2, "ring depth");
@@ -464,7 +476,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_decode_kernel(
   }
 }
 
-// Persistent launch, two blocks per CU.  Requires K % 128 == 0, Npad % 256 ==
+// Persistent launch.  Requires K % 128 == 0, Npad % 256 ==
 // 0 and n_store % 64 == 0; rows: all rows of the E segments.
 template <int EPI, bool GATHER, typename XT>
 hipError_t launch_decode(const XT* A, const fp8_t* B, const float* wscale, const float* bias0,
@@ -481,23 +493,38 @@ hipError_t launch_decode(const XT* A, const fp8_t* B, const float* wscale, const
     if (e == hipSuccess) e = hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e != hipSuccess || num_cus <= 0) num_cus = 256;
   }
-  // An item of 64 features (one wave) where those give no CU more than one,
-  // else of 128 (two waves); E or fewer tiles of rows is the estimate while they
-  // average 16 rows.  us on MI355X for 256 features and one block a CU / 128 /
-  // 64: down, E = 64, C = 2048, H = 1408, 1 token 15.2 / 12.0 / 10.8 (256 items
-  // of 64), 64 tokens 36.9 / 36.0 / 40.1 (2048); E = 16, C = 1024, H = 2816, 37
-  // tokens 23.3 / 19.8 / 16.3 (256); gate/up of the former, 1 token 20.1 / 16.6 /
-  // 17.4 (352), 64 tokens 67.1 / 66.8 / 79.6 (2816).
+  // An item of 64 features (one wave) where those give no CU more than one.  us on
+  // MI355X for 256 features and one block a CU / 128 / 64: down, E = 64, C = 2048, H =
+  // 1408, 1 token 15.2 / 12.0 / 10.8 (256 items of 64), 64 tokens 36.9 / 36.0 / 40.1
+  // (2048); E = 16, C = 1024, H = 2816, 37 tokens 23.3 / 19.8 / 16.3 (256); gate/up of the
+  // former, 1 token 20.1 / 16.6 / 17.4 (352), 64 tokens 67.1 / 66.8 / 79.6 (2816).
   const long est = (long)rows <= 16L * E ? std::min<long>(E, rows) : rows / 32 + E;
   const bool narrow = est * ((n_store + 63) / 64) <= num_cus;
+  // Else 128 features.  fp32 rows leave two blocks' rings two stages each, so they
+  // take 256 features and one block a CU where those fill one round of the CUs by more
+  // than half, or a last round, by the experts to expect under an even routing (and
+  // one and a half standard deviations more).  us of gate/up for 256 / 128: E = 32, C
+  // = 2048, H = 1024, k = 8: 1 token (a quarter of a round) 24 / 20, 4 (0.65) 26 / 29, 40
+  // (1) 28 / 31; E = 16, C = 1024, H = 2816, k = 2: 10 (1.03) 29 / 26, 37 (1.4) 28 / 28;
+  // E = 64, C = 2048, H = 1408, k = 8: 40 (2.75) 67 / 77.
+  bool wide = false;
+  if (sizeof(XT) == 4) {
+    const double per_tile = (double)((n_store + 255) / 256) / num_cus;   // rounds
+    const double p = 1.0 - std::exp(-(double)rows / E);
+    const double rounds = E * p * per_tile;
+    const double most = std::ceil(std::min((double)E, E * p + 1.5 * std::sqrt(E * p * (1.0 - p))) * per_tile);
+    wide = most < 1.33 * rounds || (most == 1.0 && rounds > 0.5);
+  }
   auto launch = [&](auto kernel, int NW) {
     const long items = (long)(rows / 32 + std::min(E, rows)) * ((n_store + 64 * NW - 1) / (64 * NW));
-    hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<long>(items, kBlocksPerCu * num_cus)), dim3(64 * NW),
-                       0, stream, A, B, wscale, bias0, bias1, counts, E, K, Npad, n_store, bias_ld, out,
-                       ldo, topk_idx, rows, k, counts_out, perm, slot_of);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<long>(items, blocks_per_cu(NW) * num_cus)),
+                       dim3(64 * NW), 0, stream, A, B, wscale, bias0, bias1, counts, E, K, Npad, n_store,
+                       bias_ld, out, ldo, topk_idx, rows, k, counts_out, perm, slot_of);
   };
   if (narrow)
     launch(gemm_decode_kernel<EPI, GATHER, XT, 1>, 1);
+  else if (wide)
+    launch(gemm_decode_kernel<EPI, GATHER, XT, 4>, 4);
   else
     launch(gemm_decode_kernel<EPI, GATHER, XT, 2>, 2);
   return hipGetLastError();
