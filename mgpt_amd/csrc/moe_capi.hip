@@ -873,13 +873,15 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
   } else {
     const bool fp8 = h->wdt == MGPT_DTYPE_FP8_E4M3;
     const bool few = small_m(h, N);
-    // A down product too narrow for 256 x 256 tiles to reach the CUs goes by
-    // 64 x 128 ones: up to 1.5 of them per CU they are faster (us on MI355X,
-    // bf16, E = 16, C = 1024, H = 2816: 800 tokens 51 -> 34, 1120 (1.6 per CU)
-    // 52 -> 52; E = 8, C = 512, H = 1376: 1040 tokens 33 -> 17; fp8, the
-    // former's 640 tokens: 55 -> 30).
-    const bool narrow_down =
-        2 * (A / 64 + std::min<size_t>(E, A)) * ((C + 127) / 128) <= 3 * (size_t)h->num_cus;
+    // A product too narrow for 256 x 256 tiles to reach the CUs goes by 64 x 128
+    // ones: up to 1.5 of them per CU they are faster (us on MI355X, down,
+    // bf16, E = 16, C = 1024, H = 2816: 800 tokens 51 -> 31, 1120 (1.6 per CU)
+    // 52 -> 50; E = 8, C = 512, H = 1376: 1040 tokens 33 -> 14; fp8, the
+    // former's 640 tokens: 55 -> 22; gate/up, fp8, E = 1, C = 4096, H = 64: 504 tokens
+    // 73 -> 28; H = 1024: 369 tokens 75 -> 29).
+    auto narrow = [&](int cols) {
+      return 2 * (A / 64 + std::min<size_t>(E, A)) * ((cols + 127) / 128) <= 3 * (size_t)h->num_cus;
+    };
     float* part = (float*)(ws + L.partials);
     if (h->fp8_decode(N)) {
       // weight streaming: the persistent direct-to-LDS decode kernel on the
@@ -899,11 +901,11 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
       // hold (width, more than 64 experts) and rows are few
       HIP_TRY((launch_gemm_stream<kEpiGateUp, fp8_t>(
           xg, (const fp8_t*)h->wgu, h->sgu, h->bg, h->bu, counts, E, C, 2 * Hp, 2 * Hp, Hp, hb, Hp, A,
-          A < (size_t)32 * E, h->num_cus, nullptr, 0, st)));
+          A < (size_t)32 * E || narrow(2 * Hp), h->num_cus, nullptr, 0, st)));
       HIP_TRY(mark(3));
       HIP_TRY((launch_gemm_stream<kEpiDown, fp8_t>(hb, (const fp8_t*)h->wd, h->sd, h->bd, nullptr,
                                                    counts, E, Hp, Cp, C, Cp, ob, C, A,
-                                                   A < (size_t)32 * E || narrow_down, h->num_cus,
+                                                   A < (size_t)32 * E || narrow(C), h->num_cus,
                                                    nullptr, 0, st)));
     } else if (few) {
       // few rows per expert: the weights are the larger operand
@@ -924,7 +926,7 @@ int forward_impl(mgpt_moe* h, const IoT* x, IoT* y, int N, char* ws, bool train,
                                           2 * Hp, 2 * Hp, Hp, hb, Hp, mt, nullptr, h->num_cus,
                                           (bf16_t*)gu, 2 * Hp, st));
       HIP_TRY(mark(3));
-      if (narrow_down)
+      if (narrow(C))
         HIP_TRY((launch_gemm_stream<kEpiDown, bf16_t>(hb, (const bf16_t*)h->wd, nullptr, h->bd, nullptr,
                                                       counts, E, Hp, Cp, C, Cp, ob, C, A, true,
                                                       h->num_cus, nullptr, 0, st)));

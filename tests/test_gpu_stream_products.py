@@ -29,6 +29,8 @@ SHAPES = [
     # groups of 64 experts as rows of one grid: 64- and 256-row tiles
     (2, 64, 130, 2, 2112, "bf16"), (700, 64, 130, 1, 64, "bf16"), (2400, 64, 70, 2, 96, "bf16"),
     (4300, 128, 130, 2, 64, "bf16"), (2500, 128, 70, 2, 96, "fp8"),
+    # enough tiles for 256 x 256 fp8 ones in both products, with and without groups
+    (2100, 576, 6, 4, 160, "fp8"), (2400, 576, 70, 4, 160, "fp8"),
 ]
 
 
