@@ -1430,7 +1430,7 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
     };
     if (pairs <= 2048)
       go(router_logits_lane_kernel<ActT, 1>, 1);
-    else if (pairs <= 6144)
+    else if (pairs <= 6144 || (sizeof(ActT) == 4 && eg == 1))
       go(router_logits_lane_kernel<ActT, 2>, 2);
     else
       go(router_logits_lane_kernel<ActT, 4>, 4);
@@ -1506,20 +1506,29 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
   // 1024 tokens at E = 16, C = 256 and about 3500 from C = 1024 on).
   //   E = 8: C = 512 65 tokens 16.9 / 15.2, 2048 20 / 19; C = 1024 1024 28 / 22; C =
   //     2048 2048 43 / 29, 6000 52 / 59
-  const bool many = (long)N * E >= 57344;
-  const float lane_us = 10.0f + N * (0.9e-3f + 3.6e-6f * C);
+  // From fp32 rows an expert per lane takes at most two tokens a wave (9000 tokens,
+  // E = 64, C = 2048: 155 against 189 with four), and product and chain waves, whose
+  // blocks then read twice the bytes, stop earlier (us of fused / here: E = 16, C =
+  // 1024 2500 tokens 37.7 / 32.1, 3000 38.8 / 42.7; C = 2048 2500 62 / 43, 3000 65 / 73;
+  // E = 12, C = 2048 4000 69 / 82; E = 8, C = 1024 3000 33.6 / 31.8, 4000 34.2 / 36.3).
+  // Up to 32 experts over wide bf16 rows, product and chain waves hold until their
+  // blocks are more than four a CU (E = 32, C = 2048, 2000 tokens 46.7 / 49.3 with an expert
+  // per lane, 2400 59 / 52; E = 20 2900 50 / 53, 3400 63 / 55).
+  const bool wide_rows = sizeof(ActT) == 4 || gamma;
+  const bool many = (long)N * E > (E <= 32 && C > 1024 && !wide_rows ? 65536 : 57343);
+  const float lane_us = 10.0f + N * (0.9e-3f + (sizeof(ActT) == 4 ? 4.1e-6f : 3.6e-6f) * C);
   const float fused_us = (10.0f + C * (0.011f + 0.73e-3f * E)) * ((nb + 255) / 256);
   const bool lane = wr4 && many && E > 16 && (N < 4096 || lane_us < fused_us);
   const long NE = (long)N * E;
   const bool pc = E > 16  ? N < 4096
-                  : E > 8 ? C >= 256 && NE < std::min(57344L, 64L * C)
-                          : E > 4 && C >= 512 && NE < 32768;
+                  : E > 8 ? C >= 256 && NE < std::min(wide_rows ? 40960L : 57344L, 64L * C)
+                          : E > 4 && C >= 512 && NE < (wide_rows ? 28672 : 32768);
   const bool mid = logits && (lane || pc);
   // With normalisation those paths run on rows normalised once (xn), where that
   // is faster than the fused kernel or router_logits_kernel, which form the
   // norm in every wave.  MI355X, us of router and permute, before / here:
-  //   E = 8: C = 1024 65 tokens 40 / 25, 1024 43 / 30; C = 512 2048 28 / 26, 3072
-  //     30 / 31
+  //   E = 8: C = 1024 65 tokens 40 / 25, 1024 43 / 30; C = 512 2048 28 / 26, 3000
+  //     29 / 34
   //   E = 16: C = 1024 65 tokens 46 / 26, 2048 50 / 38; C = 2048 2048 86 / 53
   //   E = 20: C = 1024 1024 tokens 51 / 35, 3072 54 / 56; C = 256 2048 26 / 28
   //   E = 32: C = 1024 2048 tokens 53 / 46, 3072 86 / 57, 4096 65 / 61, 6000 68 / 70
@@ -1527,7 +1536,7 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
   //     tokens 86 / 56, 3072 214 / 89, 4096 152 / 93
   // (past 256 blocks router_logits_kernel needs another round).
   const bool norm_mid =
-      mid && (E <= 16    ? NE < 48L * std::min(C, 1024)
+      mid && (E <= 16    ? NE < (E > 8 ? 48L : 40L) * std::min(C, 1024)
               : N < 4096 ? C >= 256 && (nb * ((E + kSplitExperts - 1) / kSplitExperts) > 256 ||
                                         N <= (C >= 512 ? 2048 : 1024))
                          : E * C >= 30000 && N <= (E > 32 ? 6144 : 4096));
