@@ -1184,7 +1184,11 @@ __global__ __launch_bounds__(256) void router_decode_kernel(
     int N, int C, int E, int k, int32_t* __restrict__ topk_idx, float* __restrict__ topk_p,
     float* __restrict__ probs, RowNorm nrm, float* __restrict__ rstd) {
   __shared__ float4 s_x[kDecodeRouterMaxC / 4];          // x[t] widened to fp32
-  __shared__ float4 s_p[3][kMaxExperts * kDrPLD / 4];    // products [e][column]
+  // products [e][column], three steps' worth; before the first step the squares of
+  // the row, over all of it
+  constexpr int kStep = kMaxExperts * kDrPLD / 4;
+  static_assert(3 * kStep >= kDecodeRouterMaxC / 4, "a row of squares");
+  __shared__ float4 s_p[3 * kStep];
   __shared__ __align__(16) float s_row[kMaxExperts];
   __shared__ uint64_t s_tab[32];
   const int tid = threadIdx.x;
@@ -1250,7 +1254,7 @@ __global__ __launch_bounds__(256) void router_decode_kernel(
     if constexpr (NORM) {
       // the squares into the (still unused) product buffers, then every wave
       // adds them up in column order for itself
-      float4* sq = s_p[0];
+      float4* sq = s_p;
 #pragma unroll
       for (int pp = 0; pp < kXP; ++pp) {
         const int c = 8 * tid + 8 * 256 * pp;
@@ -1289,7 +1293,7 @@ __global__ __launch_bounds__(256) void router_decode_kernel(
       constexpr int ahead = (st + kDrPS - 1) % kDrPS;
       load(j + kDrPS - 1, wv[ahead]);
       if (j >= nst) return;
-      float4* prow = s_p[j % 3] + (e * kDrPLD) / 4;
+      float4* prow = s_p + (j % 3) * kStep + (e * kDrPLD) / 4;
       const float4* xs = s_x + (size_t)j * kDrQ;
 #pragma unroll
       for (int q = 0; q < kDrPQ; ++q) {
@@ -1336,7 +1340,7 @@ __global__ __launch_bounds__(256) void router_decode_kernel(
       asm volatile("" : "+v"(v[q].x), "+v"(v[q].y), "+v"(v[q].z), "+v"(v[q].w));
   };
   auto read = [&](int j, float4 (&v)[kPQ]) __attribute__((always_inline)) {
-    const float4* prow = s_p[min(j, nst - 1) % 3] + (e * kDrPLD) / 4;
+    const float4* prow = s_p + (min(j, nst - 1) % 3) * kStep + (e * kDrPLD) / 4;
 #pragma unroll
     for (int q = 0; q < kPQ; ++q) v[q] = prow[q];
   };

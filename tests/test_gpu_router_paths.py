@@ -127,8 +127,9 @@ def test_routing_bit_exact(N, C, E, k, act, train):
 
 # (N, C, E, k, act, H): normalised rows
 NORM_SHAPES = [
-    # one launch, the block's own 1/rms
+    # one launch, the block's own 1/rms (the widest rows: every product buffer holds squares)
     (1, 64, 1, 1, "f32", 8), (64, 1024, 16, 2, "bf16", 8), (33, 4160, 8, 2, "bf16", 8), (64, 192, 64, 8, "f32", 8),
+    (17, 8192, 16, 2, "bf16", 8), (3, 8192, 33, 2, "f32", 8),
     # rows normalised once, on both sides of the lines of its rule
     (65, 1024, 16, 2, "bf16", 8), (2559, 1024, 16, 2, "bf16", 8), (2560, 1024, 16, 2, "bf16", 8),
     (258, 512, 8, 2, "f32", 8), (2559, 512, 8, 2, "bf16", 8), (2560, 512, 8, 2, "bf16", 8),
