@@ -89,7 +89,10 @@ int mgpt_moe_destroy(mgpt_moe* h);
  * parameters are always waited for (they are staged through one device
  * buffer); a re-pack of device parameters is stream-ordered on `stream`,
  * with no allocation and no host wait (a training loop re-packs after every
- * optimizer step). */
+ * optimizer step).  It also rewrites the layouts that backwards read, so it waits
+ * on the device for the handle's last mgpt_moe_backward, on whatever stream that
+ * runs; forwards in flight, and replays of a captured graph that holds a forward or
+ * backward of the handle, must be ordered before it by the caller. */
 int mgpt_moe_load_parameters(mgpt_moe* h, const float* const* params,
                              int num_params, int params_on_device, void* stream);
 

@@ -241,15 +241,20 @@ struct mgpt_moe {
   float* stage_tmp = nullptr;
   bool loaded = false;
   // Backward: the weights in the layouts the data-gradient products read,
-  // derived from the forward packs on the first backward, then written by
-  // every load (bwd_init: an eager backward has filled them, padding included)
-  // (wdb [E][Hq][C]: W_down rows h; wgub [E][Cp][2Hp]: W_gate/W_up rows c,
+  // derived from the forward packs by the first backward after a load, or
+  // written by the load itself (load_writes_bwd) (wdb [E][Hq][C]: W_down rows h; wgub [E][Cp][2Hp]: W_gate/W_up rows c,
   // columns in the packed gate/up order), and the fp32 gradients.
   int Hq = 0;
   void* wdb = nullptr;
   void* wgub = nullptr;
   float* wrt = nullptr;    // W_r as [E][C] (fp32)
-  bool bwd_ready = false, bwd_init = false;
+  bool bwd_ready = false;      // they hold the loaded parameters
+  // What load_writes_bwd goes by: whether an eager backward has ever filled them
+  // (padding included), whether one has run since the last load (bwd_done marks the
+  // end of the last one on its stream), and whether a load was ever captured into a
+  // graph (and a backward: bwd_captured below).
+  bool bwd_filled = false, bwd_used = false, load_captured = false;
+  hipEvent_t bwd_done = nullptr;
   float* grad = nullptr;   // gWr [C][E], gbr [E], gWg [E][C][H], gbg [E][H],
                            // gWu [E][C][H], gbu [E][H], gWd [E][H][C], gbd [E][C]
   size_t g_off[8] = {};
@@ -400,7 +405,7 @@ void free_weights(mgpt_moe* h) {
   h->stage = h->stage_tmp = nullptr;
   h->wgu = h->wd = h->wdb = h->wgub = h->wgu_t = h->wd_t = nullptr;
   h->loaded = false;
-  h->bwd_ready = h->bwd_init = false;
+  h->bwd_ready = h->bwd_filled = h->bwd_used = false;
 }
 
 // Training is built for bf16 x bf16 and fp32 x fp32 handles (fp8 weights
@@ -427,6 +432,7 @@ int ensure_grad(mgpt_moe* h) {
     // fence (cache write-back and invalidate) at each record
     HIP_TRY(hipEventCreateWithFlags(&h->fork_ev, hipEventDisableTiming | hipEventDisableSystemFence));
     HIP_TRY(hipEventCreateWithFlags(&h->join_ev, hipEventDisableTiming | hipEventDisableSystemFence));
+    HIP_TRY(hipEventCreateWithFlags(&h->bwd_done, hipEventDisableTiming | hipEventDisableSystemFence));
   }
   return MGPT_OK;
 }
@@ -442,10 +448,23 @@ int materialize_grad(mgpt_moe* h, hipStream_t st) {
   return MGPT_OK;
 }
 
-// The backward weight layouts, transposed from the forward packs on the
-// first backward of a handle (later loads write them with the packs).
-int ensure_bwd_weights(mgpt_moe* h, hipStream_t st) {
-  if (h->bwd_ready) return MGPT_OK;
+// Whether a load on stream st also writes the backward's layouts: where loads and
+// backwards alternate (the backward is saved a second pass over the weights, and a
+// handle that only infers from then on pays for them once), and where a graph holds
+// a backward, whose replays read them.  The load then waits, on the device, for the
+// last eager backward, which may still be reading them on another stream.
+int load_writes_bwd(mgpt_moe* h, bool capturing, hipStream_t st, bool* writes) {
+  *writes = h->bwd_filled && (h->bwd_captured || (h->bwd_used && !capturing));
+  if (!capturing) h->bwd_used = false;
+  if (*writes && !capturing) HIP_TRY(hipStreamWaitEvent(st, h->bwd_done, 0));
+  return MGPT_OK;
+}
+
+// The backward weight layouts, transposed from the forward packs unless a load
+// or an earlier backward has filled them since (a captured load may be replayed
+// unseen: they are then derived every time).
+int ensure_bwd_weights(mgpt_moe* h, bool capturing, hipStream_t st) {
+  if (h->bwd_ready && !h->load_captured) return MGPT_OK;
   const int C = h->C, E = h->E, Hp = h->Hp, Cp = h->Cp;
   h->Hq = round_up(Hp, 256);
   const size_t eb = h->act_bytes();
@@ -469,12 +488,8 @@ int ensure_bwd_weights(mgpt_moe* h, hipStream_t st) {
     HIP_TRY(launch_transpose_pad<float>((const float*)h->wgu, 2 * Hp, C, (size_t)2 * Hp * C,
                                         (float*)h->wgub, Cp, 2 * Hp, (size_t)Cp * 2 * Hp, E, st));
   }
-  h->bwd_ready = true;
-  // A captured backward fills them only when its graph runs: loads then go on
-  // leaving them to the backward.
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(st, &cap));
-  if (cap == hipStreamCaptureStatusNone) h->bwd_init = true;
+  // (a captured one fills them only when its graph runs)
+  if (!capturing) h->bwd_ready = h->bwd_filled = true;
   return MGPT_OK;
 }
 
@@ -564,6 +579,7 @@ int mgpt_moe_destroy(mgpt_moe* h) {
   if (h->done) (void)hipEventDestroy(h->done);
   if (h->fork_ev) (void)hipEventDestroy(h->fork_ev);
   if (h->join_ev) (void)hipEventDestroy(h->join_ev);
+  if (h->bwd_done) (void)hipEventDestroy(h->bwd_done);
   if (h->side) (void)hipStreamDestroy(h->side);
   delete h;
   return MGPT_OK;
@@ -587,8 +603,8 @@ int mgpt_moe_load_parameters(mgpt_moe* h, const float* const* params, int num_pa
   // The packed buffers depend only on the handle's shape: the first load
   // allocates them (and zeroes the padding the packs never write), later
   // loads re-pack into them, stream-ordered, with no allocation.  The
-  // backward's copies are rebuilt too: by this load once they exist, else by
-  // the first backward.
+  // backward's copies are rebuilt too, by this load (load_writes_bwd) or by the
+  // first backward.
   h->loaded = false;
   h->bwd_ready = false;
   const bool first = h->wgu == nullptr;
@@ -647,9 +663,12 @@ int mgpt_moe_load_parameters(mgpt_moe* h, const float* const* params, int num_pa
     if (e != hipSuccess) rc = fail(MGPT_ERR_HIP, "parameter packing failed: %s", hipGetErrorString(e));
     return e == hipSuccess;
   };
-  // The backward's layouts are written here as well once a backward has
-  // filled them (and zeroed their padding).
-  const bool bwd = h->bwd_init;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  const bool capturing = cap != hipStreamCaptureStatusNone;
+  h->load_captured |= capturing;
+  bool bwd = false;   // the backward's layouts too
+  if (int wrc = load_writes_bwd(h, capturing, st, &bwd)) return wrc;
   do {
     const float* rp[2];
     const size_t rsz[2] = {(size_t)Cx * E, (size_t)E};
@@ -733,7 +752,7 @@ int mgpt_moe_load_parameters(mgpt_moe* h, const float* const* params, int num_pa
     }
   }
   h->loaded = true;
-  h->bwd_ready = bwd;
+  h->bwd_ready = bwd && !capturing;
   return MGPT_OK;
 }
 
@@ -967,7 +986,11 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
   const int C = h->C, Cx = h->Cx, H = h->H, E = h->E, k = h->k, Hp = h->Hp, Cp = h->Cp;
   const int A = N * k;
   if (int rc = ensure_grad(h)) return rc;
-  if (int rc = ensure_bwd_weights(h, st)) return rc;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  const bool capturing = cap != hipStreamCaptureStatusNone;
+  if (!capturing) h->bwd_used = false;   // until this backward is marked
+  if (int rc = ensure_bwd_weights(h, capturing, st)) return rc;
   // padded width: dy in and dx out through zero-padded rows; x is the padded
   // copy the training forward left in the workspace
   ActT* dx_out = dx;
@@ -997,10 +1020,8 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
   float* g = h->grad;
   const ActT* wdb = (const ActT*)h->wdb;
   const ActT* wgub = (const ActT*)h->wgub;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(st, &cap));
   // no stage events inside a captured graph (as in the forward)
-  const bool prof = h->profiling && !h->prof_gemm_only && cap == hipStreamCaptureStatusNone;
+  const bool prof = h->profiling && !h->prof_gemm_only && !capturing;
   hipEvent_t* evs = h->evb[h->prof_b_count % mgpt_moe::kProfSlots];
   auto mark = [&](int i) -> hipError_t { return prof ? hipEventRecord(evs[i], st) : hipSuccess; };
 
@@ -1138,6 +1159,10 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
   if (h->padded()) HIP_TRY(launch_copy_cols<ActT>(dx, C, dx_out, Cx, N, Cx, Cx, st));
   HIP_TRY(mark(7));
   if (prof) ++h->prof_b_count;
+  if (!capturing) {
+    HIP_TRY(hipEventRecord(h->bwd_done, st));
+    h->bwd_used = true;
+  }
   return MGPT_OK;
 }
 

@@ -70,3 +70,92 @@ def test_reload_equals_a_fresh_handle(C, H, E, k, act, source):
         torch.cuda.synchronize()
         for i, (a, b) in enumerate(zip(got, want)):
             assert torch.equal(a, b), f"output {i} of {len(want)}"
+
+
+def _fresh(params, x, dy, shape):
+    layer = MoELayer(*shape, act="bf16")
+    layer.load_parameters(params)
+    return _train(layer, x, dy)
+
+
+def _train(layer, x, dy):
+    layer.zero_grad()
+    y = layer.forward(x, train=True)
+    dx = layer.backward(dy)
+    return [y, dx] + layer.get_gradients()
+
+
+def _three(C, H, E, k, N, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    def normal(*s):
+        return torch.randn(*s, generator=gen, device="cuda") * 0.05
+    sets = []
+    for _ in range(2):
+        p = [normal(C, E), normal(1, E)]
+        for _ in range(E):
+            p += [normal(C, H), normal(1, H), normal(C, H), normal(1, H), normal(H, C), normal(1, C)]
+        sets.append(p)
+    return sets, normal(N, C).bfloat16(), normal(N, C).bfloat16()
+
+
+def test_load_beside_a_running_backward():
+    """A load on a second stream, ordered after the forward only, leaves the backward
+    that still runs its own weights; the next step has the new ones."""
+    shape, N = (512, 1024, 8, 2), 8192
+    (old, new), x, dy = _three(*shape, N, 1)
+    want_old, want_new = _fresh(old, x, dy, shape), _fresh(new, x, dy, shape)
+    layer = MoELayer(*shape, act="bf16")
+    layer.load_parameters(old)
+    _train(layer, x, dy)      # a backward has filled its layouts
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s1):
+        layer.load_parameters(old)
+        layer.zero_grad()
+        y = layer.forward(x, train=True)
+        fwd = torch.cuda.Event()
+        fwd.record(s1)
+        dx = layer.backward(dy)
+    with torch.cuda.stream(s2):
+        s2.wait_event(fwd)
+        layer.load_parameters(new)
+    torch.cuda.synchronize()
+    got = [y, dx] + layer.get_gradients()
+    assert all(torch.equal(a, b) for a, b in zip(got, want_old))
+    assert all(torch.equal(a, b) for a, b in zip(_train(layer, x, dy), want_new))
+
+
+@pytest.mark.parametrize("load_in_graph", [False, True])
+def test_loads_and_captured_backwards(load_in_graph):
+    """A graph's backward, and an eager one after a graph's load, see the parameters
+    loaded last, whichever was captured first."""
+    shape, N = (128, 192, 6, 2), 700
+    (old, new), x, dy = _three(*shape, N, 2)
+    want_old, want_new = _fresh(old, x, dy, shape), _fresh(new, x, dy, shape)
+    layer = MoELayer(*shape, act="bf16")
+    layer.reserve(N, train=True)
+    held = [p.clone() for p in old]
+    layer.load_parameters(held)
+    _train(layer, x, dy)
+    torch.cuda.synchronize()
+    out = torch.empty_like(x), torch.empty_like(x)
+    step, load = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(step):
+        layer.zero_grad()
+        layer.forward_into(x, out[0], train=True)
+        layer.backward_into(dy, out[1])
+    if load_in_graph:
+        with torch.cuda.graph(load):
+            layer.load_parameters(held)
+    for params, want in ((new, want_new), (old, want_old), (new, want_new)):
+        for h, p in zip(held, params):
+            h.copy_(p)
+        if load_in_graph:
+            load.replay()
+        else:
+            layer.load_parameters(held)
+        step.replay()
+        torch.cuda.synchronize()
+        got = list(out) + layer.get_gradients()
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), "replayed step"
+        assert all(torch.equal(a, b) for a, b in zip(_train(layer, x, dy), want)), "eager step"
