@@ -101,7 +101,8 @@ constexpr int kPartialFloats = 256 * 256;   // of one split work item
 // and refills them with units 2s+3 (weights of slab s+1) and 2s+4
 // (activations of slab s+2): the activations are requested two slabs ahead
 // and the weights one (a 2-stage ring of 64 KB slabs manages one for both).
-template <int EPI, int NW, bool kSave>
+// kGroups: more than 64 experts, a group of 64 per grid row.
+template <int EPI, int NW, bool kSave, bool kGroups>
 __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, const float* __restrict__ bias0,
     const float* __restrict__ bias1, const int32_t* __restrict__ counts, int E, int e_base, int K,
@@ -118,10 +119,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
 
   const int nbx = Npad / kBN;
   const int G = gridDim.x;
-  int t = (G % kNumXcd == 0) ? (blockIdx.x % kNumXcd) * (G / kNumXcd) + blockIdx.x / kNumXcd
-                             : blockIdx.x;
   const int KT = K / 64;
-  if (gridDim.y > 1) {   // a group of 64 experts per grid row
+  if constexpr (kGroups) {
     const int g0 = (int)blockIdx.y * kMaxExperts;
     E = min(kMaxExperts, E - g0);
     e_base += g0;
@@ -133,6 +132,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
   sc.init(counts, E, e_base);
   SplitPlan plan;
   plan.init(sc.tm * nbx, G, KT, partials != nullptr);
+  // an XCD takes a contiguous run of each round's items, of one that does not fill
+  // the grid an eighth
+  int t = blockIdx.x;
+  if (G % kNumXcd == 0) {
+    const int run = min(G, plan.items + kNumXcd - 1) / kNumXcd;
+    const int in_xcd = blockIdx.x / kNumXcd;
+    t = in_xcd < run ? (blockIdx.x % kNumXcd) * run + in_xcd : plan.items;
+  }
   Work cur;
   if (!locate_work(sc, plan, E, nbx, KT, t, &cur)) return;
 
@@ -395,9 +402,15 @@ hipError_t launch_gemm_dma(const bf16_t* A, const bf16_t* B, const float* bias0,
   // the gate/up epilogue's pre-activation stores are compiled only into
   // the training instance (fewer live registers in the inference one)
   auto launch = [&](auto save_c) {
-    hipLaunchKernelGGL((gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value>),
-                       dim3(grid, groups), dim3(kRingWaves * kWave), 0, stream, A, B, bias0, bias1,
-                       counts, E, 0, K, Npad, n_store, bias_ld, out, ldo, partials, save, save_ld);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(grid, groups), dim3(kRingWaves * kWave), 0, stream, A, B, bias0,
+                         bias1, counts, E, 0, K, Npad, n_store, bias_ld, out, ldo, partials, save, save_ld);
+    };
+    // (an instance of its own: the group's offsets live in scalar registers throughout)
+    if (groups > 1)
+      go(gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value, true>);
+    else
+      go(gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value, false>);
   };
   if constexpr (EPI == kEpiGateUp) {
     if (save)

@@ -343,8 +343,12 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[W::TN][W::TM],
 // them back, a cost that only a long K amortises: 256-row tiles of fewer
 // than kMinSplitSlabs 64-column slabs stay whole.  Measured on MI355X at the
 // cfg3 shapes (skewed counts): gate/up (K = 1024, 16 slabs) 0.426 ms whole
-// vs 0.439 split; down (K = 2816, 44 slabs) 0.214 split vs 0.246 whole.
-constexpr int kMinSplitSlabs = 24;
+// vs 0.439 split; down (K = 2816, 44 slabs) 0.214 split vs 0.246 whole.  A launch
+// without a full round splits in two from kMinHalvedSlabs on (three parts and more
+// from kMinSplitSlabs); us of the down product whole / in two: E = 16, C = 1024, H =
+// 1536, 3200 tokens 44 / 52; E = 32, C = 512, 4096 tokens H = 1536 42 / 43, H = 2048 49 /
+// 50, H = 2816 75 / 66; C = 1024, H = 4096, 2560 tokens 113 / 113.
+constexpr int kMinSplitSlabs = 24, kMinHalvedSlabs = 40;
 struct SplitPlan {
   int full, rem, s, items;
   __device__ __forceinline__ void init(int T, int G, int KT, bool enable) {
@@ -353,7 +357,7 @@ struct SplitPlan {
     s = 1;
     if (enable && rem > 0 && KT >= kMinSplitSlabs) {
       s = min(min(G / rem, 8), KT);
-      if (s < 2) s = 1;
+      if (s < (full > 0 || KT >= kMinHalvedSlabs ? 2 : 3)) s = 1;
     }
     items = s > 1 ? full + rem * s : T;
   }
