@@ -101,11 +101,11 @@ constexpr int kPartialFloats = 256 * 256;   // of one split work item
 // and refills them with units 2s+3 (weights of slab s+1) and 2s+4
 // (activations of slab s+2): the activations are requested two slabs ahead
 // and the weights one (a 2-stage ring of 64 KB slabs manages one for both).
-// kGroups: more than 64 experts, a group of 64 per grid row.
+// kGroups: more than 64 experts, `group` of them (at most 64) per grid row.
 template <int EPI, int NW, bool kSave, bool kGroups>
 __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, const float* __restrict__ bias0,
-    const float* __restrict__ bias1, const int32_t* __restrict__ counts, int E, int e_base, int K,
+    const float* __restrict__ bias1, const int32_t* __restrict__ counts, int E, int group, int K,
     int Npad, int n_store, int bias_ld, bf16_t* out, int ldo, float* __restrict__ partials,
     bf16_t* save, int save_ld) {
   using W = Waves<NW>;
@@ -120,10 +120,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
   const int nbx = Npad / kBN;
   const int G = gridDim.x;
   const int KT = K / 64;
+  int e_base = 0;
   if constexpr (kGroups) {
-    const int g0 = (int)blockIdx.y * kMaxExperts;
-    E = min(kMaxExperts, E - g0);
-    e_base += g0;
+    const int g0 = (int)blockIdx.y * group;
+    E = min(group, E - g0);
+    e_base = g0;
     B += (size_t)g0 * Npad * K;
     if (bias0) bias0 += (size_t)g0 * bias_ld;
     if (bias1) bias1 += (size_t)g0 * bias_ld;
@@ -387,8 +388,8 @@ hipError_t launch_gemm_dma(const bf16_t* A, const bf16_t* B, const float* bias0,
     return hipErrorInvalidValue;
   if (K / 64 < kMinSplitSlabs) partials = nullptr;   // no split, no reduce launch
   const int tiles = max_mtiles * (Npad / kBN);
-  // More than 64 experts: groups of 64, the weights and biases from the group's
-  // first expert on; the rows come in expert order, so each group's follow the
+  // More than 64 experts: equal groups of up to 64, the weights and biases from the
+  // group's first expert on; the rows come in expert order, so each group's follow the
   // earlier groups'.  One launch takes all groups as rows of its grid, so that
   // the CUs that a group's last round leaves idle go on with the next group;
   // that round is then not split (us of gate/up + down on MI355X with a launch
@@ -404,7 +405,8 @@ hipError_t launch_gemm_dma(const bf16_t* A, const bf16_t* B, const float* bias0,
   auto launch = [&](auto save_c) {
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(grid, groups), dim3(kRingWaves * kWave), 0, stream, A, B, bias0,
-                         bias1, counts, E, 0, K, Npad, n_store, bias_ld, out, ldo, partials, save, save_ld);
+                         bias1, counts, E, (E + groups - 1) / groups, K, Npad, n_store, bias_ld, out, ldo, partials, save,
+                         save_ld);
     };
     // (an instance of its own: the group's offsets live in scalar registers throughout)
     if (groups > 1)

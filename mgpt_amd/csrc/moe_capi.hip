@@ -1096,10 +1096,13 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
     // from the second stream on the rest; the dX product waits for both.
     // Stage timing keeps the launches serial.
     const bool fork = !prof && h->side && h->fork_ev && h->join_ev;
+    // (more than 64 experts: a grid row per group, which share the launch's CUs)
+    const int groups = (E + kMaxExperts - 1) / kMaxExperts;
+    auto share = [&](int cus) { return std::max(kNumXcd, cus / groups / kNumXcd * kNumXcd); };
     if (fork) HIP_TRY(hipEventRecord(h->fork_ev, st));
     HIP_TRY(launch_gemm_dma<kEpiSwigluBwd>((const bf16_t*)dgo, (const bf16_t*)wdb, nullptr,
                                            nullptr, counts, E, C, h->Hq, Hp, 0, (bf16_t*)gu,
-                                           2 * Hp, mt, nullptr, fork ? h->dact_cus : h->num_cus,
+                                           2 * Hp, mt, nullptr, fork ? share(h->dact_cus) : h->num_cus,
                                            (bf16_t*)gu, 2 * Hp, st));
     if (fork) {
       HIP_TRY(hipStreamWaitEvent(h->side, h->fork_ev, 0));
@@ -1123,7 +1126,7 @@ int backward_impl(mgpt_moe* h, const ActT* x, const ActT* dy, ActT* dx, int N, c
     }
     HIP_TRY(launch_gemm_dma<kEpiDown>((const bf16_t*)gu, (const bf16_t*)wgub, nullptr, nullptr,
                                       counts, E, 2 * Hp, Cp, C, 0, (bf16_t*)ob, C, mt,
-                                      (float*)(ws + L.partials), fork2 ? h->dx_cus : h->num_cus,
+                                      (float*)(ws + L.partials), fork2 ? share(h->dx_cus) : h->num_cus,
                                       nullptr, 0, st));
   } else if (small_m(h, N)) {
     HIP_TRY((launch_gemm_stream<kEpiSwigluBwd, bf16_t>(
