@@ -22,8 +22,8 @@ constexpr int kNumXcd = 8;        // MI355X: 8 accelerator complex dies, one L2 
 // Experts the kernels that map one expert to one lane of a wave take (the
 // fused prefill and decode routers, the weight-streaming GEMM, the weight
 // gradients' row chunks); up to kMaxExpertsWide the layer runs the router's
-// logits in groups of 64 experts and a wide softmax, the 256 x 256 GEMMs
-// once per group of 64, the generic grouped GEMMs, a permute that scans the
+// logits in groups of 64 experts and a wide softmax, the bf16 and fp8 GEMMs
+// with a group of at most 64 experts per grid row, a permute that scans the
 // experts in wave-sized chunks, and the backward's wide token and router
 // gradients.
 constexpr int kMaxExperts = 64;

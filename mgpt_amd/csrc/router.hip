@@ -18,8 +18,8 @@
 // sum, the clamp and the insertion top-k in registers.  Phase 3: block-local
 // expert histogram (LDS atomics on ints; counts are order-free), written
 // expert-major as hist[e][block] for the per-expert scan of dispatch.hip.
-// Decode shapes (few tokens, E > 16) split phase 1 over more blocks, one
-// expert per wave, through a logits buffer.
+// Other calls form their logits in kernels of their own, through a logits
+// buffer (launch_router chooses), or a whole step of up to 64 tokens in one launch.
 #include <type_traits>
 
 #include "common.hpp"
@@ -633,29 +633,28 @@ __global__ __launch_bounds__(1024) void router_topk_uniform_kernel(
   softmax_topk_block(s_l, s_m, s_hist, tok0, N, E, k, topk_idx, topk_p, hist, num_blocks, probs);
 }
 
-// Few tokens, many experts (decode shapes): the fused kernel would run a
-// handful of blocks whose waves each walk RE experts.  Here a block of
-// kSplitExperts waves computes that many experts' logits (one each; wr1 =
-// W_r transposed, [E][C]) for 64 tokens, written to global memory, and
-// router_softmax_kernel finishes: the chains are as long as before, but
-// spread over more CUs.
+// Normalised rows that are not normalised once beforehand, of more than 16 experts
+// and too few tokens for the fused (E <= 64) or grouped kernel to fill the chip: a block of kSplitExperts waves computes that many
+// experts' logits (one each; wr1 = W_r transposed, [E][C]) for 64 tokens, written to
+// global memory, and router_softmax_kernel finishes: the chains are as long as the
+// fused kernel's, but spread over more CUs.
 constexpr int kSplitExperts = 4;
-template <typename ActT, bool NORM>
+template <typename ActT>
 __global__ __launch_bounds__(kSplitExperts * 64) void router_logits_kernel(
     const ActT* __restrict__ x, const float* __restrict__ wr1, const float* __restrict__ br,
     int N, int C, int E, float* __restrict__ logits, RowNorm nrm, float* __restrict__ rstd) {
   __shared__ __attribute__((aligned(1024)))
-  char smem[kRouterSplitLds + (NORM ? kRouterNormLds : 0)];
+  char smem[kRouterSplitLds + kRouterNormLds];
   const int lane = lane_id();
   const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
   const int e0 = blockIdx.y * kSplitExperts;
   const int tok0 = blockIdx.x * kRT;
   float acc[1];
   float r = 1.0f;
-  logit_chains<ActT, 1, NORM>(x + (size_t)tok0 * C, N - tok0, wr1 + (size_t)e0 * C,
+  logit_chains<ActT, 1, true>(x + (size_t)tok0 * C, N - tok0, wr1 + (size_t)e0 * C,
                         min(kSplitExperts, E - e0), kSplitExperts, g, C, smem, acc, nrm, &r,
                         kRouterSplitLds);
-  if (NORM && blockIdx.y == 0 && g == 0 && tok0 + lane < N) rstd[tok0 + lane] = r;
+  if (blockIdx.y == 0 && g == 0 && tok0 + lane < N) rstd[tok0 + lane] = r;
   const int e = e0 + g;
   if (e < E && tok0 + lane < N) logits[(size_t)(tok0 + lane) * E + e] = acc[0] + br[e];
 }
@@ -1468,7 +1467,7 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
         hipLaunchKernelGGL((router_logits_wide_kernel<ActT, false>), dim3(nb, eg), dim3(1024), 0,
                            stream, x, wr_g, br, N, C, E, logits, nrm, rstd);
     } else if (gamma)
-      hipLaunchKernelGGL((router_logits_kernel<ActT, true>),
+      hipLaunchKernelGGL((router_logits_kernel<ActT>),
                          dim3(nb, (E + kSplitExperts - 1) / kSplitExperts),
                          dim3(kSplitExperts * kWave), 0, stream, x, wr1, br, N, C, E, logits, nrm,
                          rstd);
@@ -1568,7 +1567,7 @@ hipError_t launch_router(const ActT* x, const float* wr_g, const float* wr1, con
   }
   if (logits && gamma && E > 16 && N < 4096) {
     const dim3 lg(nb, (E + kSplitExperts - 1) / kSplitExperts), lb(kSplitExperts * kWave);
-    hipLaunchKernelGGL((router_logits_kernel<ActT, true>), lg, lb, 0, stream, x, wr1, br, N, C, E,
+    hipLaunchKernelGGL((router_logits_kernel<ActT>), lg, lb, 0, stream, x, wr1, br, N, C, E,
                        logits, nrm, rstd);
     hipLaunchKernelGGL(router_softmax_kernel, dim3(nb), dim3(MGPT_SOFTMAX_THREADS), 0, stream,
                        logits, N, E, k,

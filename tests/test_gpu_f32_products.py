@@ -21,15 +21,41 @@ from mgpt_amd.moe import MoELayer
 pytestmark = pytest.mark.gpu
 TOL = 1.2e-5
 
-# (N, C, H, E, k): one row; segments around 64 and 128 rows; tiles enough for
-# every choice of the forward and data-gradient products, and in the last two
-# for a weight-gradient tile a wave; odd widths; one expert; more experts than
-# a wave has lanes
+# (N, C, H, E, k): one row; segments around 64 and 128 rows; odd widths; one
+# expert; more experts than a wave has lanes; many rows of narrow layers (every tile of
+# the down and input-gradient products, the largest with a column tile half empty);
+# many wide experts (a weight-gradient tile a wave)
 SHAPES = [
     (1, 64, 32, 4, 2), (63, 64, 64, 1, 1), (65, 128, 96, 1, 1), (129, 72, 33, 2, 1),
     (257, 200, 130, 3, 2), (1000, 130, 257, 5, 2), (4100, 256, 1024, 4, 2), (700, 512, 1376, 8, 2),
     (900, 64, 40, 70, 3), (8200, 64, 2560, 4, 2), (300, 256, 768, 70, 3),
+    (24600, 192, 40, 4, 2), (42003, 192, 40, 4, 2), (100, 512, 1376, 40, 2),
 ]
+
+
+def choices(N, C, H, E, k):
+    """The tiles that the products of a call take, by the launch rules restated."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    up = lambda v, m: -(-v // m)
+    C, Hp = up(C, 64) * 64, up(H, 128) * 128
+    t = lambda cols: up(N * k, 64) * up(cols, 128)
+
+    def down(cols):
+        return "64x128" if t(cols) >= 10 * cus else "32x64" if t(cols) >= 3 * cus else "32x32"
+
+    def wgrad(i, j):
+        return "a wave" if up(up(i, 64), 2) * up(up(j, 64), 2) * E >= 6 * cus else "four waves"
+
+    return {("gate/up", "64x128" if t(2 * Hp) >= 4 * cus else "32x64"), ("down, dx", down(C)),
+            ("d(act)", down(Hp)), ("dW_down", wgrad(H, C)), ("dW_gate/up", wgrad(C, 2 * Hp))}
+
+
+def test_shapes_reach_every_tile():
+    got = set().union(*(choices(*s) for s in SHAPES))
+    assert got == {("gate/up", "64x128"), ("gate/up", "32x64"), ("down, dx", "64x128"), ("down, dx", "32x64"),
+                   ("down, dx", "32x32"), ("d(act)", "64x128"), ("d(act)", "32x64"), ("d(act)", "32x32"),
+                   ("dW_down", "a wave"), ("dW_down", "four waves"), ("dW_gate/up", "a wave"),
+                   ("dW_gate/up", "four waves")}
 
 
 def _exact(layer, x, p, dy, E):

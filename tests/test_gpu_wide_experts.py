@@ -2,12 +2,12 @@
 (64 < E <= 512), and of its training, against the reference.
 
 The reference's layer takes any expert count (pipeline/CLIConfig.h:177-178).
-Here such handles run the split router (logits per expert or per group of
-64 experts, then a block softmax / top-k over rows of up to 512 experts),
-the permute's offsets scan in wave-sized chunks with eight or nine ballots
-on the expert ids, the 256 x 256 GEMMs once per group of 64 experts, and
-the generic grouped GEMMs whose tile lookup scans the counts 64 experts at
-a time.
+Here such handles run the split router (logits by product and chain waves, by
+an expert per lane or per group of 64 experts, tests/test_gpu_router_paths.py, then
+a block softmax / top-k over rows of up to 512 experts), the permute's offsets scan
+in wave-sized chunks with eight or nine ballots on the expert ids, the bf16 and fp8
+GEMMs with a group of at most 64 experts per grid row, and the fp32 GEMMs, whose tile
+lookup scans the counts 64 experts at a time.
 Routing must be bit-exact with the committed fixtures of the compiled
 reference (full arrays for the small cases, digests for the large one);
 outputs are compared with the oracle's fp32 forward at 1e-5 (fp32), 2e-2
@@ -57,8 +57,8 @@ def test_wide_forward_parity(name):
 @pytest.mark.parametrize("N,E,rb", [(150, 128, "normal"), (4096, 256, "zero")])
 def test_wide_fused_block(N, E, rb):
     """out = x + MoE(RMSNorm(x) * gamma) with E = 128 and 256: the wide
-    router normalises the rows (1/rms bit-exact; at 4096 tokens x 256
-    experts in the 64-expert-group logits kernel), routing bit-exact with the
+    router's rows are normalised once (1/rms bit-exact; 150 tokens go on to the
+    product and chain waves, 4096 to an expert per lane), routing bit-exact with the
     oracle's block, out at the bf16 bar."""
     from mgpt_amd import workload as wl
     cfg = wl.MoEConfig("wide_blk", N, 128, E, 4, 64, "bf16", "bf16", rb)
@@ -138,10 +138,10 @@ EDGE = [
     (33, 100, 255, 8, 40, "f32", "zero"),
     (64, 128, 256, 1, 64, "f32", "zero"),
     (700, 192, 97, 3, 96, "bf16", "zero"),
-    # enough (64 tokens, 64 experts) blocks for the grouped logits kernel
+    # an expert per lane, four tokens a wave
     (4096, 128, 256, 8, 64, "bf16", "zero"),
     # past 256 experts (nine id bits, the 512-wide softmax row and token
-    # gradients), prefill-sized with the grouped kernels and decode-sized
+    # gradients), prefill-sized and decode-sized
     (8192, 64, 384, 8, 64, "bf16", "zero"),
     (64, 128, 512, 4, 64, "f32", "zero"),
 ]
