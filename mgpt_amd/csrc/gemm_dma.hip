@@ -101,8 +101,8 @@ constexpr int kPartialFloats = 256 * 256;   // of one split work item
 // and refills them with units 2s+3 (weights of slab s+1) and 2s+4
 // (activations of slab s+2): the activations are requested two slabs ahead
 // and the weights one (a 2-stage ring of 64 KB slabs manages one for both).
-// kGroups: more than 64 experts, `group` of them (at most 64) per grid row.
-template <int EPI, int NW, bool kSave, bool kGroups>
+// More than 64 experts: `group` of them (at most 64) per grid row.
+template <int EPI, int NW, bool kSave>
 __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, const float* __restrict__ bias0,
     const float* __restrict__ bias1, const int32_t* __restrict__ counts, int E, int group, int K,
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
   const int G = gridDim.x;
   const int KT = K / 64;
   int e_base = 0;
-  if constexpr (kGroups) {
+  if (gridDim.y > 1) {
     const int g0 = (int)blockIdx.y * group;
     E = min(group, E - g0);
     e_base = g0;
@@ -133,13 +133,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
   sc.init(counts, E, e_base);
   SplitPlan plan;
   plan.init(sc.tm * nbx, G, KT, partials != nullptr);
-  // an XCD takes a contiguous run of each round's items, of one that does not fill
-  // the grid an eighth
-  int t = blockIdx.x;
-  if (G % kNumXcd == 0) {
-    const int run = min(G, plan.items + kNumXcd - 1) / kNumXcd;
-    const int in_xcd = blockIdx.x / kNumXcd;
-    t = in_xcd < run ? (blockIdx.x % kNumXcd) * run + in_xcd : plan.items;
+  int t = (G % kNumXcd == 0) ? (blockIdx.x % kNumXcd) * (G / kNumXcd) + blockIdx.x / kNumXcd
+                             : blockIdx.x;
+  // (a down product that does not fill the grid: an eighth of its items per XCD)
+  if (EPI == kEpiDown && plan.items < G && G % kNumXcd == 0) {
+    const int run = (plan.items + kNumXcd - 1) / kNumXcd, in_xcd = (int)blockIdx.x / kNumXcd;
+    t = in_xcd < run ? (int)(blockIdx.x % kNumXcd) * run + in_xcd : plan.items;
   }
   Work cur;
   if (!locate_work(sc, plan, E, nbx, KT, t, &cur)) return;
@@ -403,16 +402,10 @@ hipError_t launch_gemm_dma(const bf16_t* A, const bf16_t* B, const float* bias0,
   // the gate/up epilogue's pre-activation stores are compiled only into
   // the training instance (fewer live registers in the inference one)
   auto launch = [&](auto save_c) {
-    auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(grid, groups), dim3(kRingWaves * kWave), 0, stream, A, B, bias0,
-                         bias1, counts, E, (E + groups - 1) / groups, K, Npad, n_store, bias_ld, out, ldo, partials, save,
-                         save_ld);
-    };
-    // (an instance of its own: the group's offsets live in scalar registers throughout)
-    if (groups > 1)
-      go(gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value, true>);
-    else
-      go(gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value, false>);
+    hipLaunchKernelGGL((gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value>), dim3(grid, groups),
+                       dim3(kRingWaves * kWave), 0, stream, A, B, bias0, bias1, counts, E,
+                       (E + groups - 1) / groups, K, Npad, n_store, bias_ld, out, ldo, partials, save,
+                       save_ld);
   };
   if constexpr (EPI == kEpiGateUp) {
     if (save)
