@@ -344,11 +344,12 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[W::TN][W::TM],
 // than kMinSplitSlabs 64-column slabs stay whole.  Measured on MI355X at the
 // cfg3 shapes (skewed counts): gate/up (K = 1024, 16 slabs) 0.426 ms whole
 // vs 0.439 split; down (K = 2816, 44 slabs) 0.214 split vs 0.246 whole.  A launch
-// without a full round splits in two from kMinHalvedSlabs on (three parts and more
-// from kMinSplitSlabs); us of the down product whole / in two: E = 16, C = 1024, H =
-// 1536, 3200 tokens 44 / 52; E = 32, C = 512, 4096 tokens H = 1536 42 / 43, H = 2048 49 /
-// 50, H = 2816 75 / 66; C = 1024, H = 4096, 2560 tokens 113 / 113.
-constexpr int kMinSplitSlabs = 24, kMinHalvedSlabs = 40;
+// without a full round splits from three parts on: two save little or nothing, and
+// the CUs that they keep busy cost the power-limited chip clock in the products around
+// (us of gate/up + down, the latter whole / in two: E = 16, C = 1024, H = 1536, 3200
+// tokens 58 + 44 / 59 + 52; C = 256, H = 2816, 12000 tokens 92 + 65 / 101 + 64; E = 32, C =
+// 512, 4096 tokens H = 2048 51 + 49 / 57 + 50, H = 2816 90 + 75 / 91 + 66).
+constexpr int kMinSplitSlabs = 24;
 struct SplitPlan {
   int full, rem, s, items;
   __device__ __forceinline__ void init(int T, int G, int KT, bool enable) {
@@ -357,7 +358,7 @@ struct SplitPlan {
     s = 1;
     if (enable && rem > 0 && KT >= kMinSplitSlabs) {
       s = min(min(G / rem, 8), KT);
-      if (s < (full > 0 || KT >= kMinHalvedSlabs ? 2 : 3)) s = 1;
+      if (s < (full > 0 ? 2 : 3)) s = 1;
     }
     items = s > 1 ? full + rem * s : T;
   }
