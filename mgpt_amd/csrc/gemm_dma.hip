@@ -101,8 +101,11 @@ constexpr int kPartialFloats = 256 * 256;   // of one split work item
 // and refills them with units 2s+3 (weights of slab s+1) and 2s+4
 // (activations of slab s+2): the activations are requested two slabs ahead
 // and the weights one (a 2-stage ring of 64 KB slabs manages one for both).
-// More than 64 experts: `group` of them (at most 64) per grid row.
-template <int EPI, int NW, bool kSave>
+// More than 64 experts: `group` of them (at most 64) per grid row; kTurn: every other
+// row takes its tiles from the other end, so that the rows' last rounds even out over
+// the XCDs (an instance of its own: the kernel runs at the register limit, and the
+// turn cost launches of one row 1%).
+template <int EPI, int NW, bool kSave, bool kTurn>
 __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, const float* __restrict__ bias0,
     const float* __restrict__ bias1, const int32_t* __restrict__ counts, int E, int group, int K,
@@ -135,6 +138,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring5_kernel(
   plan.init(sc.tm * nbx, G, KT, partials != nullptr);
   int t = (G % kNumXcd == 0) ? (blockIdx.x % kNumXcd) * (G / kNumXcd) + blockIdx.x / kNumXcd
                              : blockIdx.x;
+  if (kTurn && (blockIdx.y & 1)) t = G - 1 - t;
   // (a down product that does not fill the grid: an eighth of its items per XCD)
   if (EPI == kEpiDown && plan.items < G && G % kNumXcd == 0) {
     const int run = (plan.items + kNumXcd - 1) / kNumXcd, in_xcd = (int)blockIdx.x / kNumXcd;
@@ -392,9 +396,9 @@ hipError_t launch_gemm_dma(const bf16_t* A, const bf16_t* B, const float* bias0,
   // earlier groups'.  One launch takes all groups as rows of its grid, so that
   // the CUs that a group's last round leaves idle go on with the next group;
   // that round is then not split (us of gate/up + down on MI355X with a launch
-  // and a split reduction per group and so: E = 128, C = 1024, H = 704, 511 rows
-  // an expert 233 + 161 -> 226 + 154; E = 256, C = 768, H = 512, 200 rows 192 +
-  // 107 -> 151 + 94).
+  // and a split reduction per group, so, and every other group turned: E = 128, C =
+  // 1024, H = 704, 511 rows an expert 238 + 163, 235 + 158, 237 + 137; E = 256, C = 768, H =
+  // 512, 200 rows 192 + 107 -> 151 + 94).
   const int groups = (E + kMaxExperts - 1) / kMaxExperts;
   if (groups > 1) partials = nullptr;
   // (with split tiles every CU has work, also where there are fewer tiles)
@@ -402,10 +406,15 @@ hipError_t launch_gemm_dma(const bf16_t* A, const bf16_t* B, const float* bias0,
   // the gate/up epilogue's pre-activation stores are compiled only into
   // the training instance (fewer live registers in the inference one)
   auto launch = [&](auto save_c) {
-    hipLaunchKernelGGL((gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value>), dim3(grid, groups),
-                       dim3(kRingWaves * kWave), 0, stream, A, B, bias0, bias1, counts, E,
-                       (E + groups - 1) / groups, K, Npad, n_store, bias_ld, out, ldo, partials, save,
-                       save_ld);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(grid, groups), dim3(kRingWaves * kWave), 0, stream, A, B, bias0,
+                         bias1, counts, E, (E + groups - 1) / groups, K, Npad, n_store, bias_ld, out, ldo,
+                         partials, save, save_ld);
+    };
+    if (groups > 1)
+      go(gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value, true>);
+    else
+      go(gemm_ring5_kernel<EPI, kRingWaves, decltype(save_c)::value, false>);
   };
   if constexpr (EPI == kEpiGateUp) {
     if (save)

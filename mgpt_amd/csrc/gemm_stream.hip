@@ -111,18 +111,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
   __shared__ __attribute__((aligned(1024))) char smem[ST * kStage];
 
   const int G = gridDim.x;
-  // Which tiles an XCD (own L2) takes.  256-row tiles: contiguous runs, which share
-  // operand panels.  64-row tiles share little beyond the (at most four) m-tiles of a
-  // weight panel and are often fewer than the blocks, so runs of four tiles are dealt
-  // to the XCDs in turn, which leaves none of them idle.
-  constexpr int kRun = 4;
-  const int xcd = blockIdx.x % kNumXcd, in_xcd = blockIdx.x / kNumXcd;
-  int t = blockIdx.x;
-  if (BM > 64) {
-    if (G % kNumXcd == 0) t = xcd * (G / kNumXcd) + in_xcd;
-  } else if (G % (kRun * kNumXcd) == 0) {
-    t = (in_xcd / kRun * kNumXcd + xcd) * kRun + in_xcd % kRun;
-  }
   const int KT = K / 64;
   int e_base = 0;
   if (gridDim.y > 1) {   // a group of 64 experts per grid row
@@ -136,6 +124,21 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(
   }
   SegScan<BM> sc;
   sc.init(counts, E, e_base);
+  // Which tiles an XCD (own L2) takes.  256-row tiles: contiguous runs of each round,
+  // which share operand panels; an eighth of a round that does not fill the grid, and
+  // every other group from the other end, so that the last rounds even out.  64-row
+  // tiles share little beyond the (at most four) m-tiles of a weight panel, so runs of
+  // four tiles are dealt to the XCDs in turn.
+  constexpr int kRun = 4;
+  const int in_xcd = blockIdx.x / kNumXcd;
+  int xcd = blockIdx.x % kNumXcd, t = blockIdx.x;
+  if (blockIdx.y & 1) xcd = kNumXcd - 1 - xcd;
+  if (BM <= 64) {
+    if (G % (kRun * kNumXcd) == 0) t = (in_xcd / kRun * kNumXcd + xcd) * kRun + in_xcd % kRun;
+  } else if (G % kNumXcd == 0) {
+    const int items = sc.tm * nbx, run = min(G, items + kNumXcd - 1) / kNumXcd;
+    t = in_xcd < run ? xcd * run + in_xcd : items;
+  }
   Tile cur;
   if (!locate_tile<BN>(sc, E, nbx, t, &cur)) return;
 
