@@ -514,6 +514,21 @@ hipError_t launch_decode(const XT* A, const fp8_t* B, const float* wscale, const
     const double rounds = E * p * per_tile;
     const double most = std::ceil(std::min((double)E, E * p + 1.5 * std::sqrt(E * p * (1.0 - p))) * per_tile);
     wide = most < 1.33 * rounds || (most == 1.0 && rounds > 0.5);
+  } else if (rows >= 4L * E && K >= 1024) {
+    // bf16 rows, one row tile an expert or two: items of 128 features read the rows'
+    // stages twice as often, which costs more than their finer last round saves where a
+    // CU has much to contract (twice that for one tile) and the 256-feature items nearly
+    // fill their rounds (and an expert has eight feature blocks, so that its row tiles
+    // share an XCD).  us of the forward for 128 / 256: E = 64, C = 4096, H = 2048, k = 8,
+    // 288 tokens 487 / 406; E = 32, C = 2048, H = 4096, k = 4, 352 tokens 270 / 228; E = 32,
+    // C = 4096, H = 1024, k = 2, 992 tokens 206 / 193; E = 64, C = 1024, H = 4096, k = 4, 448
+    // tokens 225 / 206; where the rule keeps 128, gate/up alone: E = 16, C = 1024, H = 2816,
+    // k = 2, 352 tokens 33 / 39; E = 64, C = 2048, H = 512, k = 4, 832 tokens 57 / 66; E =
+    // 64, C = 2048, H = 1408, k = 8, 240 tokens 83 / 88.
+    const int tiles = rows > 32L * E ? 2 : 1;
+    const int nb = (n_store + 255) / 256;
+    const double rounds = (double)tiles * E * nb / num_cus;
+    wide = nb >= 8 && rounds * K >= 8192.0 / tiles && rounds > 0.9 * std::ceil(rounds);
   }
   auto launch = [&](auto kernel, int NW) {
     const long items = (long)(rows / 32 + std::min(E, rows)) * ((n_store + 64 * NW - 1) / (64 * NW));
