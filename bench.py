@@ -294,7 +294,7 @@ def summarize_stats(stats_csv: str, bench_json: str, config: str) -> str:
         mode, f"{w + 2 * k} forwards ({w} warmup, {k} timed, {k} profiled)")
     out = [f"# {b['config']['workload'].split(':')[0]} MoE {what}: rocprofv3 kernel statistics "
            "(MI355X)", "",
-           "Command (repository root, on the GPU box), then "
+           "Command (repository root), then "
            "`python bench.py --summarize-stats <dir>/run_kernel_stats.csv <json line>`:", "",
            "```", cmd, "```", "",
            f"Workload: {b['config']['workload']}.  {runs}; pack/pad/quantise/copy/transpose "

@@ -5,7 +5,7 @@ The generator is counter-based (element i of stream s is a pure function of
 float64 +, -, *, / and sqrt.  Logarithm and cosine are evaluated with fixed
 polynomials below instead of libm or numpy's SIMD transcendental kernels,
 whose last bits can differ between host CPUs; the same seed therefore gives
-the same float32 arrays on this build host and on any GPU box, which is what
+the same float32 arrays on any host, which is what
 lets committed golden fixtures be checked against freshly generated inputs.
 
 Normal variates: Box-Muller, z = sqrt(-2 ln u1) cos(2 pi u2), with u1 in
